@@ -53,11 +53,14 @@ int fail(ldg_handle *h, int code, const char *msg) {
 // Candidate elements per workgroup of each kernel, per order (the
 // autotuner picks among them; index 0 is the default).
 template <int N> struct Cand;
-template <> struct Cand<2> { static constexpr int rhs[kMaxCand] = {16, 8}, grad[kMaxCand] = {16, 8}; };
-template <> struct Cand<3> { static constexpr int rhs[kMaxCand] = {8, 4}, grad[kMaxCand] = {8, 4}; };
-template <> struct Cand<4> { static constexpr int rhs[kMaxCand] = {4, 2}, grad[kMaxCand] = {4, 2}; };
-template <> struct Cand<5> { static constexpr int rhs[kMaxCand] = {2, 1}, grad[kMaxCand] = {2, 4}; };
-template <> struct Cand<6> { static constexpr int rhs[kMaxCand] = {1, 1}, grad[kMaxCand] = {1, 2}; };
+template <> struct Cand<2> { static constexpr int rhs[kMaxCand] = {16, 32}, grad[kMaxCand] = {16, 32}; };
+template <> struct Cand<3> { static constexpr int rhs[kMaxCand] = {7, 14}, grad[kMaxCand] = {7, 14}; };
+template <> struct Cand<4> { static constexpr int rhs[kMaxCand] = {4, 8}, grad[kMaxCand] = {4, 8}; };
+template <> struct Cand<5> { static constexpr int rhs[kMaxCand] = {2, 5}, grad[kMaxCand] = {5, 2}; };
+template <> struct Cand<6> { static constexpr int rhs[kMaxCand] = {3, 1}, grad[kMaxCand] = {3, 5}; };
+// elements per workgroup of the nodal gradient kernel (256 threads)
+template <int N> struct NodalE { static constexpr int value = N == 2 ? 16 : N == 3 ? 8 : N == 4 ? 4 : N == 5 ? 2 : 1; };
+int nodal_e(int n) { return n == 2 ? 16 : n == 3 ? 8 : n == 4 ? 4 : n == 5 ? 2 : 1; }
 
 int cand_e(int n, bool rhs, int c) {
   switch (n) {
@@ -95,29 +98,50 @@ Ops<N, double> make_ops(const Basis1D &B, double &asym) {
     o.L0[a] = B.at(B.M1inv, a, 0);
     o.w[a] = B.w[a];
   }
+  // Gauss form: Lagrange polynomials L_q of the Gauss points at the nodes
+  // (I^-1) and their derivatives at the Gauss points (Dg; barycentric, each
+  // diagonal minus its row, so that constants are annihilated)
+  double I[N][N], D[N][N], Ii[N][N], Dg[N][N], Dh[N][N], bw[N];
   for (int q = 0; q < N; ++q) {
-    o.IL0[q] = 0.0;
-    for (int j = 0; j < N; ++j) o.IL0[q] += o.I[q][j] * o.L0[j];
+    bw[q] = 1.0;
+    for (int j = 0; j < N; ++j)
+      if (j != q) bw[q] /= (B.g[q] - B.g[j]);
+  }
+  for (int a = 0; a < N; ++a) {
+    double sum = 0.0;
+    for (int b = 0; b < N; ++b) {
+      I[a][b] = o.I[a][b];
+      D[a][b] = o.D[a][b];
+      double v = 1.0;
+      for (int j = 0; j < N; ++j)
+        if (j != b) v *= (B.r[a] - B.g[j]) / (B.g[b] - B.g[j]);
+      Ii[a][b] = v;
+      if (b != a) {
+        Dg[a][b] = bw[b] / bw[a] / (B.g[a] - B.g[b]);
+        sum += Dg[a][b];
+      }
+    }
+    Dg[a][a] = -sum;
+  }
+  for (int q = 0; q < N; ++q) {
+    o.eta[q] = Ii[0][q] / B.w[q];   // the first node is the - face
+    for (int j = 0; j < N; ++j) Dh[q][j] = Dg[j][q] * B.w[j] / B.w[q];
   }
   // sweep operators in even/odd split form, from their (anti-)centro-symmetric
   // parts (the node sets are symmetric; this removes construction round-off)
-  double I[N][N], It[N][N], Dt[N][N], Mi[N][N], D[N][N];
-  for (int a = 0; a < N; ++a)
-    for (int b = 0; b < N; ++b) {
-      I[a][b] = o.I[a][b];
-      It[a][b] = o.I[b][a];
-      Dt[a][b] = o.D[b][a];
-      Mi[a][b] = o.Minv[a][b];
-      D[a][b] = o.D[a][b];
-    }
-  asym = std::max(std::max(symmetrize_checked<N>(I, 1), symmetrize_checked<N>(It, 1)),
-                  std::max(symmetrize_checked<N>(Dt, -1), symmetrize_checked<N>(Mi, 1)));
-  asym = std::max(asym, symmetrize_checked<N>(D, -1));
+  asym = std::max(std::max(symmetrize_checked<N>(I, 1), symmetrize_checked<N>(Ii, 1)),
+                  std::max(symmetrize_checked<N>(D, -1), symmetrize_checked<N>(Dg, -1)));
+  asym = std::max(asym, symmetrize_checked<N>(Dh, -1));
+  for (int q = 0; q < N; ++q) {     // the lifts of the two faces mirror each other
+    const double lo = Ii[0][q] / B.w[q];
+    asym = std::max(asym, std::fabs(lo - o.eta[q]));
+    o.eta[q] = lo;
+  }
   make_symmat<N, double>(I, o.sI);
-  make_symmat<N, double>(It, o.sIt);
-  make_symmat<N, double>(Dt, o.sDt);
-  make_symmat<N, double>(Mi, o.sMi);
   make_symmat<N, double>(D, o.sD);
+  make_symmat<N, double>(Ii, o.sIi);
+  make_symmat<N, double>(Dg, o.sDg);
+  make_symmat<N, double>(Dh, o.sDh);
   return o;
 }
 
@@ -148,55 +172,73 @@ StageArgs empty_stage() {
 
 // ---------------------------------------------------------------- launches
 
+LaunchArgs launch_args(const Group &g, const Tiling &t) {
+  return LaunchArgs{t.d_inst, t.d_blk, t.nblocks, (t.nblocks + 7) / 8, g.K};
+}
+
 template <int N, int E>
-void launch_grad_e(ldg_handle *h, Group &g, const Tiling &t, StageIn U, bool wq) {
-  LaunchArgs la{t.d_inst, t.d_blk, t.nblocks, (t.nblocks + 7) / 8};
+void launch_grad_e(ldg_handle *h, Group &g, const Tiling &t, StageIn U) {
+  const LaunchArgs la = launch_args(g, t);
+  const unsigned char *img = (const unsigned char *)g.sops;
+  const dim3 grid(8 * la.per_xcd), block(Shape<N, E>::NTH);
+  if (h->mixed && U.fluct)
+    hipLaunchKernelGGL((ldg_grad_kernel<N, E, float, float>), grid, block, 0, h->stream, (const float *)U.p,
+                       (float *)g.ff, la, img);
+  else if (h->mixed)
+    hipLaunchKernelGGL((ldg_grad_kernel<N, E, float, double>), grid, block, 0, h->stream, (const double *)U.p,
+                       (float *)g.ff, la, img);
+  else
+    hipLaunchKernelGGL((ldg_grad_kernel<N, E, double, double>), grid, block, 0, h->stream, (const double *)U.p,
+                       (double *)g.ff, la, img);
+}
+
+template <int N>
+void launch_nodal_n(ldg_handle *h, Group &g, StageIn U) {
+  constexpr int E = NodalE<N>::value;
+  const LaunchArgs la = launch_args(g, g.nodal);
   const Ops<N, double> *op = (const Ops<N, double> *)g.ops;
   const dim3 grid(8 * la.per_xcd), block(NT);
-  if (h->mixed && U.fluct) {
-    if (wq)
-      hipLaunchKernelGGL((ldg_grad_kernel<N, E, float, float, true>), grid, block, 0, h->stream, (const float *)U.p,
-                         (float *)g.q, (float *)g.ff, la, op);
-    else
-      hipLaunchKernelGGL((ldg_grad_kernel<N, E, float, float, false>), grid, block, 0, h->stream, (const float *)U.p,
-                         (float *)g.q, (float *)g.ff, la, op);
-  } else if (h->mixed) {
-    if (wq)
-      hipLaunchKernelGGL((ldg_grad_kernel<N, E, float, double, true>), grid, block, 0, h->stream, (const double *)U.p,
-                         (float *)g.q, (float *)g.ff, la, op);
-    else
-      hipLaunchKernelGGL((ldg_grad_kernel<N, E, float, double, false>), grid, block, 0, h->stream,
-                         (const double *)U.p, (float *)g.q, (float *)g.ff, la, op);
-  } else {
-    if (wq)
-      hipLaunchKernelGGL((ldg_grad_kernel<N, E, double, double, true>), grid, block, 0, h->stream,
-                         (const double *)U.p, (double *)g.q, (double *)g.ff, la, op);
-    else
-      hipLaunchKernelGGL((ldg_grad_kernel<N, E, double, double, false>), grid, block, 0, h->stream,
-                         (const double *)U.p, (double *)g.q, (double *)g.ff, la, op);
-  }
+  if (h->mixed && U.fluct)
+    hipLaunchKernelGGL((ldg_nodal_grad_kernel<N, E, float, float>), grid, block, 0, h->stream, (const float *)U.p,
+                       (float *)g.q, la, op);
+  else if (h->mixed)
+    hipLaunchKernelGGL((ldg_nodal_grad_kernel<N, E, float, double>), grid, block, 0, h->stream, (const double *)U.p,
+                       (float *)g.q, la, op);
+  else
+    hipLaunchKernelGGL((ldg_nodal_grad_kernel<N, E, double, double>), grid, block, 0, h->stream, (const double *)U.p,
+                       (double *)g.q, la, op);
 }
 
 template <int N, int E>
 void launch_rhs_e(ldg_handle *h, Group &g, const Tiling &t, StageIn U, const StageArgs &st) {
-  LaunchArgs la{t.d_inst, t.d_blk, t.nblocks, (t.nblocks + 7) / 8};
+  const LaunchArgs la = launch_args(g, t);
   const unsigned char *img = (const unsigned char *)g.sops;
-  const dim3 grid(8 * la.per_xcd), block(NT);
+  const dim3 grid(8 * la.per_xcd), block(Shape<N, E>::NTH);
+  if (st.diag_part) {   // diagnostics of the FP64 state
+    if (h->mixed)
+      hipLaunchKernelGGL((ldg_rhs_kernel<N, E, float, double, true>), grid, block, 0, h->stream, (const double *)U.p,
+                         (const float *)g.ff, la, img, st);
+    else
+      hipLaunchKernelGGL((ldg_rhs_kernel<N, E, double, double, true>), grid, block, 0, h->stream, (const double *)U.p,
+                         (const double *)g.ff, la, img, st);
+    return;
+  }
   if (h->mixed && U.fluct)
-    hipLaunchKernelGGL((ldg_rhs_kernel<N, E, float, float>), grid, block, 0, h->stream, (const float *)U.p,
+    hipLaunchKernelGGL((ldg_rhs_kernel<N, E, float, float, false>), grid, block, 0, h->stream, (const float *)U.p,
                        (const float *)g.ff, la, img, st);
   else if (h->mixed)
-    hipLaunchKernelGGL((ldg_rhs_kernel<N, E, float, double>), grid, block, 0, h->stream, (const double *)U.p,
+    hipLaunchKernelGGL((ldg_rhs_kernel<N, E, float, double, false>), grid, block, 0, h->stream, (const double *)U.p,
                        (const float *)g.ff, la, img, st);
   else
-    hipLaunchKernelGGL((ldg_rhs_kernel<N, E, double, double>), grid, block, 0, h->stream, (const double *)U.p,
+    hipLaunchKernelGGL((ldg_rhs_kernel<N, E, double, double, false>), grid, block, 0, h->stream, (const double *)U.p,
                        (const double *)g.ff, la, img, st);
 }
 
 template <int N>
 void launch_grad_n(ldg_handle *h, Group &g, int c, StageIn U, bool wq) {
-  if (c == 0) launch_grad_e<N, Cand<N>::grad[0]>(h, g, g.grad[0], U, wq);
-  else launch_grad_e<N, Cand<N>::grad[1]>(h, g, g.grad[1], U, wq);
+  if (c == 0) launch_grad_e<N, Cand<N>::grad[0]>(h, g, g.grad[0], U);
+  else launch_grad_e<N, Cand<N>::grad[1]>(h, g, g.grad[1], U);
+  if (wq) launch_nodal_n<N>(h, g, U);
 }
 
 template <int N>
@@ -247,14 +289,12 @@ int upload_ops_t(ldg_handle *h, Group &g) {
   if (!(asym < 1e-9)) return fail(h, LDG_EINVAL, "1D operators are not centro-symmetric (node sets must be symmetric)");
   HIPCHECK(h, hipMalloc(&g.ops, sizeof(o)));
   HIPCHECK(h, hipMemcpy(g.ops, &o, sizeof(o), hipMemcpyHostToDevice));
-  // the rhs kernel's operator images, one per member (slot order)
-  std::vector<unsigned char> img((size_t)SOpsImage<N>::BYTES * g.members.size(), 0);
+  // the kernels' operator images, one per member (slot order)
+  std::vector<unsigned char> img((size_t)GImage<N>::BYTES * g.members.size(), 0);
   for (size_t j = 0; j < g.members.size(); ++j) {
     const Inst &in = h->inst[g.members[j]];
     const double a[3] = {2.0 / in.dx[0], 2.0 / in.dx[1], 2.0 / in.dx[2]};
-    unsigned char *b = img.data() + j * SOpsImage<N>::BYTES;
-    fill_sops<N, float>(*reinterpret_cast<SOps<N, float> *>(b + SOpsImage<N>::template offset<float>()), o, a);
-    fill_sops<N, double>(*reinterpret_cast<SOps<N, double> *>(b + SOpsImage<N>::template offset<double>()), o, a);
+    fill_image<N>(img.data() + j * GImage<N>::BYTES, o, a);
   }
   HIPCHECK(h, hipMalloc(&g.sops, img.size()));
   HIPCHECK(h, hipMemcpy(g.sops, img.data(), img.size(), hipMemcpyHostToDevice));
@@ -274,7 +314,9 @@ int upload_ops(ldg_handle *h, Group &g) {
 
 // Instance table entry of instance `in` for a tiling of E elements per
 // workgroup, with its first element and first logical workgroup.
-int inst_desc(const ldg_config &cfg, const Inst &in, int E, long elem_off, int block_off, InstDesc &d) {
+// The gradient and right-hand-side kernels number their workgroups by spans
+// of elements, the nodal gradient kernel (bricks) by bricks.
+int inst_desc(const ldg_config &cfg, const Inst &in, int E, bool bricks, long elem_off, int block_off, InstDesc &d) {
   std::memset(&d, 0, sizeof(d));
   d.nx = in.nx; d.ny = in.ny; d.nz = in.nz;
   d.nelem = in.K;
@@ -288,8 +330,12 @@ int inst_desc(const ldg_config &cfg, const Inst &in, int E, long elem_off, int b
   d.nbrick[0] = (d.nbx + d.tb[0] - 1) / d.tb[0];
   d.nbrick[1] = (in.ny + d.tb[1] - 1) / d.tb[1];
   d.nbrick[2] = (in.nz + d.tb[2] - 1) / d.tb[2];
-  const long nb = (long)d.nbrick[0] * d.nbrick[1] * d.nbrick[2] * d.tb[0] * d.tb[1] * d.tb[2];
+  long nb = (long)d.nbrick[0] * d.nbrick[1] * d.nbrick[2] * d.tb[0] * d.tb[1] * d.tb[2];
   if (nb > (1L << 30)) return LDG_EINVAL;
+  if (!bricks) {
+    nb = make_spans(d, in.p + 1, E);
+    if (nb > (1L << 30) || in.K > 0x7fffffffL) return LDG_EINVAL;
+  }
   d.nblocks = (int)nb;
   d.block_off = block_off;
   for (int l = 0; l < 3; ++l) d.ialpha[l] = 2.0 / in.dx[l];
@@ -303,7 +349,7 @@ int inst_desc(const ldg_config &cfg, const Inst &in, int E, long elem_off, int b
   return LDG_OK;
 }
 
-int build_tiling(ldg_handle *h, Group &g, Tiling &t, int E) {
+int build_tiling(ldg_handle *h, Group &g, Tiling &t, int E, bool bricks = false) {
   t.E = E;
   t.h_inst.clear();
   std::vector<int> blk;
@@ -312,7 +358,7 @@ int build_tiling(ldg_handle *h, Group &g, Tiling &t, int E) {
   for (int idx : g.members) {
     const Inst &in = h->inst[idx];
     InstDesc d;
-    if (inst_desc(h->cfg, in, E, off, boff, d) != LDG_OK)
+    if (inst_desc(h->cfg, in, E, bricks, off, boff, d) != LDG_OK)
       return fail(h, LDG_EINVAL, "mesh too large for the block numbering");
     for (int b = 0; b < d.nblocks; ++b) blk.push_back(in.slot);
     off += in.K;
@@ -432,6 +478,7 @@ int create_impl(const ldg_config *cfg, const ldg_instance *insts, int n, ldg_han
         return bad(LDG_EDEVICE);
       maxblk = std::max(maxblk, g.rhs[c].nblocks);
     }
+    if (build_tiling(h, g, g.nodal, nodal_e(g.n), true)) return bad(LDG_EDEVICE);
     std::vector<double> sc;
     for (int idx : g.members) sc.push_back(ke_scale(h->cfg, h->inst[idx]));
     if (hipMalloc((void **)&g.ke_part, sizeof(double) * (maxblk + 1)) != hipSuccess ||
@@ -771,6 +818,7 @@ void ldg_destroy(ldg_handle *h) {
     if (g.ops) (void)hipFree(g.ops);
     if (g.sops) (void)hipFree(g.sops);
     for (int c = 0; c < kMaxCand; ++c) { free_tiling(g.rhs[c]); free_tiling(g.grad[c]); }
+    free_tiling(g.nodal);
     closure_release(g);
   }
   if (h->ke_hist) (void)hipFree(h->ke_hist);
@@ -929,20 +977,14 @@ int ldg_set_graph(ldg_handle *h, int enable) {
 int ldg_instance_diagnostics(ldg_handle *h, int i, double out[3]) {
   if (!h || !out || i < 0 || i >= (int)h->inst.size()) return LDG_EINVAL;
   const int ni = (int)h->inst.size();
-  // one zero-length RK epilogue per group (acc = u + 0 k) gives the nodal KE
-  // of u; the Gauss-point sums come from the volume phase of the same launch
+  // the nodal and the Gauss-point sums of u per workgroup, from the state and
+  // its volume gradient alone (no face fluxes, nothing is written back)
   int first = 0;
   for (Group &g : h->groups) {
-    int rc = launch_grad(h, g, state_in(g.u));
-    if (rc) return rc;
     StageArgs st = empty_stage();
-    st.u0 = g.u;
-    st.acc = g.acc;
-    st.acc_init = 1;
-    st.cb = 0.0;
     st.ke_part = g.ke_part;
     st.diag_part = g.diag_part;
-    rc = launch_rhs(h, g, state_in(g.u), st);
+    const int rc = launch_rhs(h, g, state_in(g.u), st);
     if (rc) return rc;
     const Tiling &t = g.rhs[g.crhs];
     hipLaunchKernelGGL(ldg_finalize_kernel, dim3(g.members.size()), dim3(NT), 0, h->stream, (const double *)g.ke_part,
@@ -1103,14 +1145,10 @@ static __device__ __align__(256) unsigned char scratch[LDG_NOALLOC_SCRATCH_BYTES
 
 namespace ldg_host {
 
-constexpr size_t kScrOps = 0, kScrInstGrad = 4096, kScrInstRhs = 6144, kScrFF = 8192;
-// the rhs kernel's operator image of the precision in use follows the
-// operators in their slot
-template <int N>
-constexpr size_t kScrImg = kScrOps + (sizeof(Ops<N, double>) + 15) / 16 * 16;
-static_assert(kScrImg<6> + SOpsImage<6>::D <= kScrInstGrad && SOpsImage<6>::F <= SOpsImage<6>::D,
-              "operators do not fit their scratch slot");
-static_assert(sizeof(InstDesc) <= kScrInstRhs - kScrInstGrad, "instance table does not fit its scratch slot");
+constexpr size_t kScrImg = 0, kScrInstGrad = 5120, kScrInstRhs = 6656, kScrFF = 8192;
+static_assert(GImage<6>::BYTES <= kScrInstGrad, "the operator image does not fit its scratch slot");
+static_assert(sizeof(InstDesc) <= kScrInstRhs - kScrInstGrad && sizeof(InstDesc) <= kScrFF - kScrInstRhs,
+              "an instance table does not fit its scratch slot");
 
 constexpr int kMaxDevices = 64;
 std::mutex g_scratch_mu;
@@ -1176,43 +1214,30 @@ hipError_t noalloc_launch(const ldg_config &cfg, const Inst &in, unsigned char *
                           hipStream_t s, InstDesc dsc[2], unsigned char *img) {
   constexpr int EG = Cand<N>::grad[0], ER = Cand<N>::rhs[0];
   const Ops<N, double> &o = ops_of<N>(ops_tables());
-  if (inst_desc(cfg, in, EG, 0, 0, dsc[0]) != LDG_OK || inst_desc(cfg, in, ER, 0, 0, dsc[1]) != LDG_OK)
+  if (inst_desc(cfg, in, EG, false, 0, 0, dsc[0]) != LDG_OK || inst_desc(cfg, in, ER, false, 0, 0, dsc[1]) != LDG_OK)
     return hipErrorInvalidValue;
-  // the image of the precision in use only, at kScrImg; the kernel is given
-  // the base from which that image's offset lands there
   const double a[3] = {dsc[1].ialpha[0], dsc[1].ialpha[1], dsc[1].ialpha[2]};
-  const bool mixed = cfg.precision == LDG_MIXED;
-  if (mixed) fill_sops<N, float>(*reinterpret_cast<SOps<N, float> *>(img), o, a);
-  else fill_sops<N, double>(*reinterpret_cast<SOps<N, double> *>(img), o, a);
-  const size_t ib = mixed ? sizeof(SOps<N, float>) : sizeof(SOps<N, double>);
-  const unsigned char *simg =
-      scr + kScrImg<N> - (mixed ? SOpsImage<N>::template offset<float>() : SOpsImage<N>::template offset<double>());
-  hipError_t e = hipMemcpyAsync(scr + kScrOps, &o, sizeof(o), hipMemcpyHostToDevice, s);
-  if (e == hipSuccess) e = hipMemcpyAsync(scr + kScrImg<N>, img, ib, hipMemcpyHostToDevice, s);
+  fill_image<N>(img, o, a);
+  hipError_t e = hipMemcpyAsync(scr + kScrImg, img, GImage<N>::BYTES, hipMemcpyHostToDevice, s);
   if (e == hipSuccess) e = hipMemcpyAsync(scr + kScrInstGrad, &dsc[0], sizeof(InstDesc), hipMemcpyHostToDevice, s);
   if (e == hipSuccess) e = hipMemcpyAsync(scr + kScrInstRhs, &dsc[1], sizeof(InstDesc), hipMemcpyHostToDevice, s);
   if (e != hipSuccess) return e;
-  const Ops<N, double> *op = reinterpret_cast<const Ops<N, double> *>(scr + kScrOps);
   const LaunchArgs lg{reinterpret_cast<const InstDesc *>(scr + kScrInstGrad), nullptr, dsc[0].nblocks,
-                      (dsc[0].nblocks + 7) / 8};
+                      (dsc[0].nblocks + 7) / 8, in.K};
   const LaunchArgs lr{reinterpret_cast<const InstDesc *>(scr + kScrInstRhs), nullptr, dsc[1].nblocks,
-                      (dsc[1].nblocks + 7) / 8};
+                      (dsc[1].nblocks + 7) / 8, in.K};
+  const dim3 gg(8 * lg.per_xcd), gr(8 * lr.per_xcd), bg(Shape<N, EG>::NTH), br(Shape<N, ER>::NTH);
+  const unsigned char *simg = scr + kScrImg;
   StageArgs st = empty_stage();
   st.kout = k;
-  // the gradient kernel writes no nodal gradient here (WQ = false): the
-  // scratch holds the face fluxes only
   if (cfg.precision == LDG_MIXED) {
     float *ff = reinterpret_cast<float *>(scr + kScrFF);
-    hipLaunchKernelGGL((ldg_grad_kernel<N, EG, float, double, false>), dim3(8 * lg.per_xcd), dim3(NT), 0, s, u,
-                       nullptr, ff, lg, op);
-    hipLaunchKernelGGL((ldg_rhs_kernel<N, ER, float, double>), dim3(8 * lr.per_xcd), dim3(NT), 0, s, u,
-                       (const float *)ff, lr, simg, st);
+    hipLaunchKernelGGL((ldg_grad_kernel<N, EG, float, double>), gg, bg, 0, s, u, ff, lg, simg);
+    hipLaunchKernelGGL((ldg_rhs_kernel<N, ER, float, double, false>), gr, br, 0, s, u, (const float *)ff, lr, simg, st);
   } else {
     double *ff = reinterpret_cast<double *>(scr + kScrFF);
-    hipLaunchKernelGGL((ldg_grad_kernel<N, EG, double, double, false>), dim3(8 * lg.per_xcd), dim3(NT), 0, s, u,
-                       nullptr, ff, lg, op);
-    hipLaunchKernelGGL((ldg_rhs_kernel<N, ER, double, double>), dim3(8 * lr.per_xcd), dim3(NT), 0, s, u,
-                       (const double *)ff, lr, simg, st);
+    hipLaunchKernelGGL((ldg_grad_kernel<N, EG, double, double>), gg, bg, 0, s, u, ff, lg, simg);
+    hipLaunchKernelGGL((ldg_rhs_kernel<N, ER, double, double, false>), gr, br, 0, s, u, (const double *)ff, lr, simg, st);
   }
   return hipGetLastError();
 }
@@ -1259,7 +1284,7 @@ extern "C" int ldg_rhs_noalloc(const ldg_config *cfg, const double *u, double *k
   if (!scr) return LDG_EDEVICE;
   hipStream_t s = static_cast<hipStream_t>(stream);
   InstDesc dsc[2];
-  alignas(16) unsigned char img[SOpsImage<6>::D];   // (read by the copies until the synchronisation below)
+  alignas(16) unsigned char img[GImage<6>::BYTES];   // (read by the copies until the synchronisation below)
   hipError_t e = hipErrorInvalidValue;
   switch (n) {
     case 2: e = noalloc_launch<2>(*cfg, in, scr, u, k, s, dsc, img); break;

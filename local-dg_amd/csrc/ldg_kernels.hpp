@@ -3,17 +3,18 @@
 // One RK4 stage is two launches over the whole periodic mesh:
 //   ldg_grad_kernel  auxiliary gradient Q_l = (1/alpha_l)(Dn U + L0 jump_l)
 //                    (Solver::rk4Rhs first half, solver.cpp:490-508) on the
-//                    faces, the Roe + one-sided viscous face fluxes of both
+//                    faces and the Roe + one-sided viscous face fluxes of both
 //                    elements of every face (solver.cpp:643-698, 750-814,
-//                    891-921, 1194-1374), lifted to the face nodes
+//                    891-921, 1194-1374)
 //   ldg_rhs_kernel   the volume gradient and volume integrals, minus the
-//                    lifted face terms, inverse mass and the fused RK4
-//                    stage epilogue (solver.cpp:510-535 and 410-434)
+//                    face terms, inverse mass and the fused RK4 stage
+//                    epilogue (solver.cpp:510-535 and 410-434)
 // Both stage a block of E consecutive elements in LDS, work in 1D "lines"
-// of N = p+1 values owned by one thread (in-place sum-factorised sweeps,
-// with the even/odd split of the centro-symmetric 1D operators, symop.hpp),
-// and read the periodic neighbours' face slices straight from HBM (the
-// on-device form of the single-rank halo exchange, solver.cpp:929-998).
+// of N = p+1 values owned by one thread (in-place sum-factorised sweeps in
+// Gauss form, see GOps, with the even/odd split of the centro-symmetric 1D
+// operators, symop.hpp), and read the periodic neighbours' face slices
+// straight from HBM (the on-device form of the single-rank halo exchange,
+// solver.cpp:929-998).
 //
 // Precision: the state, the RK4 combination, the inverse mass and every
 // reduction are FP64.  The interpolation, flux evaluation and test-function
@@ -29,13 +30,17 @@
 //   u0, acc, unext : FP64 (node, state, element) -- the reference layout
 //   U (stage input): the same, or in the mixed path (RK stages 2-4) FP32
 //                    fluctuations about the background in that layout
-//   FF             : T, per element [direction][side][state][face node]:
-//                    the lifted face fluxes (gradient kernel -> rhs kernel)
+//   FF             : T, [direction][side][state][element][face Gauss point]:
+//                    the face fluxes (gradient kernel -> rhs kernel)
 //   Q              : TQ (node, s + 5*l, element) -- the nodal gradient, 15
 //                    fields per element, written only when asked for
 #pragma once
 
 #include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <cmath>
+#include <type_traits>
 
 #include "symop.hpp"
 
@@ -53,10 +58,12 @@ struct Ops {
   T Dn[N][N];     // Dn[i][j] = l_j'(r_i)
   T Minv[N][N];   // inverse 1D mass matrix
   T L0[N];        // Minv[:, 0]: lift of the jump at the left face
-  T IL0[N];       // I L0: that lift at the Gauss points
   T w[N];         // Gauss weights
-  // the sweep operators in even/odd split form: I, I^T, D^T, Minv, D
-  SymMat<N, T> sI, sIt, sDt, sMi, sD;
+  T eta[N];       // L_q(-1) / w_q: that lift in Gauss form (I L0)
+  // sweep operators in even/odd split form: I, D = I Dn, I^-1, the
+  // derivative Dg at the Gauss points of the polynomial through them, and
+  // W^-1 Dg^T W
+  SymMat<N, T> sI, sD, sIi, sDg, sDh;
 };
 
 struct MeshArgs {
@@ -124,6 +131,16 @@ struct InstDesc {
   int tb[3];             // brick of tb[0] x tb[1] x tb[2] blocks (x blocks, y rows, z planes)
   int nbrick[3];         // bricks per direction
   FastDiv div_bs, div_nb0, div_nb1, div_tb0, div_tb1;   // by tb0 tb1 tb2, nbrick[0], nbrick[1], tb[0], tb[1]
+  // spans (see span_elements): ncy strips of rows, cut into ncx columns of
+  // pieces of rows (ncx = 0: whole rows)
+  int ncx, ncy, nbr;                     // nbr: workgroups per row (pieces) or per strip plane (whole rows)
+  int rows, main_blocks;                 // whole rows: rows per strip, workgroups of all strips but the last
+  FastDiv div_nx, div_ny, div_nz;
+  FastDiv div_row, div_nbr;              // by nz nbr (pieces) and nbr
+  FastDiv div_last;                      // by the last strip's workgroups per plane
+  int h0, w0;                            // strip heights h0, h0 + 1; column widths w0, w0 + 1
+  FastDiv div_ncx, div_ncy;
+  FastDiv div_col[2], div_pl[2][2], div_w[2];   // by h nz, h w, w
   double ialpha[3];      // 2 / dx_l
   double dt;             // its time step
   PhysArgs ph;
@@ -151,11 +168,108 @@ __host__ __device__ inline void block_elements(const InstDesc &d, int E, int lbl
   ne = (d.nx - ec[0]) < E ? (d.nx - ec[0]) : E;
 }
 
+// Elements of an instance's logical workgroup lbl in the span numbering of
+// the gradient and right-hand-side kernels: E consecutive elements kl ..
+// kl + ne - 1 (ne < E only at the end of a run; there are no empty
+// workgroups).  The mesh is cut into columns along z that are walked plane by
+// plane: strips of rows in y and, where rows are long, pieces of rows in x,
+// the strip heights (and piece widths, in workgroups) differing by at most
+// one.  The traces a workgroup gathers from its -y and -z neighbours were
+// read one row and one plane of the column earlier and are still in the XCD's
+// L2.  Whole rows of a strip are consecutive elements, so there a run is the
+// strip's part of a plane.
+__host__ __device__ inline void span_elements(const InstDesc &d, int E, int lbl, int &kl, int &ne) {
+  int start, len, j;
+  if (d.ncx == 0) {
+    int st, z;
+    if (lbl < d.main_blocks) {
+      const int run = d.div_nbr.div(lbl);
+      j = lbl - run * d.nbr;
+      st = d.div_nz.div(run);
+      z = run - st * d.nz;
+    } else {
+      const int r = lbl - d.main_blocks, last = d.ny - (d.ncy - 1) * d.rows, nb = (last * d.nx + E - 1) / E;
+      st = d.ncy - 1;
+      z = d.div_last.div(r);
+      j = r - z * nb;
+    }
+    const int y0 = st * d.rows;
+    start = (z * d.ny + y0) * d.nx;
+    len = (d.ny - y0 < d.rows ? d.ny - y0 : d.rows) * d.nx;
+  } else {
+    // strip i has rows floor(i ny / ncy) .. floor((i + 1) ny / ncy) - 1, so
+    // row y is in strip floor(((y + 1) ncy - 1) / ny); columns alike
+    const int st = d.div_ny.div((d.div_row.div(lbl) + 1) * d.ncy - 1);
+    const int y0 = d.div_ncy.div(st * d.ny), h = d.div_ncy.div((st + 1) * d.ny) - y0, hi = h - d.h0;
+    const int r = lbl - y0 * d.nz * d.nbr;
+    const int cx = d.div_nbr.div((d.div_col[hi].div(r) + 1) * d.ncx - 1);
+    const int b0 = d.div_ncx.div(cx * d.nbr), w = d.div_ncx.div((cx + 1) * d.nbr) - b0, wi = w - d.w0;
+    const int q = r - b0 * h * d.nz;
+    const int z = d.div_pl[hi][wi].div(q), p = q - z * h * w;
+    const int y = d.div_w[wi].div(p);
+    start = (z * d.ny + y0 + y) * d.nx;
+    len = d.nx;
+    j = b0 + p - y * w;
+  }
+  kl = start + j * E;
+  ne = len - j * E < E ? len - j * E : E;
+}
+
+// Sets d's span numbering (d.nx, ny, nz, nelem given) for workgroups of E
+// elements with n nodes per direction; returns the number of workgroups.  A
+// column's part of a plane is about 1 MB of FP64 state: with the face fluxes
+// the two planes in use at a time fill about the 4 MB of an XCD's L2.
+// Columns about as wide as deep cost the fewest reads across their sides
+// (64^3, p = 4, FP64: the gradient kernel reads 1.2x the state instead of
+// 1.8x with columns of single rows).
+inline long make_spans(InstDesc &d, int n, int E) {
+  const double el = 8.0 * NSTATE * n * n * n, want = 1024.0 * 1024;
+  const double side = std::sqrt(want / el);               // elements
+  long nb;
+  if (d.nx <= 1.5 * side) {                               // whole rows
+    d.ncx = 0;
+    const int r = std::max(1, (int)(want / (el * d.nx)));
+    d.ncy = (d.ny + r - 1) / r;
+    d.rows = (d.ny + d.ncy - 1) / d.ncy;
+    d.ncy = (d.ny + d.rows - 1) / d.rows;
+    const int last = d.ny - (d.ncy - 1) * d.rows;
+    d.nbr = (int)(((long)d.rows * d.nx + E - 1) / E);
+    const long nl = ((long)last * d.nx + E - 1) / E, main = (long)(d.ncy - 1) * d.nz * d.nbr;
+    nb = main + nl * d.nz;
+    if (nb > (1L << 30)) return nb;
+    d.main_blocks = (int)main;
+    d.div_last = make_fastdiv((int)nl);
+  } else {
+    d.nbr = (d.nx + E - 1) / E;
+    d.ncx = std::max(1, (int)(d.nx / side + 0.5));
+    d.ncx = std::min(d.ncx, d.nbr);
+    d.ncy = std::min(d.ny, std::max(1, (int)(d.ny / side + 0.5)));
+    nb = (long)d.nbr * d.ny * d.nz;
+    if (nb > (1L << 30)) return nb;
+    d.h0 = d.ny / d.ncy;
+    d.w0 = d.nbr / d.ncx;
+    d.div_row = make_fastdiv(d.nz * d.nbr);
+    d.div_ncx = make_fastdiv(d.ncx);
+    d.div_ncy = make_fastdiv(d.ncy);
+    for (int a = 0; a < 2; ++a) {
+      d.div_col[a] = make_fastdiv((d.h0 + a) * d.nz);
+      d.div_w[a] = make_fastdiv(d.w0 + a);
+      for (int b = 0; b < 2; ++b) d.div_pl[a][b] = make_fastdiv((d.h0 + a) * (d.w0 + b));
+    }
+  }
+  d.div_nbr = make_fastdiv(d.nbr);
+  d.div_nx = make_fastdiv(d.nx);
+  d.div_ny = make_fastdiv(d.ny);
+  d.div_nz = make_fastdiv(d.nz);
+  return nb;
+}
+
 struct LaunchArgs {
   const InstDesc *inst;
   const int *blk_inst;   // logical workgroup -> instance (nullptr: one instance)
   int nblocks;           // logical workgroups of the launch
   int per_xcd;           // ceil(nblocks / 8)
+  long nelem;            // elements of the launch (all instances)
 };
 
 // Workgroups are dispatched round-robin over the 8 XCDs; give each XCD a
@@ -165,6 +279,16 @@ __device__ inline int logical_block(const LaunchArgs &la) {
   const int b = blockIdx.x;
   const int lb = (b & 7) * la.per_xcd + (b >> 3);
   return lb < la.nblocks ? lb : -1;
+}
+
+__device__ inline int instance_of(const LaunchArgs &la, int lb) { return la.blk_inst ? la.blk_inst[lb] : 0; }
+
+// The instance of logical workgroup lb and the block's span of elements
+// (local to the instance).
+__device__ inline const InstDesc &block_span(const LaunchArgs &la, int lb, int E, int &kl, int &ne) {
+  const InstDesc &d = la.inst[instance_of(la, lb)];
+  span_elements(d, E, lb - d.block_off, kl, ne);
+  return d;
 }
 
 // The instance of logical workgroup lb, its mesh, and the block's first
@@ -370,146 +494,447 @@ __device__ inline double block_sum(double v, double *sw) {
 }
 
 // ---------------------------------------------------------------------
-// Kernel A: auxiliary gradient (solver.cpp:490-508, restated in strong
-// form: -M1^{-1} S1 + face lifts = Dn + M1^{-1} e_0 e_0^T, exactly), and
-// the face fluxes of the elements' negative faces.
+// The element's operators in Gauss form.
 //
-// Gradient: computed in the gradient's own type TQ (FP64, or FP32 in the
-// mixed path) from the fluctuation of the state about the background.
-// One thread per node computes all 15 components and stores them straight
-// to HBM (consecutive threads -> consecutive nodes, coalesced).
-//
-// Face fluxes: the face between an element N and its -d neighbour K needs
-// K's trace (already staged here for the gradient's jump term), N's trace
-// and N's gradient trace (the one-sided switch picks it for both sides), so
-// the workgroup that owns N evaluates that face once for both elements:
-// interpolation of the two states and the 11 gradient components the
-// viscous flux reads to the face Gauss points (two sweeps), then Roe +
-// viscous fluxes (face_flux_pair), weighted for the lift
-// (w_a w_b 2/dx_d), written to FF[element][d][side][state][face point] with
-// side 0 = N's own flux on its -d face and side 1 = K's flux on its +d face.
-// The right-hand-side kernel only lifts them.  In type TQ, on fluctuations
-// about the background, like the rest of the flux arithmetic.
+// A basis polynomial is as well given by its values at the N Gauss points
+// (u_g = I u) as by those at the nodes, and in that form every operator of
+// the scheme is a 1D derivative, a rank-1 face term, or I and its inverse:
+//   LDG gradient     Q_l = a_l (Dg u_g + eta J_l)             a_l = 2/dx_l
+//   volume + faces   k_g = sum_l a_l (Dh F_l) - eta f_l^- - eta' f_l^+
+//   rate             k   = (I^-1 (x) I^-1 (x) I^-1) k_g
+// with Dg the derivative at the Gauss points of the polynomial through
+// them, Dh = W^-1 Dg^T W, eta_q = L_q(-1) / w_q (L_q: Lagrange polynomial of
+// Gauss point q; eta'_q = eta_{N-1-q} for the + face), J_l the jump u - u_nbr
+// on the -l face and f_l the face fluxes times a_l, both at the face Gauss
+// points.  It is the weak form of the nodal scheme, exactly: M1 = I^T W I
+// (the rule integrates products of two basis polynomials exactly), so
+// M1^-1 I^T = I^-1 W^-1 turns the test functions and the inverse mass into
+// W^-1 in Gauss form, D^T = I^T Dg^T, and M1^-1 e_0 = I^-1 eta.
+// Against sweeping with I, D, I^T, D^T and M1^-1 at the nodes it needs 60
+// field sweeps of a line instead of 100, no weights at the points, and the
+// face fluxes stay at the face Gauss points (no lift).
 // ---------------------------------------------------------------------
-// Gradient components that the viscous flux across a face of direction D
-// reads (numericalFluxV, solver.cpp:891-921, with the face normal +-e_D:
-// the stress row sigma_D. and the heat flux along D): the derivatives of all
-// five conserved variables along D, and along each other direction l those
-// of rho, m_D and m_l -- 11 of the 15.  The other four enter the
-// reference's face flux multiplied by a zero normal component, so only
-// these are carried to the face points.  Slot j of direction D holds
-// component k = s + 5 l.
-constexpr int NFG = 11;
-__host__ __device__ constexpr int face_grad(int D, int j) {
-  return j < NSTATE ? j + NSTATE * D
-                    : ((j - NSTATE) % 3 == 0 ? 0 : (j - NSTATE) % 3 == 1 ? 1 + D : 1 + (D + 1 + (j - NSTATE) / 3) % 3) +
-                          NSTATE * ((D + 1 + (j - NSTATE) / 3) % 3);
-}
-
-// Occupancy target of the gradient kernel (waves per SIMD), which sets its
-// register budget: 5 with an FP32 gradient up to p = 4 (the face flux needs
-// more registers than the 80 of 6 waves), 4 with FP64 and at p = 5; never
-// more than its LDS footprint allows (one workgroup = one wave per SIMD,
-// 160 KiB of LDS per CU).
-template <int N, int E, typename TQ>
-struct GradWaves {
-  static constexpr int NFF = 2 * NSTATE + NFG;
-  static constexpr int lds = (int)sizeof(TQ) * (E * NSTATE * N * N * N + E * 3 * NFF * N * N + N * (N + 1) + N) +
-                             (int)sizeof(SymMat<N, TQ>) + 8 * 6 * E;
-  static constexpr int by_lds = (160 * 1024) / lds;
-  static constexpr int want = sizeof(TQ) == 4 && N <= 5 ? 5 : 4;
-  static constexpr int value = want < by_lds ? want : by_lds;
+template <int N, typename T>
+struct GOps {
+  SymMat<N, T> I;                          // nodes -> Gauss points
+  SymMat<N, T> Dg[3], Dh[3];               // a_l Dg, a_l Dh (l = x, y, z)
+  T eta[N];
+  T aeta[3][N];                            // a_l eta: the lift of J_l
+  // the face kernel: D = I Dn along the face (unscaled), the derivative
+  // along the normal at the - face node, a_d (Dn[0][:] + L0[0] e_0), and the
+  // neighbour's weight in it, -a_d L0[0]
+  SymMat<N, T> D;
+  T nrm[3][N];
+  T nbr[3];
+  T a[3];
+};
+template <int N>
+struct GOpsD {                             // FP64 in every path
+  SymMat<N, double> Ii;                    // Gauss points -> nodes
+  double w[N];                             // Gauss weights
 };
 
-// Face-flux array: per element, 3 directions x 2 sides, each a chunk of 5
-// states x N^2 face nodes.
-__host__ __device__ constexpr int ff_chunk(int n, int /*bytes*/) { return NSTATE * n * n; }
 template <int N, typename T>
-__host__ __device__ constexpr int ff_per_element() { return 6 * ff_chunk(N, (int)sizeof(T)); }
-
-// 16-byte vector of T
-template <typename T> struct Vec16;
-template <> struct Vec16<float> { using type = float4; };
-template <> struct Vec16<double> { using type = double2; };
-
-// Face fluxes of direction D at one face point: fp points at the point's
-// slot of field 0 (fields NF apart: own trace 0-4, neighbour's trace 5-9,
-// the gradient components face_grad(D, j) 10-20).
-template <typename C, int D, int NF>
-__device__ inline void face_point_flux(const C *fp, const Bg<C> &bg, C outK[5], C outN[5]) {
-  C wN[5], wK[5], q[NGRAD];
-#pragma unroll
-  for (int s = 0; s < NSTATE; ++s) { wN[s] = fp[s * NF]; wK[s] = fp[(NSTATE + s) * NF]; }
-#pragma unroll
-  for (int k = 0; k < NGRAD; ++k) q[k] = C(0);   // not read by the direction-D flux
-#pragma unroll
-  for (int j = 0; j < NFG; ++j) q[face_grad(D, j)] = fp[(2 * NSTATE + j) * NF];
-  face_flux_pair<C, D>(wK, wN, q, bg, outK, outN);
+void fill_gops(GOps<N, T> &g, const Ops<N, double> &op, const double a[3]) {
+  constexpr int MS = sizeof(SymMat<N, T>) / sizeof(T);
+  static_assert(sizeof(SymMat<N, double>) == MS * sizeof(double), "operators are plain coefficient arrays");
+  auto put = [&](SymMat<N, T> &d, const SymMat<N, double> &s, double f) {
+    for (int i = 0; i < MS; ++i) reinterpret_cast<T *>(&d)[i] = T(reinterpret_cast<const double *>(&s)[i] * f);
+  };
+  put(g.I, op.sI, 1.0);
+  put(g.D, op.sD, 1.0);
+  for (int l = 0; l < 3; ++l) {
+    put(g.Dg[l], op.sDg, a[l]);
+    put(g.Dh[l], op.sDh, a[l]);
+    for (int q = 0; q < N; ++q) {
+      g.aeta[l][q] = T(op.eta[q] * a[l]);
+      g.nrm[l][q] = T((op.Dn[0][q] + (q == 0 ? op.L0[0] : 0.0)) * a[l]);
+    }
+    g.nbr[l] = T(-op.L0[0] * a[l]);
+    g.a[l] = T(a[l]);
+  }
+  for (int q = 0; q < N; ++q) g.eta[q] = T(op.eta[q]);
 }
 
-// Gradient components of one -D face node for the face flux (the sums of
-// the full gradient at that node): along D the line through the node,
-// along the two other directions l lines in the face plane, each with the
-// lift of the jump on its -l face (the neighbour traces staged in sf); the
-// node's own trace with them.  su, sf: the element's state and face slots.
-template <int N, int D, int NFF, typename C>
-__device__ inline void face_node_grad(const C *__restrict__ su, C *__restrict__ sf, const C (*__restrict__ sD)[N + 1],
-                                      const double *ia, unsigned ab) {
-  constexpr int NN = N * N * N, NF = N * N;
-  constexpr unsigned ST[3] = {1, N, NF};   // memory stride along x, y, z
-  const unsigned a = ab % N, b = ab / N;
-  // the node (0, a, b), (a, 0, b) or (a, b, 0)
-  const unsigned c[3] = {D == 0 ? 0u : a, D == 0 ? a : D == 1 ? 0u : b, D == 2 ? 0u : b};
-  const unsigned node = c[0] + N * c[1] + NF * c[2];
-  C *fs = sf + D * NFF * NF + ab;
+// Operator image of one instance: FP64-only part, FP32 and FP64 operators,
+// each padded to 16 bytes.
+template <int N>
+struct GImage {
+  static constexpr int pad(size_t b) { return (int)((b + 15) / 16 * 16); }
+  static constexpr int OF = pad(sizeof(GOpsD<N>)), OD = OF + pad(sizeof(GOps<N, float>));
+  static constexpr int BYTES = OD + pad(sizeof(GOps<N, double>));
+  template <typename T>
+  __host__ __device__ static constexpr int offset() { return sizeof(T) == sizeof(double) ? OD : OF; }
+};
+template <int N>
+void fill_image(unsigned char *b, const Ops<N, double> &op, const double a[3]) {
+  GOpsD<N> &d = *reinterpret_cast<GOpsD<N> *>(b);
+  d.Ii = op.sIi;
+  for (int q = 0; q < N; ++q) d.w[q] = op.w[q];
+  fill_gops<N, float>(*reinterpret_cast<GOps<N, float> *>(b + GImage<N>::OF), op, a);
+  fill_gops<N, double>(*reinterpret_cast<GOps<N, double> *>(b + GImage<N>::OD), op, a);
+}
+
+// A wave-uniform constant object (an operator) through the scalar cache:
+// its coefficients become scalar registers, one of which a vector
+// instruction reads as an operand, so a sweep holds no coefficients in
+// vector registers and reads none from LDS.
+template <typename S, typename T>
+__device__ inline S uniform_load(const S *p) {
+  static_assert(sizeof(S) % sizeof(T) == 0, "whole words");
+  S s;
+  const __attribute__((address_space(4))) T *src = (const __attribute__((address_space(4))) T *)(unsigned long long)p;
+  T *d = reinterpret_cast<T *>(&s);
 #pragma unroll
-  for (int s = 0; s < NSTATE; ++s) {
-    const C *us = su + s * NN + node;
-    C q = sD[0][N] * sf[(D * NFF + NSTATE + s) * NF + ab];
+  for (int i = 0; i < (int)(sizeof(S) / sizeof(T)); ++i) d[i] = src[i];
+  return s;
+}
+
+// Workgroup shape of the two kernels: E elements, one thread per (element,
+// line) with N^2 lines per element; a thread works on the five variables of
+// its line at once, so a phase's addresses are computed once and all its
+// LDS and register accesses are at compile-time offsets from them.
+template <int N, int E>
+struct Shape {
+  static constexpr int NN = N * N * N, NF = N * N, EV = NSTATE * NN;
+  static constexpr int NTH = (E * NF + 63) / 64 * 64;
+};
+
+// Sum of one double per thread over a workgroup of NTH threads -> thread 0
+// (fixed order: butterfly in each wave, then the waves in order).
+template <int NTH>
+__device__ inline double group_sum(double v, double *sw) {
 #pragma unroll
-    for (int j = 0; j < N; ++j) q += sD[0][j] * us[j * ST[D]];
-    fs[s * NF] = us[0];
-    fs[(2 * NSTATE + s) * NF] = q * C(ia[D]);
+  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+  if constexpr (NTH > 64) {
+    if ((threadIdx.x & 63) == 0) sw[threadIdx.x >> 6] = v;
+    __syncthreads();
+    v = sw[0];
+#pragma unroll
+    for (int w = 1; w < NTH / 64; ++w) v += sw[w];
+    __syncthreads();
   }
+  return v;
+}
+
+// Face-flux array FF, T: 30 planes (direction 2 d + side, state), each of
+// the launch's elements x N^2 face Gauss points: the fluxes times a_d, side 0
+// the element's own -d face, side 1 its +d face (written by the +d
+// neighbour's workgroup, see ldg_grad_kernel).  Plane-major, so that a
+// workgroup's threads (element, point) read and write each plane in one
+// contiguous piece.
+__host__ __device__ constexpr int ff_chunk(int n, int /*bytes*/) { return NSTATE * n * n; }
+
+// Coordinates of element kl of an instance.
+__host__ __device__ inline void element_coords(const InstDesc &d, int kl, int c[3]) {
+  const int row = d.div_nx.div(kl);
+  c[0] = kl - row * d.nx;
+  c[2] = d.div_ny.div(row);
+  c[1] = row - c[2] * d.ny;
+}
+// Element number difference to the periodic neighbour along axis l (dir +-1).
+__host__ __device__ inline int neighbor_step(const InstDesc &d, const int c[3], int l, int dir) {
+  const int n = l == 0 ? d.nx : l == 1 ? d.ny : d.nz, st = l == 0 ? 1 : l == 1 ? d.nx : d.nx * d.ny;
+  const bool wrap = dir > 0 ? c[l] == n - 1 : c[l] == 0;
+  return wrap ? -dir * (n - 1) * st : dir * st;
+}
+
+// The stage input as the fluctuation about the background in type T.  An
+// FP64 input in the mixed path (RK stage 1 of a call) is rounded to the
+// FP32 fluctuation the other stages read, so a step's result does not depend
+// on which form its input came in.
+template <typename T, typename UT>
+__device__ inline T fluctuation(UT x, int s, double rho0, double E0) {
+  if constexpr (sizeof(UT) == 4) return T(x);
+  else return T((double)x - (s == 0 ? rho0 : s == 4 ? E0 : 0.0));
+}
+
+// ---------------------------------------------------------------------
+// Kernel A: the fluxes of the elements' -d faces, for both sides.
+//
+// The face between an element N and its -d neighbour K needs K's trace, N's
+// trace and N's gradient trace (the one-sided switch picks it for both
+// sides), so the workgroup that owns N evaluates that face once for both
+// elements: the two traces, the normal derivative at the face nodes
+// (a_d (Dn u + L0 J)_0) and, along the face, the derivatives of the
+// variables the viscous flux reads (rho, m_D and the momentum along that
+// direction), each interpolated or differentiated to the face Gauss points
+// by two sweeps in the face plane, then Roe + viscous fluxes
+// (face_flux_pair).  A derivative along l in the face plane carries the lift
+// of the jump on the element's -l face, at the edge the two faces share: for
+// the first sweep direction that is the neighbour's nodal trace there, for
+// the second the same interpolated along the first (sedge).
+//
+// Threads: at nodes and points (element, point); the sweeps of one
+// direction are (variable, line) items over the whole workgroup, each doing
+// the line of the own trace, of the neighbour's trace, of the normal
+// derivative and of the in-face derivative, which share their addresses.
+// The three directions take turns in one set of face fields, with the own
+// traces and normal derivatives waiting in registers: against all three at
+// once the LDS footprint is 915 instead of 1620 values per element (p = 4;
+// 0.56 -> 0.41 ms mixed, 1.20 -> 0.89 ms FP64 at 64^3 with the column
+// numbering of span_elements).
+//
+// Measured at 64^3, p = 4: mixed 0.41 ms (0.68 with the gradient at the face
+// nodes, 21 interpolated fields and lifted fluxes), bound by vector issue (91 %
+// of it); FP64 0.89 ms (1.22), vector issue and LDS at 52 % each.
+// ---------------------------------------------------------------------
+template <int N, int E, typename T>
+struct GradLds {
+  using S = Shape<N, E>;
+  static constexpr int FS = E * S::NF;                     // one field
+  static constexpr int NFIELD = 21;                        // own 0-4, nbr 5-9, normal 10-14, d/da 15-17, d/db 18-20
+  static constexpr int NB = 3 * NSTATE * FS;               // the neighbours' nodal traces
+  static constexpr int BUF = NB + NFIELD * FS > E * S::EV ? NB + NFIELD * FS : E * S::EV;
+  static constexpr int EDGE = 3 * E * N;
+  static constexpr int WAVES = sizeof(T) == 4 ? 4 : 2;
+};
+
+// Fluxes of direction D at one face point: fp points at the point in field
+// 0 of the direction, fields FS apart.
+template <typename T, int D, int FS>
+__device__ inline void face_point_flux(const T *fp, const Bg<T> &bg, T outK[5], T outN[5]) {
+  constexpr int la = D == 0 ? 1 : 0, lb = D == 2 ? 1 : 2;
+  T wN[5], wK[5], q[NGRAD];
 #pragma unroll
-  for (int t = 0; t < 2; ++t) {
-    const int l = (D + 1 + t) % 3;
-    const unsigned il = c[l];
-    // the node's coordinates on the -l face
-    const unsigned abl = l == 0 ? c[1] + N * c[2] : l == 1 ? c[0] + N * c[2] : c[0] + N * c[1];
-    const unsigned start = node - il * ST[l];
-    const C *row = sD[il];
+  for (int s = 0; s < NSTATE; ++s) { wN[s] = fp[s * FS]; wK[s] = fp[(NSTATE + s) * FS]; }
 #pragma unroll
-    for (int idx = 0; idx < 3; ++idx) {
-      const int s = idx == 0 ? 0 : idx == 1 ? 1 + D : 1 + l;
-      const C *us = su + s * NN + start;
-      C q = row[N] * sf[(l * NFF + NSTATE + s) * NF + abl];
+  for (int k = 0; k < NGRAD; ++k) q[k] = T(0);   // the rest is not read by the direction-D flux
 #pragma unroll
-      for (int j = 0; j < N; ++j) q += row[j] * us[j * ST[l]];
-      fs[(2 * NSTATE + NSTATE + 3 * t + idx) * NF] = q * C(ia[l]);
+  for (int s = 0; s < NSTATE; ++s) q[s + NSTATE * D] = fp[(2 * NSTATE + s) * FS];
+  q[0 + NSTATE * la] = fp[15 * FS];
+  q[1 + D + NSTATE * la] = fp[16 * FS];
+  q[1 + la + NSTATE * la] = fp[17 * FS];
+  q[0 + NSTATE * lb] = fp[18 * FS];
+  q[1 + D + NSTATE * lb] = fp[19 * FS];
+  q[1 + lb + NSTATE * lb] = fp[20 * FS];
+  face_flux_pair<T, D>(wK, wN, q, bg, outK, outN);
+}
+
+template <int N, int E, typename T, typename UT>
+__global__ void __launch_bounds__((Shape<N, E>::NTH), (GradLds<N, E, T>::WAVES))
+ldg_grad_kernel(const UT *__restrict__ U, T *__restrict__ FF, LaunchArgs la, const unsigned char *__restrict__ img) {
+  using S = Shape<N, E>;
+  using L = GradLds<N, E, T>;
+  constexpr int NN = S::NN, NF = S::NF, EV = S::EV, NTH = S::NTH, FS = L::FS;
+  __shared__ __align__(16) T sb[L::BUF];     // the block's state, then the neighbours' traces and the face fields
+  __shared__ T sedge[L::EDGE];               // edge values of the second sweep direction's -l neighbour
+  const int lb = logical_block(la);
+  if (lb < 0) return;
+  int kl, ne;
+  const InstDesc &d = block_span(la, lb, E, kl, ne);
+  if (ne <= 0) return;
+  const long k0 = d.elem_off + kl;
+  const int t = threadIdx.x, e = t / NF, ab = t - e * NF, b = ab / N, a = ab - b * N;
+  const bool act = e < ne;
+  const GOps<N, T> *const op =
+      reinterpret_cast<const GOps<N, T> *>(img + (long)instance_of(la, lb) * GImage<N>::BYTES + GImage<N>::template offset<T>());
+  const double rho0 = d.ph.rho0, E0 = d.ph.E0;
+
+  // loads: the block's state (contiguous), and each thread's point of the -d
+  // neighbours' traces on their +d faces
+  constexpr int UL = (E * EV + NTH - 1) / NTH;
+  UT v[UL], vn[3][NSTATE];
+  const int tot = ne * EV;
+#pragma unroll
+  for (int i = 0; i < UL; ++i) {
+    const int w = t + i * NTH;
+    v[i] = U[k0 * EV + (w < tot ? w : tot - 1)];
+  }
+  {
+    int c[3];
+    element_coords(d, kl + (act ? e : 0), c);
+    const int node[3] = {N - 1 + N * ab, a + N * (N - 1) + NF * b, ab + NF * (N - 1)};
+#pragma unroll
+    for (int D = 0; D < 3; ++D) {
+      const UT *src = U + (k0 + (act ? e : 0) + neighbor_step(d, c, D, -1)) * EV + node[D];
+#pragma unroll
+      for (int s = 0; s < NSTATE; ++s) vn[D][s] = src[s * NN];
     }
   }
+#pragma unroll
+  for (int i = 0; i < UL; ++i) {
+    const int w = t + i * NTH;
+    const int s = sizeof(UT) == 4 ? 0 : (w % EV) / NN;
+    if (w < tot) sb[w] = fluctuation<T>(v[i], s, rho0, E0);
+  }
+  __syncthreads();
+
+  // own trace and normal derivative at the thread's node of the three faces
+  T own[3][NSTATE], nbr[3][NSTATE], qn[3][NSTATE];
+  if (act) {
+    const int base[3] = {N * ab, a + NF * b, ab};
+    constexpr int ST[3] = {1, N, NF};
+#pragma unroll
+    for (int D = 0; D < 3; ++D) {
+      struct Row { T r[N]; };
+      const Row nrm = uniform_load<Row, T>(reinterpret_cast<const Row *>(op->nrm[D]));
+      const T nw = uniform_load<T, T>(&op->nbr[D]);
+#pragma unroll
+      for (int s = 0; s < NSTATE; ++s) {
+        const T *us = sb + e * EV + s * NN + base[D];
+        nbr[D][s] = fluctuation<T>(vn[D][s], s, rho0, E0);
+        own[D][s] = us[0];
+        T q = nw * nbr[D][s];
+#pragma unroll
+        for (int j = 0; j < N; ++j) q += nrm.r[j] * us[j * ST[D]];
+        qn[D][s] = q;
+      }
+    }
+  }
+  __syncthreads();
+  T *const nb = sb, *const wk = sb + L::NB;   // nb: field 5 D + s
+  if (act) {
+#pragma unroll
+    for (int D = 0; D < 3; ++D)
+#pragma unroll
+      for (int s = 0; s < NSTATE; ++s) nb[(NSTATE * D + s) * FS + t] = nbr[D][s];
+  }
+  int c[3];
+  element_coords(d, kl + (act ? e : 0), c);
+  const size_t plane = (size_t)la.nelem * NF;
+  const Bg<T> bg(d.ph);
+  struct Vec { T r[N]; };
+
+  auto direction = [&](auto dir) {
+    constexpr int D = decltype(dir)::value;
+    constexpr int la_ = D == 0 ? 1 : 0, lb_ = D == 2 ? 1 : 2;   // the directions of a and b
+    // items of the sweeps: (variable s, line x = e N + position); the in-face
+    // derivative of variable s along l is one of three (rho, m_D, m_l)
+    constexpr int IT = NSTATE * E * N, PASS = (IT + NTH - 1) / NTH;
+    auto deriv = [&](int s, int l) -> int { return s == 0 ? 0 : s == 1 + D ? 1 : s == 1 + l ? 2 : -1; };
+    if (act) {
+#pragma unroll
+      for (int s = 0; s < NSTATE; ++s) {
+        wk[s * FS + t] = own[D][s];
+        wk[(2 * NSTATE + s) * FS + t] = qn[D][s];
+      }
+    }
+    __syncthreads();
+    {
+      const SymMat<N, T> I = uniform_load<SymMat<N, T>, T>(&op->I);
+      const SymMat<N, T> Dm = uniform_load<SymMat<N, T>, T>(&op->D);
+      const Vec eta = uniform_load<Vec, T>(reinterpret_cast<const Vec *>(op->eta));
+      const T al = uniform_load<T, T>(&op->a[la_]), be = uniform_load<T, T>(&op->a[lb_]);
+      // first sweep (along a)
+#pragma unroll
+      for (int p = 0; p < PASS; ++p) {
+        const int i = t + p * NTH;
+        if (i < IT) {
+          const int s = i / (E * N), x0 = i - s * (E * N);
+          T *f0 = wk + s * FS + N * x0;
+          T x[N], o[N];
+#pragma unroll
+          for (int j = 0; j < N; ++j) x[j] = f0[j];
+          sym_apply<N, 1, T>(I, x, o);
+#pragma unroll
+          for (int j = 0; j < N; ++j) f0[j] = o[j];
+          const int f = deriv(s, la_);
+          if (f >= 0) {
+            // the -l neighbour's trace at the edge: l = y on the -x face: -y
+            // trace at (x, z) = (0, b); l = x on the -y face: -x trace at
+            // (y, z) = (0, b); l = x on the -z face: at (b, 0)
+            const int at = D < 2 ? N * x0 : x0 / N * NF + x0 % N;
+            const T jmp = x[0] - nb[(NSTATE * la_ + s) * FS + at];
+            sym_apply<N, -1, T>(Dm, x, o);
+            T *fd = wk + (15 + f) * FS + N * x0;
+#pragma unroll
+            for (int j = 0; j < N; ++j) fd[j] = al * (o[j] + eta.r[j] * jmp);
+          }
+          const T *g = nb + (NSTATE * D + s) * FS + N * x0;
+#pragma unroll
+          for (int j = 0; j < N; ++j) x[j] = g[j];
+          sym_apply<N, 1, T>(I, x, o);
+#pragma unroll
+          for (int j = 0; j < N; ++j) (f0 + NSTATE * FS)[j] = o[j];
+          T *fg = f0 + 2 * NSTATE * FS;
+#pragma unroll
+          for (int j = 0; j < N; ++j) x[j] = fg[j];
+          sym_apply<N, 1, T>(I, x, o);
+#pragma unroll
+          for (int j = 0; j < N; ++j) fg[j] = o[j];
+        }
+      }
+      // the second sweep's edge lines: the -l neighbour's trace along a
+      for (int i = t; i < 3 * E; i += NTH) {
+        const int f = i / E, ee = i - f * E, s = f == 0 ? 0 : f == 1 ? 1 + D : 1 + lb_;
+        const T *p = nb + (NSTATE * lb_ + s) * FS + ee * NF;
+        T x[N], o[N];
+#pragma unroll
+        for (int j = 0; j < N; ++j) x[j] = p[D == 0 ? N * j : j];
+        sym_apply<N, 1, T>(I, x, o);
+#pragma unroll
+        for (int q = 0; q < N; ++q) sedge[i * N + q] = o[q];
+      }
+      __syncthreads();
+      // second sweep (along b, in place)
+#pragma unroll
+      for (int p = 0; p < PASS; ++p) {
+        const int i = t + p * NTH;
+        if (i < IT) {
+          const int s = i / (E * N), x0 = i - s * (E * N), at = x0 / N * NF + x0 % N;
+          T *f0 = wk + s * FS + at;
+          T x[N], o[N];
+          auto interp = [&](T *f) {
+#pragma unroll
+            for (int j = 0; j < N; ++j) x[j] = f[N * j];
+            sym_apply<N, 1, T>(I, x, o);
+#pragma unroll
+            for (int j = 0; j < N; ++j) f[N * j] = o[j];
+          };
+          interp(f0 + NSTATE * FS);
+          interp(f0 + 2 * NSTATE * FS);
+          const int fa = deriv(s, la_), fb = deriv(s, lb_);
+          if (fa >= 0) interp(wk + (15 + fa) * FS + at);
+          interp(f0);   // x: the own trace before it
+          if (fb >= 0) {
+            const T jmp = x[0] - sedge[fb * (E * N) + x0];
+            sym_apply<N, -1, T>(Dm, x, o);
+            T *fd = wk + (18 + fb) * FS + at;
+#pragma unroll
+            for (int j = 0; j < N; ++j) fd[N * j] = be * (o[j] + eta.r[j] * jmp);
+          }
+        }
+      }
+    }
+    __syncthreads();
+    // fluxes of both sides at the thread's point; side 1 goes to the -d
+    // neighbour's record
+    if (act) {
+      T oK[5], oN[5];
+      face_point_flux<T, D, FS>(wk + t, bg, oK, oN);
+      T *const f0 = FF + (size_t)k0 * NF;
+      const int st = t + neighbor_step(d, c, D, -1) * NF;
+      const T ad = uniform_load<T, T>(&op->a[D]);
+#pragma unroll
+      for (int s = 0; s < NSTATE; ++s) {
+        (f0 + (2 * D * NSTATE + s) * plane)[t] = oN[s] * ad;
+        (f0 + ((2 * D + 1) * NSTATE + s) * plane)[st] = oK[s] * ad;
+      }
+    }
+  };
+  direction(std::integral_constant<int, 0>());
+  __syncthreads();
+  direction(std::integral_constant<int, 1>());
+  __syncthreads();
+  direction(std::integral_constant<int, 2>());
 }
 
-// WQ: also compute the gradient at every node and write it to Q (for the
-// closure's features and ldg_rhs's gradient output); the time-stepping path
-// needs only the face nodes' components, the right-hand-side kernel
-// computes the volume gradient at the Gauss points itself.
-template <int N, int E, typename TQ, typename UT, bool WQ>
-__global__ void __launch_bounds__(NT, (GradWaves<N, E, TQ>::value))
-ldg_grad_kernel(const UT *__restrict__ U, TQ *__restrict__ Q, TQ *__restrict__ FF, LaunchArgs la,
-                const Ops<N, double> *__restrict__ opp) {
+// ---------------------------------------------------------------------
+// Nodal LDG gradient Q_l = a_l (Dn u + L0 J_l) (solver.cpp:490-508, restated
+// in strong form: -M1^{-1} S1 + face lifts = Dn + M1^{-1} e_0 e_0^T, exactly),
+// for ldg_rhs's gradient output and the closure's features.  One thread per
+// node computes all 15 components and stores them straight to HBM
+// (consecutive threads -> consecutive nodes, coalesced).
+// ---------------------------------------------------------------------
+template <int N, int E, typename TQ, typename UT>
+__global__ void __launch_bounds__(NT) ldg_nodal_grad_kernel(const UT *__restrict__ U, TQ *__restrict__ Q, LaunchArgs la,
+                                                            const Ops<N, double> *__restrict__ opp) {
   constexpr int NN = N * N * N, NF = N * N;
-  // face fields of each element's -d face: own U (0-4), the -d neighbour's U
-  // (5-9), the gradient components of direction d (10-20)
-  constexpr int NFF = 2 * NSTATE + NFG;
-  // arithmetic type: FP32 with an FP32 gradient (mixed), FP64 otherwise
   using C = TQ;
   __shared__ C su[E][NSTATE][NN];
-  __shared__ C sf[E][3][NFF][NF];   // -d face of each element: nodal traces, then Gauss-point values
+  __shared__ C sf[E][3][NSTATE][NF];   // the -d neighbours' traces on their +d faces
   __shared__ C sD[N][N + 1];
-  __shared__ C sw[N];
-  __shared__ SymMat<N, C> sI, sIt;
   __shared__ long snb[E][6];
   const int lb = logical_block(la);
   if (lb < 0) return;
@@ -518,94 +943,33 @@ ldg_grad_kernel(const UT *__restrict__ U, TQ *__restrict__ Q, TQ *__restrict__ F
   int ne, ec[3];
   const InstDesc &d = block_instance<E>(la, lb, m, ec, kl, ne);
   if (ne == 0) return;                // padding block of a partial brick
-  const long k0 = d.elem_off + kl;    // first element of the block in the arrays
+  const long k0 = d.elem_off + kl;
   const unsigned tid = threadIdx.x;
   fill_neighbors(m, ec, d.elem_off, ne, snb, tid);
-
-  // Q_l(i) = (Dn u)(i) + L0(i) (u_0 - u_nbr): the own trace u_0 is the line's
-  // first node, so its lift joins column 0 of Dn and only the neighbour's
-  // trace enters separately, with weight -L0(i) in column N
+  // the own trace u_0 is the line's first node, so its lift joins column 0
+  // of Dn and only the neighbour's trace enters separately, with weight
+  // -L0(i) in column N
   if (tid < N * (N + 1)) {
     const int i = tid / (N + 1), j = tid % (N + 1);
     sD[i][j] = C(j < N ? opp->Dn[i][j] + (j == 0 ? opp->L0[i] : 0.0) : -opp->L0[i]);
   }
-  {
-    constexpr int MS = sizeof(SymMat<N, C>) / sizeof(C);   // coefficients of I, one per thread
-    if (tid >= 64 && tid < 64 + MS)
-      reinterpret_cast<C *>(&sI)[tid - 64] = C(reinterpret_cast<const double *>(&opp->sI)[tid - 64]);
-    if (tid >= 192 && tid < 192 + MS)
-      reinterpret_cast<C *>(&sIt)[tid - 192] = C(reinterpret_cast<const double *>(&opp->sIt)[tid - 192]);
+  __syncthreads();
+  const double rho0 = d.ph.rho0, E0 = d.ph.E0;
+  for (unsigned w = tid; w < (unsigned)ne * NN; w += NT) {
+    const unsigned e = w / NN, node = w - e * NN;
+#pragma unroll
+    for (int s = 0; s < NSTATE; ++s)
+      su[e][s][node] = fluctuation<C>(U[(k0 + e) * (NSTATE * NN) + s * NN + node], s, rho0, E0);
   }
-  if (tid >= 128 && tid < 128 + N) sw[tid - 128] = C(opp->w[tid - 128]);
-  __syncthreads();   // neighbour table
-
-  // the block's state (one node per thread, its five variables) and the -d
-  // neighbours' traces on their positive faces (one face point per thread)
-  // into LDS as fluctuations about the background, all of a thread's loads
-  // issued before the first is stored.  The loads are unconditional (an
-  // index past the block is clamped to its last item) and converted only
-  // when stored: a load under a branch is waited for at the branch's end.
-  // An FP64 input in the mixed path (RK stage 1) is rounded to the FP32
-  // fluctuation the other stages read, so a step's result does not depend
-  // on which form its input came in; the FP64 path differentiates the
-  // fluctuation too (the same gradient: Dn annihilates constants).
-  {
-    constexpr int UL = (E * NN + NT - 1) / NT;
-    constexpr int JL = (E * 3 * NF + NT - 1) / NT;
-    const unsigned tot = ne * NN, totj = ne * 3 * NF;
-    UT v[UL][NSTATE], vj[JL][NSTATE];
-    unsigned so[UL], sj[JL];
+  for (unsigned w = tid; w < (unsigned)ne * 3 * NF; w += NT) {
+    const unsigned ed = w / NF, ab = w - ed * NF, e = ed / 3, dd = ed - 3 * e, b = ab / N, a = ab - b * N;
+    const unsigned node = (dd == 0 ? N : 1) * a + (dd == 2 ? N : NF) * b + (dd == 0 ? 1 : dd == 1 ? N : NF) * (N - 1);
 #pragma unroll
-    for (int it = 0; it < UL; ++it) {
-      const unsigned w = tid + it * NT < tot ? tid + it * NT : tot - 1;
-      const unsigned e = w / NN;
-      so[it] = w + e * ((NSTATE - 1) * NN);   // su[e][0][node]
-      const UT *src = U + k0 * (NSTATE * NN) + (e * (NSTATE * NN) + (w - e * NN));
-#pragma unroll
-      for (int s = 0; s < NSTATE; ++s) v[it][s] = src[s * NN];
-    }
-#pragma unroll
-    for (int it = 0; it < JL; ++it) {
-      const unsigned w = tid + it * NT < totj ? tid + it * NT : totj - 1;
-      const unsigned ed = w / NF, ab = w - ed * NF;   // ed = e * 3 + d
-      const unsigned e = ed / 3, dd = ed - 3 * e;
-      const unsigned b = ab / N, a = ab - b * N;
-      sj[it] = ed * (NFF * NF) + NSTATE * NF + ab;    // sf[e][dd][NSTATE][ab]
-      // node (N-1, a, b), (a, N-1, b) or (a, b, N-1) of the -d neighbour: its +d face
-      const unsigned node = (dd == 0 ? N : 1) * a + (dd == 2 ? N : NF) * b + (dd == 0 ? 1 : dd == 1 ? N : NF) * (N - 1);
-      const UT *src = U + snb[e][2 * dd] * (NSTATE * NN) + node;
-#pragma unroll
-      for (int s = 0; s < NSTATE; ++s) vj[it][s] = src[s * NN];
-    }
-    const double brho = d.ph.rho0, bE = d.ph.E0;
-    auto fluct = [&](UT x, int s) -> C {
-      if (sizeof(UT) == 4) return C(x);   // already the FP32 fluctuation
-      const double f = (double)x - (s == 0 ? brho : s == 4 ? bE : 0.0);
-      return C(f);
-    };
-    C *const suf = &su[0][0][0];
-    C *const sff = &sf[0][0][0][0];
-#pragma unroll
-    for (int it = 0; it < UL; ++it) {
-      if (tid + it * NT < tot) {
-#pragma unroll
-        for (int s = 0; s < NSTATE; ++s) suf[so[it] + s * NN] = fluct(v[it][s], s);
-      }
-    }
-#pragma unroll
-    for (int it = 0; it < JL; ++it) {
-      if (tid + it * NT < totj) {
-#pragma unroll
-        for (int s = 0; s < NSTATE; ++s) sff[sj[it] + s * NF] = fluct(vj[it][s], s);
-      }
-    }
+    for (int s = 0; s < NSTATE; ++s)
+      sf[e][dd][s][ab] = fluctuation<C>(U[snb[e][2 * dd] * (NSTATE * NN) + s * NN + node], s, rho0, E0);
   }
   __syncthreads();
-
-  // gradient, one node per thread; the node's own trace on the element's -d
-  // faces and the face components of its gradient go to the face slots (a
-  // node on an edge or corner belongs to several faces)
-  auto node_grad = [&](unsigned w) {
+  for (unsigned w = tid; w < (unsigned)ne * NN; w += NT) {
     const unsigned e = w / NN, node = w - e * NN;
     const unsigned iz = node / NF, rem = node - iz * NF;
     const unsigned iy = rem / N, ix = rem - iy * N;
@@ -613,889 +977,520 @@ ldg_grad_kernel(const UT *__restrict__ U, TQ *__restrict__ Q, TQ *__restrict__ F
 #pragma unroll
     for (int j = 0; j <= N; ++j) { rx[j] = sD[ix][j]; ry[j] = sD[iy][j]; rz[j] = sD[iz][j]; }
     TQ *Qe = Q + (k0 + e) * NGRAD * NN + node;
-    C g[NGRAD], ox[NSTATE], oy[NSTATE], oz[NSTATE];
 #pragma unroll
     for (int s = 0; s < NSTATE; ++s) {
       const C *us = su[e][s];
-      C qx = rx[N] * sf[e][0][NSTATE + s][iy + N * iz];
-      C qy = ry[N] * sf[e][1][NSTATE + s][ix + N * iz];
-      C qz = rz[N] * sf[e][2][NSTATE + s][ix + N * iy];
+      C qx = rx[N] * sf[e][0][s][iy + N * iz];
+      C qy = ry[N] * sf[e][1][s][ix + N * iz];
+      C qz = rz[N] * sf[e][2][s][ix + N * iy];
 #pragma unroll
       for (int j = 0; j < N; ++j) {
-        const C ux = us[j + N * iy + NF * iz], uy = us[ix + N * j + NF * iz], uz = us[ix + N * iy + NF * j];
-        if (j == 0) { ox[s] = ux; oy[s] = uy; oz[s] = uz; }   // the line's first node: the -d face trace
-        qx += rx[j] * ux;
-        qy += ry[j] * uy;
-        qz += rz[j] * uz;
+        qx += rx[j] * us[j + N * iy + NF * iz];
+        qy += ry[j] * us[ix + N * j + NF * iz];
+        qz += rz[j] * us[ix + N * iy + NF * j];
       }
-      g[0 * NSTATE + s] = qx * C(m.ialpha[0]);
-      g[1 * NSTATE + s] = qy * C(m.ialpha[1]);
-      g[2 * NSTATE + s] = qz * C(m.ialpha[2]);
-      Qe[(0 * NSTATE + s) * NN] = g[0 * NSTATE + s];
-      Qe[(1 * NSTATE + s) * NN] = g[1 * NSTATE + s];
-      Qe[(2 * NSTATE + s) * NN] = g[2 * NSTATE + s];
-    }
-    if (ix == 0) {
-      C *fs = &sf[e][0][0][iy + N * iz];
-#pragma unroll
-      for (int s = 0; s < NSTATE; ++s) fs[s * NF] = ox[s];
-#pragma unroll
-      for (int j = 0; j < NFG; ++j) fs[(2 * NSTATE + j) * NF] = g[face_grad(0, j)];
-    }
-    if (iy == 0) {
-      C *fs = &sf[e][1][0][ix + N * iz];
-#pragma unroll
-      for (int s = 0; s < NSTATE; ++s) fs[s * NF] = oy[s];
-#pragma unroll
-      for (int j = 0; j < NFG; ++j) fs[(2 * NSTATE + j) * NF] = g[face_grad(1, j)];
-    }
-    if (iz == 0) {
-      C *fs = &sf[e][2][0][ix + N * iy];
-#pragma unroll
-      for (int s = 0; s < NSTATE; ++s) fs[s * NF] = oz[s];
-#pragma unroll
-      for (int j = 0; j < NFG; ++j) fs[(2 * NSTATE + j) * NF] = g[face_grad(2, j)];
-    }
-  };
-  if constexpr (WQ) {
-    if constexpr (E * NN <= NT) {
-      if (tid < (unsigned)ne * NN) node_grad(tid);   // one pass (every order's default tiling)
-    } else {
-      for (unsigned w = tid; w < (unsigned)ne * NN; w += NT) node_grad(w);
-    }
-  } else {
-    // the face nodes only; the points of one direction padded to whole
-    // waves, as in the flux phase below
-    constexpr unsigned PD = (E * NF + 63) / 64 * 64;
-    constexpr unsigned FSTEP = 3 * PD <= NT ? 0x40000000u : NT;
-    for (unsigned w = tid; w < 3 * PD; w += FSTEP) {
-      const unsigned dd = w / PD, r = w - dd * PD;
-      if (r >= (unsigned)ne * NF) continue;
-      const unsigned e = r / NF, ab = r - e * NF;
-      if (dd == 0) face_node_grad<N, 0, NFF, C>(su[e][0], sf[e][0][0], sD, m.ialpha, ab);
-      else if (dd == 1) face_node_grad<N, 1, NFF, C>(su[e][0], sf[e][0][0], sD, m.ialpha, ab);
-      else face_node_grad<N, 2, NFF, C>(su[e][0], sf[e][0][0], sD, m.ialpha, ab);
-    }
-  }
-  __syncthreads();
-
-  // interpolate the 21 face fields to the face Gauss points: along a, then
-  // along b, in place; face coordinates (a, b) = (y, z), (x, z), (x, y) for
-  // d = 0, 1, 2.  A line is (element, direction, field, position): w = fl N
-  // + x with fl = (e 3 + d) NFF + f, whose face slot starts at fl NF in sf;
-  // the two sweeps share the decomposition, done once per thread.
-  {
-    constexpr unsigned SW = 3 * NFF * N;              // lines per element
-    constexpr int SL = (E * SW + NT - 1) / NT;        // lines per thread
-    C *const sff = &sf[0][0][0][0];
-    unsigned pa[SL], pb[SL];                          // line starts of the two sweeps, ~0 past the block
-#pragma unroll
-    for (int it = 0; it < SL; ++it) {
-      const unsigned w = tid + it * NT, fl = w / N, x = w - fl * N;
-      const bool in = w < (unsigned)ne * SW;
-      pa[it] = in ? fl * NF + N * x : ~0u;
-      pb[it] = fl * NF + x;
-    }
-    SymReg<N, C> I;
-    I.load(sI);
-#pragma unroll
-    for (int it = 0; it < SL; ++it) {
-      if (pa[it] == ~0u) continue;
-      C v[N], o[N];
-#pragma unroll
-      for (int a = 0; a < N; ++a) v[a] = sff[pa[it] + a];
-      sym_apply<N, 1, C>(I.m, v, o);
-#pragma unroll
-      for (int q = 0; q < N; ++q) sff[pa[it] + q] = o[q];
-    }
-    __syncthreads();
-#pragma unroll
-    for (int it = 0; it < SL; ++it) {
-      if (pa[it] == ~0u) continue;
-      C v[N], o[N];
-#pragma unroll
-      for (int b = 0; b < N; ++b) v[b] = sff[pb[it] + N * b];
-      sym_apply<N, 1, C>(I.m, v, o);
-#pragma unroll
-      for (int q = 0; q < N; ++q) sff[pb[it] + N * q] = o[q];
-    }
-  }
-  __syncthreads();
-
-  // fluxes of both sides at every face Gauss point, weighted for the lift,
-  // into the point's slots 0-9 (read only by the thread of that point).
-  // The points of one direction are padded to whole waves, so that every
-  // wave evaluates one direction's flux (the direction is a template
-  // parameter: a wave holding points of several directions would run each
-  // variant with part of its lanes)
-  {
-    const Bg<C> bg(d.ph);
-    constexpr unsigned PD = (E * NF + 63) / 64 * 64;
-    constexpr unsigned FSTEP = 3 * PD <= NT ? 0x40000000u : NT;   // one pass when the points fit
-    for (unsigned w = tid; w < 3 * PD; w += FSTEP) {
-      const unsigned dd = w / PD, r = w - dd * PD;
-      if (r >= (unsigned)ne * NF) continue;
-      const unsigned e = r / NF, ab = r - e * NF;
-      C *fp = &sf[e][dd][0][ab];
-      C outK[5], outN[5];
-      if (dd == 0) face_point_flux<C, 0, NF>(fp, bg, outK, outN);
-      else if (dd == 1) face_point_flux<C, 1, NF>(fp, bg, outK, outN);
-      else face_point_flux<C, 2, NF>(fp, bg, outK, outN);
-      // (a select, not an index: a run-time index into m would put it in scratch)
-      const double ia = dd == 0 ? m.ialpha[0] : dd == 1 ? m.ialpha[1] : m.ialpha[2];
-      const C wt = sw[ab % N] * sw[ab / N] * C(ia);
-#pragma unroll
-      for (int s = 0; s < NSTATE; ++s) {
-        fp[s * NF] = outN[s] * wt;                   // side 0: this element, its -d face
-        fp[(NSTATE + s) * NF] = outK[s] * wt;        // side 1: the -d neighbour, its +d face
-      }
-    }
-  }
-  __syncthreads();
-
-  // lift to the face nodes, I^T along a then along b, and write FF: per
-  // element and direction the 10 flux fields (side, state) are lines
-  // (field f, x) of N values; the b sweep stores straight to HBM
-  // (FF[element][2 d + side][state][node]), so the right-hand-side kernel
-  // only adds them
-  {
-    constexpr unsigned LL = 2 * NSTATE * N;           // lines per (element, direction)
-    constexpr int LI = (E * 3 * LL + NT - 1) / NT;
-    constexpr int CH = ff_chunk(N, (int)sizeof(TQ));
-    C *const sff = &sf[0][0][0][0];
-    unsigned lb_[LI], lf[LI], lx[LI];                 // (e 3 + d), field, x; lb_ = ~0 past the block
-#pragma unroll
-    for (int it = 0; it < LI; ++it) {
-      const unsigned w = tid + it * NT, ed = w / LL, r = w - ed * LL, f = r / N;
-      lb_[it] = w < (unsigned)ne * 3 * LL ? ed : ~0u;
-      lf[it] = f;
-      lx[it] = r - f * N;
-    }
-    SymReg<N, C> It;
-    It.load(sIt);
-#pragma unroll
-    for (int it = 0; it < LI; ++it) {
-      if (lb_[it] == ~0u) continue;
-      C *p = sff + (lb_[it] * NFF + lf[it]) * NF + N * lx[it];
-      C v[N], o[N];
-#pragma unroll
-      for (int a = 0; a < N; ++a) v[a] = p[a];
-      sym_apply<N, 1, C>(It.m, v, o);
-#pragma unroll
-      for (int a = 0; a < N; ++a) p[a] = o[a];
-    }
-    __syncthreads();
-    TQ *const ffb = FF + k0 * ff_per_element<N, TQ>();
-#pragma unroll
-    for (int it = 0; it < LI; ++it) {
-      if (lb_[it] == ~0u) continue;
-      const unsigned ed = lb_[it], f = lf[it], x = lx[it];
-      const C *p = sff + (ed * NFF + f) * NF + x;
-      C v[N], o[N];
-#pragma unroll
-      for (int b = 0; b < N; ++b) v[b] = p[N * b];
-      sym_apply<N, 1, C>(It.m, v, o);
-      // element ed / 3, chunk 2 d + side, state f mod 5, node x + N b
-      const unsigned e = ed / 3, dd = ed - 3 * e, side = f / NSTATE;
-      TQ *dst = ffb + (e * ff_per_element<N, TQ>() + (2 * dd + side) * CH + (f - NSTATE * side) * NF + x);
-#pragma unroll
-      for (int b = 0; b < N; ++b) dst[N * b] = o[b];
+      Qe[(0 * NSTATE + s) * NN] = qx * C(m.ialpha[0]);
+      Qe[(1 * NSTATE + s) * NN] = qy * C(m.ialpha[1]);
+      Qe[(2 * NSTATE + s) * NN] = qz * C(m.ialpha[2]);
     }
   }
 }
 
 // ---------------------------------------------------------------------
 // Kernel B: volume gradient and integrals, the face terms, inverse mass,
-// RK epilogue.
+// RK epilogue, in Gauss form (GOps above).
 //
-// LDS per element: a 20-field volume buffer of type T (in FP32 with room
-// for the two jump face sets after it), which last holds the FP64
-// inverse-mass sweeps (5 FP64 fields fit in the space of 10 FP32 fields).
-// The face terms come from HBM into registers (the gradient kernel lifted
-// them to the face nodes).
+// A thread owns one line (element e, face position ab) for all five
+// variables; x-lines (y, z) = (a, b), y-lines (x, z) = (a, b), z-lines
+// (x, y) = (a, b).  LDS holds two sets of five fields per element (A, B), at
+// the end the FP64 rates.  Phases, with the values a thread keeps in
+// registers between them in brackets:
+//   x    nodes from HBM, I -> A; the jumps J_l at the face nodes
+//   y    I on A; J along a
+//   z    I on A [u_g on the thread's z-line]; J along b
+//   d    Qx = a (Dg u + eta J) on A's x-lines, Qy on its y-lines -> A, B
+//   p    Qz on the z-line; fluxes at its points: Fx, Fy -> A, B; [Dh Fz - faces]
+//   t    Dh Fx - faces on A's x-lines, Dh Fy - faces on B's y-lines
+//   zi   sum of the three, I^-1 along z in FP64 -> the FP64 buffer
+//   yi   I^-1 along y;   xi   along x
+//   epilogue: rate, running sum, next stage input (flat, coalesced)
+//
+// Measured at 64^3, p = 4, average of the four stages: mixed 1.18 ms (1.42
+// with sweeps at the nodes and one line of one variable per thread), 4.8 TB/s
+// of HBM traffic where a streaming kernel with the same mix of reads and
+// writes reaches 5.4; FP64 1.57 ms (2.26), 4.8 TB/s, LDS busy for 57 %.
 // ---------------------------------------------------------------------
-template <int N, typename T>
+template <int N, int E, typename T>
 struct RhsLds {
-  static constexpr int NN = N * N * N, NF = N * N;
-  static constexpr int NV = NSTATE + NGRAD;          // 20 volume fields
-  static constexpr int SV = NV * NN;
-  static constexpr int CH = ff_chunk(N, (int)sizeof(T));
-  static constexpr int FE = 6 * CH;                  // face fluxes of one element (3 directions, 2 sides)
-  static constexpr int SJ = NSTATE * NF;             // one face field set: the y or z jumps
-  static constexpr int VW = 16 / (int)sizeof(T);     // values per 16-byte word
-  // the y and z jump sets: in FP64 inside the Q_z slot (which the volume
-  // stage fills last; less LDS, so more workgroups fit a CU), in FP32 after
-  // the volume fields (LDS does not limit the FP32 kernel's occupancy, and
-  // the Q_z slot would cost a barrier)
-  static constexpr bool JQZ = sizeof(T) == sizeof(double);
-  static_assert(2 * SJ <= NSTATE * NN, "the jump sets fit the Q_z slot");
-  static constexpr int SJ0 = JQZ ? 3 * NSTATE * NN : SV;   // start of the jump sets
-  static constexpr int BUF = ((JQZ ? SV : SV + 2 * SJ) + VW - 1) / VW * VW;   // per element (16-byte multiple)
-  // occupancy target (waves per SIMD) handed to the register allocator
-  static constexpr int WAVES = sizeof(T) == 4 ? (N <= 5 ? 4 : 2) : (N <= 2 ? 4 : N <= 5 ? 3 : 2);
+  using S = Shape<N, E>;
+  // the jumps' face fields: in FP64 in set B, which is free until phase d
+  // stores Qy (the smaller footprint lets more workgroups share a CU)
+  static constexpr bool JB = N >= 3;
+  // element stride in a set: padded so that the lines of a wave's elements
+  // fall on different LDS banks (p = 4: the x, y and z lines of 32 lanes in
+  // 12 instead of 20 cycles per wave and value)
+  static constexpr int PAD = N == 2 ? 0 : N == 3 ? 6 : N == 4 ? 20 : N == 5 ? 8 : 5;
+  static constexpr int ES = S::EV + PAD;
+  static constexpr int SET = E * ES, JS = 3 * NSTATE * E * S::NF;
+  static constexpr int BUF = JB ? 2 * SET : 2 * SET + JS;
+  static constexpr int WAVES = sizeof(T) == 4 && N <= 5 ? 3 : 2;
 };
 
-// Operators in LDS: the compute-type copies used by the sweeps and the FP64
-// inverse mass.  Each phase loads the matrix it needs into a register array
-// before its loop (LDS loads produce VGPRs: the coefficients neither occupy
-// SGPRs nor spill).
-template <int N, typename T>
-struct SOps {
-  SymMat<N, T> I, It, Dt;   // interpolation, its transpose, D^T (compute type)
-  SymMat<N, T> Ds[3];       // D = I Dn times 1/alpha_l, l = x, y, z
-  T il0[3][N];              // I L0 times 1/alpha_l
-  SymMat<N, double> Mi;     // inverse mass (FP64)
-  T w[N];                   // Gauss weights (compute type and FP64)
-  double wd[N];
-};
-
-// The rhs kernel's operators for one instance, built on the host from the
-// FP64 operators and the instance's a_l = 1/alpha_l = 2/dx_l: I, I^T, D^T
-// and D a_l (l = x, y, z) in type T, each coefficient rounded once; the
-// FP64 inverse mass; (I L0) a_l; the Gauss weights.  The kernel copies the
-// image of its instance into LDS (no conversion or scaling on the device).
-template <int N, typename T>
-void fill_sops(SOps<N, T> &so, const Ops<N, double> &op, const double a[3]) {
-  constexpr int MS = sizeof(SymMat<N, T>) / sizeof(T);   // coefficients per operator
-  static_assert(sizeof(SymMat<N, T>) == MS * sizeof(T) && sizeof(SymMat<N, double>) == MS * sizeof(double),
-                "operators are plain coefficient arrays");
-  using SO = SOps<N, T>;
-  static_assert(offsetof(SO, Ds) == 3 * sizeof(SymMat<N, T>), "I, I^T, D^T, D_x, D_y, D_z are contiguous");
-  const SymMat<N, double> *src[6] = {&op.sI, &op.sIt, &op.sDt, &op.sD, &op.sD, &op.sD};
-  const double f[6] = {1.0, 1.0, 1.0, a[0], a[1], a[2]};
-  T *dst = reinterpret_cast<T *>(&so.I);
-  for (int o = 0; o < 6; ++o)
-    for (int i = 0; i < MS; ++i) dst[o * MS + i] = T(reinterpret_cast<const double *>(src[o])[i] * f[o]);
-  so.Mi = op.sMi;
-  for (int l = 0; l < 3; ++l)
-    for (int q = 0; q < N; ++q) so.il0[l][q] = T(op.IL0[q] * a[l]);
-  for (int q = 0; q < N; ++q) {
-    so.w[q] = T(op.w[q]);
-    so.wd[q] = op.w[q];
-  }
-}
-
-// Per instance, the FP32 image then the FP64 image, each padded to 16 bytes.
-template <int N>
-struct SOpsImage {
-  static constexpr int F = (int)((sizeof(SOps<N, float>) + 15) / 16 * 16);
-  static constexpr int D = (int)((sizeof(SOps<N, double>) + 15) / 16 * 16);
-  static constexpr int BYTES = F + D;
-  template <typename T>
-  static constexpr int offset() { return sizeof(T) == sizeof(double) ? F : 0; }
-};
-
-template <int N, typename T>
-struct Mat {
-  T v[N][N];
-  __device__ inline void load(const T (&src)[N][N]) {
-#pragma unroll
-    for (int a = 0; a < N; ++a)
-#pragma unroll
-      for (int b = 0; b < N; ++b) v[a][b] = src[a][b];
-  }
-};
-
-template <int N, int E, typename T, typename UT>
-__global__ void __launch_bounds__(NT, (RhsLds<N, T>::WAVES))
-ldg_rhs_kernel(const UT *__restrict__ U, const T *__restrict__ FF, LaunchArgs la, const unsigned char *__restrict__ simg,
-               StageArgs st) {
-  using L = RhsLds<N, T>;
-  constexpr int NN = L::NN, NF = L::NF, BUF = L::BUF;
-  __shared__ __align__(16) T sbuf[E][BUF];
-  __shared__ double sred[NT / 64];
-  __shared__ double sbg[NSTATE];      // the background state (rho0, 0, 0, 0, E0)
-  __shared__ SOps<N, T> sops;
-  __shared__ long snb[E][6];
+// DIAG: instead of the rate, the diagnostics of the state U: st.ke_part and
+// st.diag_part (the nodal and the Gauss-point sums), from the state and its
+// gradient at the Gauss points; no face fluxes are read.
+template <int N, int E, typename T, typename UT, bool DIAG>
+__global__ void __launch_bounds__((Shape<N, E>::NTH), (RhsLds<N, E, T>::WAVES))
+ldg_rhs_kernel(const UT *__restrict__ U, const T *__restrict__ FF, LaunchArgs la,
+               const unsigned char *__restrict__ img, StageArgs st) {
+  using S = Shape<N, E>;
+  using L = RhsLds<N, E, T>;
+  constexpr int NN = S::NN, NF = S::NF, EV = S::EV, ES = L::ES, NTH = S::NTH;
+  __shared__ __align__(16) T sbuf[L::BUF];
+  __shared__ double sred[NTH / 64];
   const int lb = logical_block(la);
   if (lb < 0) return;
-  MeshArgs m;
-  long kl;
-  int ne, ec[3];
-  const InstDesc &d = block_instance<E>(la, lb, m, ec, kl, ne);
-  if (ne == 0) {                      // padding block of a partial brick: empty partial sums
-    if (threadIdx.x == 0) {
-      if (st.ke_part) st.ke_part[lb] = 0.0;
-      if (st.diag_part) { st.diag_part[2 * lb] = 0.0; st.diag_part[2 * lb + 1] = 0.0; }
+  const int t = threadIdx.x;
+  int kl, ne;
+  const InstDesc &d = block_span(la, lb, E, kl, ne);
+  if (ne <= 0) {                      // padding block: empty partial sums
+    if (t == 0 && st.ke_part) st.ke_part[lb] = 0.0;
+    if (DIAG && t == 0) st.diag_part[2 * lb] = st.diag_part[2 * lb + 1] = 0.0;
+    return;
+  }
+  const long k0 = d.elem_off + kl;
+  const int e = t / NF, ab = t - e * NF, b = ab / N, a = ab - b * N;
+  const bool act = e < ne;
+  const unsigned char *const im = img + (long)instance_of(la, lb) * GImage<N>::BYTES;
+  const GOps<N, T> *const op = reinterpret_cast<const GOps<N, T> *>(im + GImage<N>::template offset<T>());
+  const GOpsD<N> *const opd = reinterpret_cast<const GOpsD<N> *>(im);
+  struct Vec { T r[N]; };
+  T *const sA = sbuf, *const sB = sbuf + L::SET, *const sJ = L::JB ? sB : sbuf + 2 * L::SET;
+  double *const md = reinterpret_cast<double *>(sbuf);
+  const int lx = N * ab, ly = a + NF * b, lz = ab;                                // the thread's lines
+  const int bx = e * ES + lx, by = e * ES + ly, bz = e * ES + lz;                // in a set
+  int c[3];
+  element_coords(d, kl + (act ? e : 0), c);
+
+  // ---- x
+  double dkn = 0.0, dke = 0.0, dens = 0.0;   // (DIAG)
+  if (act) {
+    const double rho0 = d.ph.rho0, E0 = d.ph.E0;
+    const UT *const ue = U + (k0 + e) * EV;
+    UT v[NSTATE][N], vy[NSTATE], vz[NSTATE], nx[NSTATE], ny[NSTATE], nz[NSTATE];
+    const UT *const ux = U + (k0 + e + neighbor_step(d, c, 0, -1)) * EV + (N - 1 + N * ab);
+    const UT *const uy = U + (k0 + e + neighbor_step(d, c, 1, -1)) * EV + (a + N * (N - 1) + NF * b);
+    const UT *const uz = U + (k0 + e + neighbor_step(d, c, 2, -1)) * EV + (ab + NF * (N - 1));
+#pragma unroll
+    for (int s = 0; s < NSTATE; ++s) {
+#pragma unroll
+      for (int q = 0; q < N; ++q) v[s][q] = (ue + lx)[s * NN + q];
+      vy[s] = (ue + ly)[s * NN];
+      vz[s] = (ue + lz)[s * NN];
+      nx[s] = ux[s * NN];
+      ny[s] = uy[s * NN];
+      nz[s] = uz[s * NN];
+    }
+    if constexpr (DIAG) {
+#pragma unroll
+      for (int q = 0; q < N; ++q)
+        dkn += opd->w[a] * opd->w[b] * opd->w[q] *
+               (v[1][q] * v[1][q] + v[2][q] * v[2][q] + v[3][q] * v[3][q]) / (2.0 * v[0][q]);
+    }
+    const SymMat<N, T> I = uniform_load<SymMat<N, T>, T>(&op->I);
+#pragma unroll
+    for (int s = 0; s < NSTATE; ++s) {
+      auto fl = [&](UT x) -> T { return fluctuation<T>(x, s, rho0, E0); };
+      T x[N], o[N];
+#pragma unroll
+      for (int q = 0; q < N; ++q) x[q] = fl(v[s][q]);
+      sym_apply<N, 1, T>(I, x, o);
+#pragma unroll
+      for (int q = 0; q < N; ++q) sA[bx + s * NN + q] = o[q];
+      sJ[(0 * NSTATE + s) * (E * NF) + t] = x[0] - fl(nx[s]);
+      sJ[(1 * NSTATE + s) * (E * NF) + t] = fl(vy[s]) - fl(ny[s]);
+      sJ[(2 * NSTATE + s) * (E * NF) + t] = fl(vz[s]) - fl(nz[s]);
+    }
+  }
+  __syncthreads();
+  // ---- y, and the jumps along a
+  T ug[NSTATE][N];
+  {
+    const SymMat<N, T> I = uniform_load<SymMat<N, T>, T>(&op->I);
+    if (act) {
+#pragma unroll
+      for (int s = 0; s < NSTATE; ++s) {
+        T *p = sA + by + s * NN;
+        T x[N], o[N];
+#pragma unroll
+        for (int q = 0; q < N; ++q) x[q] = p[N * q];
+        sym_apply<N, 1, T>(I, x, o);
+#pragma unroll
+        for (int q = 0; q < N; ++q) p[N * q] = o[q];
+      }
+    }
+    constexpr int JL = 3 * NSTATE * E * N;
+#pragma unroll
+    for (int i0 = 0; i0 < JL; i0 += NTH) {
+      const int i = i0 + t;
+      if (i < JL) {
+        T *p = sJ + N * i;
+        T x[N], o[N];
+#pragma unroll
+        for (int q = 0; q < N; ++q) x[q] = p[q];
+        sym_apply<N, 1, T>(I, x, o);
+#pragma unroll
+        for (int q = 0; q < N; ++q) p[q] = o[q];
+      }
+    }
+    __syncthreads();
+    // ---- z, and the jumps along b
+    if (act) {
+#pragma unroll
+      for (int s = 0; s < NSTATE; ++s) {
+        T *p = sA + bz + s * NN;
+        T x[N];
+#pragma unroll
+        for (int q = 0; q < N; ++q) x[q] = p[NF * q];
+        sym_apply<N, 1, T>(I, x, ug[s]);
+#pragma unroll
+        for (int q = 0; q < N; ++q) p[NF * q] = ug[s][q];
+      }
+    }
+#pragma unroll
+    for (int i0 = 0; i0 < JL; i0 += NTH) {
+      const int i = i0 + t;
+      if (i < JL) {
+        T *p = sJ + (i / N) * NF + i % N;
+        T x[N], o[N];
+#pragma unroll
+        for (int q = 0; q < N; ++q) x[q] = p[N * q];
+        sym_apply<N, 1, T>(I, x, o);
+#pragma unroll
+        for (int q = 0; q < N; ++q) p[N * q] = o[q];
+      }
+    }
+  }
+  __syncthreads();
+  // ---- d
+  // (the face fluxes are loaded a phase before they are used)
+  const size_t plane = (size_t)la.nelem * NF;
+  const T *const ffo = FF + (size_t)k0 * NF;
+  T fz[2][NSTATE], fx[2][NSTATE], fy[2][NSTATE];
+  auto load_faces = [&](T (&f)[2][NSTATE], int l) {
+    if (act) {
+#pragma unroll
+      for (int g = 0; g < 2; ++g)
+#pragma unroll
+        for (int s = 0; s < NSTATE; ++s) f[g][s] = (ffo + ((2 * l + g) * NSTATE + s) * plane)[(unsigned)t];
+    }
+  };
+  if constexpr (!DIAG) load_faces(fz, 2);
+  T jz[NSTATE];
+  {
+    T qx[NSTATE][N], qy[NSTATE][N];
+    if (act) {
+      T jx[NSTATE], jy[NSTATE];
+#pragma unroll
+      for (int s = 0; s < NSTATE; ++s) {
+        jx[s] = sJ[(0 * NSTATE + s) * (E * NF) + t];
+        jy[s] = sJ[(1 * NSTATE + s) * (E * NF) + t];
+        jz[s] = sJ[(2 * NSTATE + s) * (E * NF) + t];
+      }
+      {
+        const SymMat<N, T> Dx = uniform_load<SymMat<N, T>, T>(&op->Dg[0]);
+        const Vec ax = uniform_load<Vec, T>(reinterpret_cast<const Vec *>(op->aeta[0]));
+#pragma unroll
+        for (int s = 0; s < NSTATE; ++s) {
+          const T *p = sA + bx + s * NN;
+          T x[N];
+#pragma unroll
+          for (int q = 0; q < N; ++q) x[q] = p[q];
+          sym_apply<N, -1, T>(Dx, x, qx[s]);
+#pragma unroll
+          for (int q = 0; q < N; ++q) qx[s][q] += ax.r[q] * jx[s];
+        }
+      }
+      {
+        const SymMat<N, T> Dy = uniform_load<SymMat<N, T>, T>(&op->Dg[1]);
+        const Vec ay = uniform_load<Vec, T>(reinterpret_cast<const Vec *>(op->aeta[1]));
+#pragma unroll
+        for (int s = 0; s < NSTATE; ++s) {
+          const T *p = sA + by + s * NN;
+          T x[N];
+#pragma unroll
+          for (int q = 0; q < N; ++q) x[q] = p[N * q];
+          sym_apply<N, -1, T>(Dy, x, qy[s]);
+#pragma unroll
+          for (int q = 0; q < N; ++q) {
+            qy[s][q] += ay.r[q] * jy[s];
+            if (!L::JB) sB[by + s * NN + N * q] = qy[s][q];
+          }
+        }
+      }
+    }
+    __syncthreads();
+    if (act) {
+#pragma unroll
+      for (int s = 0; s < NSTATE; ++s)
+#pragma unroll
+        for (int q = 0; q < N; ++q) {
+          sA[bx + s * NN + q] = qx[s][q];
+          if (L::JB) sB[by + s * NN + N * q] = qy[s][q];
+        }
+    }
+  }
+  __syncthreads();
+  // ---- p
+  T kz[NSTATE][N];
+  if (act) {
+    {
+      const SymMat<N, T> Dz = uniform_load<SymMat<N, T>, T>(&op->Dg[2]);
+      const Vec az = uniform_load<Vec, T>(reinterpret_cast<const Vec *>(op->aeta[2]));
+#pragma unroll
+      for (int s = 0; s < NSTATE; ++s) {
+        sym_apply<N, -1, T>(Dz, ug[s], kz[s]);
+#pragma unroll
+        for (int q = 0; q < N; ++q) kz[s][q] += az.r[q] * jz[s];
+      }
+    }
+    const Bg<T> bg(d.ph);
+#pragma unroll
+    for (int q = 0; q < N; ++q) {
+      T w[NSTATE], g[NGRAD], F[NGRAD];
+#pragma unroll
+      for (int s = 0; s < NSTATE; ++s) {
+        w[s] = ug[s][q];
+        g[s] = sA[bz + s * NN + NF * q];
+        g[NSTATE + s] = sB[bz + s * NN + NF * q];
+        g[2 * NSTATE + s] = kz[s][q];
+      }
+      if constexpr (DIAG) {
+        const double rho = d.ph.rho0 + (double)w[0];
+        const double ir = 1.0 / rho;
+        const double vv[3] = {(double)w[1] * ir, (double)w[2] * ir, (double)w[3] * ir};
+        double gd[15], gv[3][3], ge[3];
+#pragma unroll
+        for (int k = 0; k < 15; ++k) gd[k] = g[k];
+        prim_grads<double>(ir, d.ph.E0 + (double)w[4], vv, gd, gv, ge);
+        const double w1 = gv[2][1] - gv[1][2], w2 = gv[0][2] - gv[2][0], w3 = gv[1][0] - gv[0][1];
+        const double wq = opd->w[a] * opd->w[b] * opd->w[q];
+        dke += wq * 0.5 * ((double)w[1] * vv[0] + (double)w[2] * vv[1] + (double)w[3] * vv[2]);
+        dens += wq * 0.5 * rho * (w1 * w1 + w2 * w2 + w3 * w3);
+        continue;
+      }
+      volume_flux<T>(w, g, bg, F);
+#pragma unroll
+      for (int s = 0; s < NSTATE; ++s) {
+        sA[bz + s * NN + NF * q] = F[s];
+        sB[bz + s * NN + NF * q] = F[NSTATE + s];
+        kz[s][q] = F[2 * NSTATE + s];
+      }
+    }
+    if constexpr (!DIAG) {
+      load_faces(fx, 0);
+      load_faces(fy, 1);
+    }
+    const SymMat<N, T> Dz = uniform_load<SymMat<N, T>, T>(&op->Dh[2]);
+    const Vec eta = uniform_load<Vec, T>(reinterpret_cast<const Vec *>(op->eta));
+#pragma unroll
+    for (int s = 0; s < NSTATE; ++s) {
+      T o[N];
+      sym_apply<N, -1, T>(Dz, kz[s], o);
+#pragma unroll
+      for (int q = 0; q < N; ++q) kz[s][q] = o[q] - (eta.r[q] * fz[0][s] + eta.r[N - 1 - q] * fz[1][s]);
+    }
+  }
+  if constexpr (DIAG) {
+    const double n = group_sum<NTH>(dkn, sred), x = group_sum<NTH>(dke, sred), y = group_sum<NTH>(dens, sred);
+    if (t == 0) {
+      st.ke_part[lb] = n;
+      st.diag_part[2 * lb] = x;
+      st.diag_part[2 * lb + 1] = y;
     }
     return;
   }
-  const long k0 = d.elem_off + kl;    // first element of the block in the arrays
-  const PhysArgs ph = d.ph;
-  // the stage input is the conserved state (UT = double) or its FP32
-  // fluctuation about the background (UT = float, written by the previous
-  // stage's epilogue)
-  constexpr bool FLUCT = sizeof(UT) == 4;
-  const double brho = FLUCT ? 0.0 : ph.rho0, bE = FLUCT ? 0.0 : ph.E0;
-  const double dtb = d.dt * st.cb, dta = d.dt * st.ca;
-  const int tid = threadIdx.x;
-  const SOps<N, T> *so = &sops;
-  const Bg<T> bg(ph);
-  // FP64 view of an element's volume buffer, used by the inverse-mass
-  // sweeps and the epilogue
-  auto md = [&](int e) -> double * { return reinterpret_cast<double *>(&sbuf[e][0]); };
-
-  // The volume lines of the x sweep stage (below): item i = (e, s, ab) of
-  // the block's ne x 5 x N^2 x-lines, in wave-aligned ranges of KP items per
-  // kind.  Their HBM loads are issued here, so that they land while the
-  // face terms are lifted.  Kind 0 computes I u and the y and z jumps, kind
-  // 1 D u and the x jump; when both kinds fit the workgroup side by side
-  // (one element per workgroup at p = 4) they run on separate waves,
-  // otherwise every item does both.
-  constexpr int XL = NSTATE * NF;                    // lines of one direction per element
-  constexpr unsigned KP = (E * XL + 63) / 64 * 64;   // items of one kind, padded to whole waves
-  constexpr bool XSPLIT = 2 * KP <= NT;
-  constexpr int XI = XSPLIT ? 1 : (int)((KP + NT - 1) / NT);
-  const unsigned totx = ne * XL;
-  UT vo[XI][N], vx[XI], vy[XI][N], vz[XI][N];
-  // the item's face terms (lifted to the nodes by the gradient kernel): the
-  // -x face at the line's first node, the +x face at its last, and the
-  // line's nodes on a -y/+y and a -z/+z face where it lies on one
-  T fa[XI], fb[XI], fy[XI][N], fz[XI][N];
-  // Line items (e, s, ab) of the sweep phases below run in kinds of KP
-  // items (a kind = one family of lines, e.g. the z-lines of F_x).  When KP
-  // divides the workgroup (p = 4: E = 2 fills it, E = 1 half of it) a
-  // thread's item is the same in every pass and phase: it is decomposed once
-  // here, and kind_loop gives the thread the kinds (pass * NT / KP +
-  // tid / KP) of its wave-uniform share.
-  constexpr bool HOIST = KP <= NT && NT % KP == 0;
-  struct LineIt {
-    unsigned e, s, ab;
-  };
-  auto line_at = [&](unsigned i) -> LineIt {
-    LineIt L;
-    L.e = i / XL;
-    const unsigned r = i - L.e * XL;
-    L.s = r / NF;
-    L.ab = r - L.s * NF;
-    return L;
-  };
-  const unsigned own_i = HOIST ? (unsigned)tid % KP : 0u;
-  const LineIt own = line_at(own_i < totx ? own_i : 0u);
-  // body(kind, item, pass): pass = the loop pass the item came in (kind-0
-  // items come in passes 0, 1, ... in order)
-  auto kind_loop = [&](const unsigned K, auto &&body) {
-    if constexpr (HOIST) {
-      constexpr unsigned PER = NT / KP;
-#pragma unroll
-      for (unsigned pass = 0; pass < (K + PER - 1) / PER; ++pass) {
-        const unsigned kind = pass * PER + (unsigned)tid / KP;
-        if (kind < K && own_i < totx) body(kind, own, pass);
-      }
-    } else {
-#pragma unroll
-      for (unsigned pass = 0; pass < (K * KP + NT - 1) / NT; ++pass) {
-        const unsigned w = tid + pass * NT;
-        const unsigned kind = w / KP, i = w - kind * KP;
-        if (kind < K && i < totx) body(kind, line_at(i), pass);
-      }
-    }
-  };
-  unsigned xi[XI];                                   // the item, or ~0
-  auto x_item = [&](int it) -> unsigned {
-    const unsigned w = tid + it * NT, i = XSPLIT ? w % KP : w;
-    return i < totx ? i : ~0u;
-  };
-#pragma unroll
-  for (int it = 0; it < XI; ++it) {
-    xi[it] = x_item(it);
-    const unsigned i = xi[it] == ~0u ? totx - 1 : xi[it];
-    const unsigned e = i / XL, r = i - e * XL;       // r = s NF + ab: the line starts at N r in its element
-    const UT *src = U + k0 * (NSTATE * NN) + (e * (NSTATE * NN) + N * r);
-#pragma unroll
-    for (int q = 0; q < N; ++q) vo[it][q] = src[q];
-  }
-
-  fill_neighbors(m, ec, d.elem_off, ne, snb, tid);
-  {
-    // the instance's operator image (8-byte words) into LDS
-    static_assert(sizeof(SOps<N, T>) % 8 == 0, "whole 8-byte words");
-    constexpr int W8 = sizeof(SOps<N, T>) / 8;
-    const int ii = la.blk_inst ? la.blk_inst[lb] : 0;
-    const uint2 *src = reinterpret_cast<const uint2 *>(simg + (long)ii * SOpsImage<N>::BYTES +
-                                                       SOpsImage<N>::template offset<T>());
-    for (int w = tid; w < W8; w += NT) reinterpret_cast<uint2 *>(&sops)[w] = src[w];
-  }
-  if (tid < NSTATE) sbg[tid] = tid == 0 ? ph.rho0 : tid == NSTATE - 1 ? ph.E0 : 0.0;
   __syncthreads();
-  // the neighbours' traces the jumps need: the -x neighbour's node at the
-  // line's start, and the -y (-z) neighbour's x-line along the -y (-z) face;
-  // the latter loaded by every item (from the line itself where the line is
-  // not on that face: unconditional loads are not waited for at a branch)
+  // ---- t
+  if (act) {
+    const Vec eta = uniform_load<Vec, T>(reinterpret_cast<const Vec *>(op->eta));
 #pragma unroll
-  for (int it = 0; it < XI; ++it) {
-    const unsigned i = xi[it] == ~0u ? totx - 1 : xi[it];
-    const unsigned e = i / XL, r = i - e * XL, s = r / NF, ab = r - s * NF;
-    const unsigned iy = ab % N, iz = ab / N;
-    const UT *own = U + k0 * (NSTATE * NN) + (e * (NSTATE * NN) + N * r);
-    vx[it] = U[snb[e][0] * (NSTATE * NN) + (N * r + (N - 1))];
-    const UT *ny = iy == 0 ? U + snb[e][2] * (NSTATE * NN) + (s * NN + N * (N - 1) + NF * iz) : own;
-    const UT *nz = iz == 0 ? U + snb[e][4] * (NSTATE * NN) + (s * NN + NF * (N - 1) + N * iy) : own;
+    for (int l = 0; l < 2; ++l) {
+      const SymMat<N, T> Dh = uniform_load<SymMat<N, T>, T>(&op->Dh[l]);
 #pragma unroll
-    for (int q = 0; q < N; ++q) {
-      vy[it][q] = ny[q];
-      vz[it][q] = nz[q];
-    }
-    // FF[element][2 d + side][state][node]: side 0 of the element's own
-    // record for its -d faces, side 1 of the +d neighbour's for its +d faces
-    constexpr int CH = L::CH, FE = L::FE;
-    const T *const ffo = FF + (k0 + e) * FE + s * NF;
-    fa[it] = ffo[ab];
-    fb[it] = FF[snb[e][1] * FE + (CH + s * NF + ab)];
-    const T *fyp = iy == N - 1 ? FF + snb[e][3] * FE + (3 * CH + s * NF + N * iz) : ffo + 2 * CH + N * iz;
-    const T *fzp = iz == N - 1 ? FF + snb[e][5] * FE + (5 * CH + s * NF + N * iy) : ffo + 4 * CH + N * iy;
+      for (int s = 0; s < NSTATE; ++s) {
+        T *p = l == 0 ? sA + bx + s * NN : sB + by + s * NN;
+        T x[N], o[N];
 #pragma unroll
-    for (int q = 0; q < N; ++q) {
-      fy[it][q] = fyp[q];
-      fz[it][q] = fzp[q];
-    }
-  }
-
-  // ================= volume =================
-  // The state and its gradient at the volume Gauss points, from the state
-  // alone.  The gradient kernel's Q_l = (1/alpha_l) (Dn u + L0 J_l) along
-  // direction l (J_l: the jump u - u_nbr on the element's -l face, the only
-  // face whose neighbour trace enters the one-sided LDG gradient),
-  // interpolated to the Gauss points, factorises as
-  //   Q_l = (1/alpha_l) [ D_l (x) I (x) I u + (I L0)_l (x) (I (x) I) J_l ]
-  // with D = I Dn, the basis derivatives at the Gauss points (exact: the
-  // derivative of a basis polynomial lies in their span).  Sweeps:
-  //   x (lines from HBM):  X = I u,  Q_x <- D u + IL0 J_x;  J_y, J_z <- I J
-  //   y:  XY = I X,  Q_y <- D X + IL0 (I J_y);  Q_x <- I Q_x;  J_z <- I J_z
-  //   z:  u_g = I XY,  Q_z <- D XY + IL0 (I I J_z);  Q_x, Q_y <- I Q
-  // (45 field sweeps instead of 60 for interpolating a stored gradient, and
-  // no gradient traffic).  Fields of the volume buffer: u 0-4, Q_l 5+5l..;
-  // the y and z jumps after them.  In type T on fluctuations about the
-  // background, as the face terms.  A line item (e, s, ab) names the x-line
-  // (y, z) = (a, b), the y-line (x, z) = (a, b) and the z-line (x, y) =
-  // (a, b) of field s; each stage runs its kinds of lines in wave-aligned
-  // ranges of KP items.
-  auto sjy = [&](int e) -> T * { return &sbuf[e][L::SJ0]; };
-  auto sjz = [&](int e) -> T * { return &sbuf[e][L::SJ0 + L::SJ]; };
-  {
-    SymReg<N, T> I, Dx;
-    I.load(so->I);
-    Dx.load(so->Ds[0]);
-    T l0[N];
+        for (int q = 0; q < N; ++q) x[q] = p[l == 0 ? q : N * q];
+        sym_apply<N, -1, T>(Dh, x, o);
 #pragma unroll
-    for (int q = 0; q < N; ++q) l0[q] = so->il0[0][q];
-#pragma unroll
-    for (int it = 0; it < XI; ++it) {
-      if (xi[it] == ~0u) continue;
-      const unsigned i = xi[it];
-      const unsigned e = i / XL, r = i - e * XL, s = r / NF, ab = r - s * NF;
-      const unsigned iy = ab % N, iz = ab / N;
-      const double bgs = s == 0 ? brho : s == 4 ? bE : 0.0;
-      auto fl = [&](UT x) -> T { return FLUCT ? T(x) : T((double)x - bgs); };
-      const bool k0s = !XSPLIT || tid < KP, k1s = !XSPLIT || tid >= KP;   // kinds of this item
-      T u[N], o[N];
-#pragma unroll
-      for (int q = 0; q < N; ++q) u[q] = fl(vo[it][q]);
-      T *px = &sbuf[e][N * r];
-      if (k0s) {
-        sym_apply<N, 1, T>(I.m, u, o);
-#pragma unroll
-        for (int q = 0; q < N; ++q) px[q] = o[q];
-        if (iy == 0) {
-          T j[N];
-#pragma unroll
-          for (int q = 0; q < N; ++q) j[q] = u[q] - fl(vy[it][q]);
-          sym_apply<N, 1, T>(I.m, j, o);
-#pragma unroll
-          for (int q = 0; q < N; ++q) sjy(e)[s * NF + q + N * iz] = o[q];
-        }
-        if (iz == 0) {
-          T j[N];
-#pragma unroll
-          for (int q = 0; q < N; ++q) j[q] = u[q] - fl(vz[it][q]);
-          sym_apply<N, 1, T>(I.m, j, o);
-#pragma unroll
-          for (int q = 0; q < N; ++q) sjz(e)[s * NF + q + N * iy] = o[q];
-        }
-      }
-      if (k1s) {
-        const T jx = u[0] - fl(vx[it]);
-        sym_apply<N, -1, T>(Dx.m, u, o);
-#pragma unroll
-        for (int q = 0; q < N; ++q) px[NSTATE * NN + q] = o[q] + l0[q] * jx;
+        for (int q = 0; q < N; ++q)
+          p[l == 0 ? q : N * q] = o[q] - (eta.r[q] * (l == 0 ? fx : fy)[0][s] + eta.r[N - 1 - q] * (l == 0 ? fx : fy)[1][s]);
       }
     }
   }
   __syncthreads();
-  // y sweeps: kind 0 I X (in place) and D X + IL0 J_y into the Q_y slot;
-  // kind 1 I Q_x (in place); then I J_z along y
-  {
-    SymReg<N, T> I, Dy;
-    I.load(so->I);
-    Dy.load(so->Ds[1]);
-    T l0[N];
-#pragma unroll
-    for (int q = 0; q < N; ++q) l0[q] = so->il0[1][q];
-    kind_loop(2, [&](unsigned kind, const LineIt &L, unsigned pass) {
-      const unsigned a = L.ab % N, b = L.ab / N;
-      T *p = &sbuf[L.e][(kind == 0 ? L.s : NSTATE + L.s) * NN + a + NF * b];
-      T v[N], o[N];
-#pragma unroll
-      for (int q = 0; q < N; ++q) v[q] = p[N * q];
-      sym_apply<N, 1, T>(I.m, v, o);
-#pragma unroll
-      for (int q = 0; q < N; ++q) p[N * q] = o[q];
-      if (kind == 0) {
-        const T jy = sjy(L.e)[L.s * NF + L.ab];
-        sym_apply<N, -1, T>(Dy.m, v, o);
-        T *pq = p + 2 * NSTATE * NN;
-#pragma unroll
-        for (int q = 0; q < N; ++q) pq[N * q] = o[q] + l0[q] * jy;
-      }
-    });
-    for (unsigned w = tid; w < (unsigned)ne * NSTATE * N; w += NT) {
-      const unsigned e = w / (NSTATE * N), r = w - e * (NSTATE * N);
-      T *p = sjz(e) + (r / N) * NF + r % N;
-      T v[N], o[N];
-#pragma unroll
-      for (int q = 0; q < N; ++q) v[q] = p[N * q];
-      sym_apply<N, 1, T>(I.m, v, o);
-#pragma unroll
-      for (int q = 0; q < N; ++q) p[N * q] = o[q];
-    }
-  }
-  __syncthreads();
-  // z sweeps: kind 0 I XY (in place) and D XY + IL0 J_z into the Q_z slot;
-  // kinds 1 and 2 I Q_x and I Q_y (in place).  Where the z jumps share the
-  // Q_z slot (FP64), each kind-0 item reads its jump before a barrier that
-  // precedes the first Q_z store.
-  {
-    SymReg<N, T> I, Dz;
-    I.load(so->I);
-    Dz.load(so->Ds[2]);
-    T l0[N];
-#pragma unroll
-    for (int q = 0; q < N; ++q) l0[q] = so->il0[2][q];
-    constexpr int ZI = HOIST ? 1 : (int)((KP + NT - 1) / NT);   // kind-0 items per thread
-    T jzr[ZI];
-#pragma unroll
-    for (int it = 0; it < ZI; ++it) {
-      const unsigned i = HOIST ? own_i : tid + it * NT;
-      const LineIt L = HOIST ? own : line_at(i < totx ? i : 0u);
-      jzr[it] = (HOIST ? (unsigned)tid < KP : i < KP) && i < totx ? sjz(L.e)[L.s * NF + L.ab] : T(0);
-    }
-    if constexpr (L::JQZ) __syncthreads();
-    kind_loop(3, [&](unsigned kind, const LineIt &L, unsigned pass) {
-      T *p = &sbuf[L.e][(kind * NSTATE + L.s) * NN + L.ab];
-      T v[N], o[N];
-#pragma unroll
-      for (int q = 0; q < N; ++q) v[q] = p[NF * q];
-      sym_apply<N, 1, T>(I.m, v, o);
-#pragma unroll
-      for (int q = 0; q < N; ++q) p[NF * q] = o[q];
-      if (kind == 0) {
-        // this item's jump (kind-0 items come in passes 0 .. ZI-1)
-        const T jz = jzr[HOIST ? 0 : pass];
-        sym_apply<N, -1, T>(Dz.m, v, o);
-        T *pq = p + 3 * NSTATE * NN;
-#pragma unroll
-        for (int q = 0; q < N; ++q) pq[NF * q] = o[q] + l0[q] * jz;
-      }
-    });
-  }
-  __syncthreads();
-
-  // pointwise volume flux, weighted; optional Gauss diagnostics (FP64 sums)
-  double dke = 0.0, dens = 0.0;
-  for (int w = tid; w < ne * NN; w += NT) {
-    const int e = w / NN, q = w - e * NN;
-    T *pv = &sbuf[e][q];
-    T u[5], g[15], F[15];
-#pragma unroll
-    for (int s = 0; s < 5; ++s) u[s] = pv[s * NN];
-#pragma unroll
-    for (int k = 0; k < 15; ++k) g[k] = pv[(NSTATE + k) * NN];
-    if (st.diag_part) {
-      const double rho = ph.rho0 + (double)u[0];
-      const double ir = 1.0 / rho;
-      const double v[3] = {(double)u[1] * ir, (double)u[2] * ir, (double)u[3] * ir};
-      double gd[15], gv[3][3], ge[3];
-#pragma unroll
-      for (int k = 0; k < 15; ++k) gd[k] = g[k];
-      prim_grads<double>(ir, ph.E0 + (double)u[4], v, gd, gv, ge);
-      const double w1 = gv[2][1] - gv[1][2], w2 = gv[0][2] - gv[2][0], w3 = gv[1][0] - gv[0][1];
-      const double wq = so->wd[q % N] * so->wd[(q / N) % N] * so->wd[q / NF];
-      dke += wq * 0.5 * ((double)u[1] * v[0] + (double)u[2] * v[1] + (double)u[3] * v[2]);
-      dens += wq * 0.5 * rho * (w1 * w1 + w2 * w2 + w3 * w3);
-    }
-    volume_flux<T>(u, g, bg, F);
-    const T wq = so->w[q % N] * so->w[(q / N) % N] * so->w[q / NF];
-#pragma unroll
-    for (int l = 0; l < 3; ++l) {
-      const T sc = wq * T(m.ialpha[l]);
-#pragma unroll
-      for (int s = 0; s < 5; ++s) pv[(NSTATE + 5 * l + s) * NN] = F[s + 5 * l] * sc;
-    }
-  }
-  if (st.diag_part) {
-    const double a = block_sum(dke, sred);
-    __syncthreads();
-    const double b = block_sum(dens, sred);
-    if (tid == 0) { st.diag_part[2 * lb] = a; st.diag_part[2 * lb + 1] = b; }
-  }
-  __syncthreads();
-
-  // test-function contraction: z sweep (kinds 0, 1: I^T on F_x, F_y; kind
-  // 2: D^T on F_z)
-  {
-    SymReg<N, T> It, Dt;
-    It.load(so->It);
-    Dt.load(so->Dt);
-    kind_loop(3, [&](unsigned kind, const LineIt &L, unsigned pass) {
-      T *p = &sbuf[L.e][(NSTATE + kind * NSTATE + L.s) * NN + L.ab];
-      T v[N], o[N];
-#pragma unroll
-      for (int q = 0; q < N; ++q) v[q] = p[q * NF];
-      if (kind < 2) sym_apply<N, 1, T>(It.m, v, o);
-      else sym_apply<N, -1, T>(Dt.m, v, o);
-#pragma unroll
-      for (int i = 0; i < N; ++i) p[i * NF] = o[i];
-    });
-  }
-  __syncthreads();
-  // y sweep: F_x <- I^T F_x ; G <- D^T F_y + I^T F_z (stored in the F_y slot)
-  {
-    SymReg<N, T> It;
-    It.load(so->It);
-    kind_loop(1, [&](unsigned, const LineIt &L, unsigned) {
-      const unsigned base = (L.ab % N) + NF * (L.ab / N);
-      T *px = &sbuf[L.e][(NSTATE + L.s) * NN + base];
-      T *py = px + NSTATE * NN;
-      const T *pz = px + 2 * NSTATE * NN;
-      T vx[N], vy[N], vz[N], ox[N], og[N];
-#pragma unroll
-      for (int q = 0; q < N; ++q) { vx[q] = px[q * N]; vy[q] = py[q * N]; vz[q] = pz[q * N]; }
-      sym_apply<N, 1, T>(It.m, vx, ox);
-      sym_apply2<N, -1, 1, T>(so->Dt, vy, It.m, vz, og);
-#pragma unroll
-      for (int i = 0; i < N; ++i) {
-        px[i * N] = ox[i];
-        py[i * N] = og[i];
-      }
-    });
-  }
-  __syncthreads();
-  // x sweep: r = D^T F_x + I^T G + face residual (T), then M1^{-1} along x
-  // in FP64.  The FP64 result goes to the start of the element's buffer
-  // (5 FP64 fields), which overlaps the F_x fields still being read by other
-  // threads when T = float: every thread keeps its results in registers
-  // until all reads are done.
-  {
-    constexpr int XR = HOIST ? 1 : (E * XL + NT - 1) / NT;
-    double res[XR][N];
-    bool has[XR];
-    SymReg<N, T> It;
-    It.load(so->It);
-    // volume minus the face terms of the line's nodes (the gradient
-    // kernel's lifted face fluxes, loaded with the x-stage lines: item it)
-    auto xline = [&](const LineIt &L, int it, double (&out)[N]) {
-      const unsigned base = N * L.ab;
-      const T *px = &sbuf[L.e][(NSTATE + L.s) * NN + base];
-      const T *pg = px + NSTATE * NN;
-      T vx[N], vg[N], o[N];
-      double rr[N];
-#pragma unroll
-      for (int q = 0; q < N; ++q) { vx[q] = px[q]; vg[q] = pg[q]; }
-      sym_apply2<N, -1, 1, T>(so->Dt, vx, It.m, vg, o);
-      o[0] -= fa[it];
-      o[N - 1] -= fb[it];
-      const unsigned iy = L.ab % N, iz = L.ab / N;
-      if (iy == 0 || iy == N - 1) {
-#pragma unroll
-        for (int i = 0; i < N; ++i) o[i] -= fy[it][i];
-      }
-      if (iz == 0 || iz == N - 1) {
-#pragma unroll
-        for (int i = 0; i < N; ++i) o[i] -= fz[it][i];
-      }
-#pragma unroll
-      for (int i = 0; i < N; ++i) rr[i] = (double)o[i];
-      sym_apply<N, 1, double>(so->Mi, rr, out);
-    };
-    if constexpr (HOIST) {
-      has[0] = tid < (int)KP && own_i < totx;
-      if (has[0]) xline(own, 0, res[0]);
-    } else {
-#pragma unroll
-      for (int it = 0; it < XR; ++it) {
-        const unsigned w = tid + it * NT;
-        has[it] = w < totx;
-        if (has[it]) xline(line_at(w), it, res[it]);
-      }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int it = 0; it < XR; ++it) {
-      if (!has[it]) continue;
-      const LineIt L = HOIST ? own : line_at(tid + it * NT);
-      double *po = md(L.e) + L.s * NN + N * L.ab;
-#pragma unroll
-      for (int i = 0; i < N; ++i) po[i] = res[it][i];
-    }
-  }
-  __syncthreads();
-  // FP64 layout: the RK epilogue's HBM operands (u^n and the running sum)
-  // are copied straight into the part of the volume buffer that is free from
-  // here on (after the 5 FP64 result fields) by LDS-direct loads, so their
-  // latency is covered by the inverse-mass sweeps below (1.5 % faster at
-  // 64^3, p = 4).  The FP32 layout has room for one of the two only; there
-  // they are loaded into registers at the same point instead.
-  const bool need_u0 = st.acc || st.unext || st.unext32;
+  // ---- zi, yi, xi (FP64)
+  const bool need_u0 = (st.acc && st.acc_init) || st.unext || st.unext32;
   const bool need_acc = st.acc && !st.acc_init;
-  constexpr bool PF = sizeof(T) == sizeof(double);
-  auto pf_u0 = [&](int e) -> double * { return md(e) + NSTATE * NN; };
-  auto pf_acc = [&](int e) -> double * { return md(e) + 2 * NSTATE * NN; };
-  if (PF) {
-    constexpr int DW = 2 * NSTATE * NN;    // dwords per element and array
-    const int lane = tid & 63, wave = tid >> 6;
-    for (int e = 0; e < ne; ++e) {
-      const long gofs_e = (k0 + e) * NSTATE * NN;
-      for (int c = wave; c * 64 < DW; c += NT / 64) {
-        const int i = c * 64 + lane;
-        if (i < DW) {
-          if (need_u0)
-            __builtin_amdgcn_global_load_lds(reinterpret_cast<const unsigned *>(st.u0 + gofs_e) + i,
-                                             (__attribute__((address_space(3))) void *)(reinterpret_cast<unsigned *>(pf_u0(e)) + c * 64),
-                                             4, 0, 0);
-          if (need_acc)
-            __builtin_amdgcn_global_load_lds(reinterpret_cast<const unsigned *>(st.acc + gofs_e) + i,
-                                             (__attribute__((address_space(3))) void *)(reinterpret_cast<unsigned *>(pf_acc(e)) + c * 64),
-                                             4, 0, 0);
+  const long gofs = k0 * EV;
+  // Epilogue items: word it NTH + t of the block's values of one variable
+  // (element after element), for variable 0 at `ew` past the block's base in
+  // every (node, state, element) array and at `lw` in the FP64 buffer, and s
+  // N^3 further for variable s.  (Coalesced, through LDS: with the epilogue on
+  // the thread's own x-lines, lanes 8 N bytes apart, the mixed kernel was 5 %
+  // slower at 64^3, p = 4, the FP64 kernel the same.)
+  constexpr int EPI = (E * NN + NTH - 1) / NTH;
+  unsigned ew[EPI], lw[EPI];
+#pragma unroll
+  for (int it = 0; it < EPI; ++it) {
+    const int i = t + it * NTH, j = i < ne * NN ? i : ne * NN - 1;
+    ew[it] = (unsigned)(j + j / NN * (EV - NN));
+    lw[it] = (unsigned)(j + j / NN * (ES - NN));
+  }
+  // (a uniform base and a 32-bit byte offset: no 64-bit address per item)
+  auto at = [&](auto *p, int it) {
+    return reinterpret_cast<decltype(p)>((char *)p + ew[it] * (unsigned)sizeof(*p));
+  };
+  double ru[EPI][NSTATE], ra[EPI][NSTATE];
+  {
+    const SymMat<N, double> Ii = uniform_load<SymMat<N, double>, double>(&opd->Ii);
+    constexpr bool INPLACE = sizeof(T) == sizeof(double);   // a thread's FP64 results replace its own A values
+    {
+      double r[NSTATE][N];
+      if (act) {
+#pragma unroll
+        for (int s = 0; s < NSTATE; ++s) {
+          double x[N];
+#pragma unroll
+          for (int q = 0; q < N; ++q)
+            x[q] = (double)(kz[s][q] + (sA[bz + s * NN + NF * q] + sB[bz + s * NN + NF * q]));
+          sym_apply<N, 1, double>(Ii, x, r[s]);
         }
       }
-    }
-  }
-  // Epilogue items.  The block's values are contiguous in every (node,
-  // state, element) array: group g = 5 e + s (element e, state s) is words
-  // g N^3 .. g N^3 + N^3 - 1 past the block's base gofs (uniform base,
-  // 32-bit offset), and words e BUFD + s N^3 + q of the FP64 view of the
-  // volume buffer.  Item (it, thread t) is word w = t + it NT.  When N^3 is
-  // a multiple of the wave (N = 4) a wave's items lie in one group, which
-  // is then computed as a wave-uniform value (no per-lane division).
-  constexpr int EPI = (E * NSTATE * NN + NT - 1) / NT;
-  constexpr bool GS = NN % 64 == 0;
-  constexpr unsigned BUFD = L::BUF * sizeof(T) / sizeof(double);   // an element's buffer, in doubles
-  const unsigned tot_epi = ne * NSTATE * NN;
-  const long gofs = k0 * NSTATE * NN;
-  struct EpiItem {
-    bool ok;
-    unsigned w, li, s;   // word past gofs, word of the FP64 view, state
-  };
-  auto epi_item = [&](int it) -> EpiItem {
-    EpiItem x;
-    unsigned g, q;
-    if constexpr (GS) {
-      g = (unsigned)__builtin_amdgcn_readfirstlane((int)((tid + it * NT) / NN));
-      q = (unsigned)tid % NN;
-    } else {
-      g = (tid + it * NT) / NN;
-      q = tid + it * NT - g * NN;
-    }
-    const unsigned e = g / NSTATE;
-    x.w = g * NN + q;
-    x.ok = x.w < tot_epi;
-    x.s = g - e * NSTATE;
-    x.li = x.w + e * (BUFD - NSTATE * NN);
-    return x;
-  };
-  double ru[EPI], ra[EPI];
-  {
-    const double *const u0b = st.u0 + gofs, *const accb = st.acc + gofs;
+      if (!INPLACE) __syncthreads();
+      if (act) {
 #pragma unroll
-    for (int it = 0; it < EPI; ++it) {
-      const EpiItem x = epi_item(it);
-      ru[it] = 0.0;
-      ra[it] = 0.0;
-      if (!PF && x.ok) {
-        if (need_u0) ru[it] = u0b[x.w];
-        if (need_acc) ra[it] = accb[x.w];
+        for (int s = 0; s < NSTATE; ++s)
+#pragma unroll
+          for (int q = 0; q < N; ++q) md[bz + s * NN + NF * q] = r[s][q];
       }
     }
+    // the epilogue's HBM operands, covered by the sweeps below
+    if (need_u0) {
+      const double *const p = st.u0 + gofs;
+#pragma unroll
+      for (int it = 0; it < EPI; ++it)
+#pragma unroll
+        for (int v = 0; v < NSTATE; ++v) ru[it][v] = at(p, it)[v * NN];
+    }
+    __syncthreads();
+    if (act) {
+#pragma unroll
+      for (int s = 0; s < NSTATE; ++s) {
+        double *p = md + by + s * NN;
+        double x[N], o[N];
+#pragma unroll
+        for (int q = 0; q < N; ++q) x[q] = p[N * q];
+        sym_apply<N, 1, double>(Ii, x, o);
+#pragma unroll
+        for (int q = 0; q < N; ++q) p[N * q] = o[q];
+      }
+    }
+    if (need_acc) {
+      const double *const p = st.acc + gofs;
+#pragma unroll
+      for (int it = 0; it < EPI; ++it)
+#pragma unroll
+        for (int v = 0; v < NSTATE; ++v) ra[it][v] = at(p, it)[v * NN];
+    }
+    __syncthreads();
+    if (act) {
+#pragma unroll
+      for (int s = 0; s < NSTATE; ++s) {
+        double *p = md + bx + s * NN;
+        double x[N], o[N];
+#pragma unroll
+        for (int q = 0; q < N; ++q) x[q] = p[q];
+        sym_apply<N, 1, double>(Ii, x, o);
+#pragma unroll
+        for (int q = 0; q < N; ++q) p[q] = o[q];
+      }
+    }
+    __syncthreads();
   }
-  // M1^{-1} along y, then along z (FP64)
+
+  // ---- epilogue (FP64): k, RK4 accumulation and next stage input
+  {
+    const double dtb = d.dt * st.cb, dta = d.dt * st.ca;
+    // background of variable v (the FP32 copies are fluctuations)
+    const double bg[NSTATE] = {d.ph.rho0, 0.0, 0.0, 0.0, d.ph.E0};
+    auto items = [&](auto &&body) {
 #pragma unroll
-  for (int dd = 1; dd < 3; ++dd) {
-    {
-      SymReg<N, double> Mi;
-      Mi.load(so->Mi);
-      kind_loop(1, [&](unsigned, const LineIt &L, unsigned) {
-        constexpr unsigned LS[3] = {1, N, N * N};
-        const unsigned a = L.ab % N, b = L.ab / N;
-        double *p = md(L.e) + L.s * NN + (dd == 1 ? a + NF * b : a + N * b);
-        double v[N], o[N];
+      for (int it = 0; it < EPI; ++it)
+        if (t + it * NTH < ne * NN) {
 #pragma unroll
-        for (int i = 0; i < N; ++i) v[i] = p[i * LS[dd]];
-        sym_apply<N, 1, double>(Mi.m, v, o);
-#pragma unroll
-        for (int i = 0; i < N; ++i) p[i * LS[dd]] = o[i];
+          for (int v = 0; v < NSTATE; ++v) body(it, v, md + lw[it] + v * NN);
+        }
+    };
+    if (st.corr) {
+      const double *const p = st.corr + gofs;
+      const unsigned char *const gate = st.gate + k0;
+      items([&](int it, int v, double *k) {
+        if (gate[ew[it] / EV]) *k += at(p, it)[v * NN];
       });
     }
-    __syncthreads();
-  }
-
-  // the LDS-direct loads above have landed once this wave's memory counter
-  // is zero; the barrier makes every wave's copies visible
-  if (PF) {
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
-  }
-
-  // ---- epilogue (FP64): k, RK4 accumulation and next stage input.  All of
-  // a thread's HBM reads are issued before any is used.
-  {
-    double *const mb = md(0);
-    double kv[EPI];
-#pragma unroll
-    for (int it = 0; it < EPI; ++it) {
-      const EpiItem x = epi_item(it);
-      kv[it] = 0.0;
-      if (x.ok) {
-        if (PF && need_u0) ru[it] = mb[x.li + NSTATE * NN];
-        if (PF && need_acc) ra[it] = mb[x.li + 2 * NSTATE * NN];
-        kv[it] = mb[x.li];
-        if (st.corr && st.gate[k0 + x.w / (NSTATE * NN)]) kv[it] += st.corr[gofs + x.w];
-      }
+    if (st.kout) {
+      double *const p = st.kout + gofs;
+      items([&](int it, int v, double *k) { at(p, it)[v * NN] = *k; });
     }
-    if (st.ke_part) __syncthreads();   // every k read before the new state reuses the buffer
-    double *const koutb = st.kout + gofs, *const accb = st.acc + gofs, *const unextb = st.unext + gofs;
-    float *const next32b = st.next32 + gofs, *const unext32b = st.unext32 + gofs;
+    if (st.acc_init) {
 #pragma unroll
-    for (int it = 0; it < EPI; ++it) {
-      const EpiItem x = epi_item(it);
-      if (x.ok) {
-        const unsigned w = x.w;
-        const double k = kv[it];
-        // background of the item's state variable (the FP32 copies are fluctuations)
-        const double bgv = sbg[x.s];
-        if (st.kout) koutb[w] = k;
-        if (st.acc) {
-          const double a = (st.acc_init ? ru[it] : ra[it]) + dtb * k;
-          accb[w] = a;
-          if (st.ke_part) mb[x.li] = a;
-          if (st.next32) next32b[w] = (float)(a - bgv);
+      for (int it = 0; it < EPI; ++it)
+#pragma unroll
+        for (int v = 0; v < NSTATE; ++v) ra[it][v] = ru[it][v];
+    }
+    // one branch-free loop per combination of outputs
+    auto step = [&](auto acc, auto un, auto un32, auto nx32) {
+      double *const pa = st.acc + gofs, *const pu = st.unext + gofs;
+      float *const pu32 = st.unext32 + gofs, *const pn32 = st.next32 + gofs;
+      items([&](int it, int v, double *kp) {
+        const double k = *kp;
+        if constexpr (un) at(pu, it)[v * NN] = ru[it][v] + dta * k;
+        if constexpr (un32) at(pu32, it)[v * NN] = (float)(ru[it][v] + dta * k - bg[v]);
+        if constexpr (acc) {
+          ra[it][v] += dtb * k;
+          at(pa, it)[v * NN] = ra[it][v];
         }
-        if (st.unext) unextb[w] = ru[it] + dta * k;
-        if (st.unext32) unext32b[w] = (float)(ru[it] + dta * k - bgv);
-      }
+        if constexpr (nx32) at(pn32, it)[v * NN] = (float)(ra[it][v] - bg[v]);
+      });
+    };
+    constexpr std::true_type Y;
+    constexpr std::false_type X;
+    if (st.acc) {
+      if (st.unext) step(Y, Y, X, X);
+      else if (st.unext32) step(Y, X, Y, X);
+      else if (st.next32) step(Y, X, X, Y);
+      else step(Y, X, X, X);
+    } else if (st.unext32) {
+      step(X, X, Y, X);
     }
+    if (st.ke_part) items([&](int it, int v, double *k) { *k = ra[it][v]; });
   }
   if (st.ke_part) {
     __syncthreads();
     double kel = 0.0;
-    for (int w = tid; w < ne * NN; w += NT) {
-      const int e = w / NN, q = w - e * NN;
-      const double *a = md(e);
-      const double rho = a[q], m1 = a[NN + q], m2 = a[2 * NN + q], m3 = a[3 * NN + q];
-      const double wq = so->wd[q % N] * so->wd[(q / N) % N] * so->wd[q / NF];
-      kel += wq * (m1 * m1 + m2 * m2 + m3 * m3) / (2.0 * rho);
+    if (act) {
+#pragma unroll
+      for (int q = 0; q < N; ++q) {
+        const double *x = md + bz + NF * q;
+        const double rho = x[0], m1 = x[NN], m2 = x[2 * NN], m3 = x[3 * NN];
+        kel += opd->w[a] * opd->w[b] * opd->w[q] * (m1 * m1 + m2 * m2 + m3 * m3) / (2.0 * rho);
+      }
     }
-    const double t = block_sum(kel, sred);
-    if (tid == 0) st.ke_part[lb] = t;
+    const double x = group_sum<NTH>(kel, sred);
+    if (t == 0) st.ke_part[lb] = x;
   }
 }
 
