@@ -10,7 +10,7 @@
 
 #include "basis.hpp"
 #include "ldg.h"
-#include "ldg_kernels.hpp"
+#include "wave_kernels.hpp"
 
 struct ldg_closure;
 
@@ -19,7 +19,7 @@ namespace ldg_host {
 using namespace ldg;
 
 // Candidate tilings (elements per workgroup) per kernel and order.
-constexpr int kMaxCand = 2;
+constexpr int kMaxCand = 3;
 // steps of kinetic-energy history held on the device (per instance); a call
 // recording more steps copies the history out in chunks of this many
 constexpr int kKeHistSteps = 1024;
@@ -32,12 +32,13 @@ struct Inst {
   int group, slot;        // group and position inside it
 };
 
-// Per (group, candidate E): instance table and block -> instance map.
+// A numbering of a group's elements by workgroups of E: its part of the
+// group's instance tables, and the block -> instance map.
 struct Tiling {
   int E = 1, nblocks = 0;
-  InstDesc *d_inst = nullptr;
-  int *d_blk = nullptr;   // nullptr when the group has one instance
-  std::vector<InstDesc> h_inst;
+  bool bricks = false;
+  const InstDesc *d_inst = nullptr;
+  const int *d_blk = nullptr;   // nullptr when the group has one instance
 };
 
 // Learned-closure state of one group (inference buffers, device).
@@ -64,7 +65,13 @@ struct Group {
   double *ke_part = nullptr, *diag_part = nullptr, *d_scale = nullptr;
   void *ops = nullptr;
   void *sops = nullptr;   // the kernels' operator images (GImage), one per member
-  Tiling rhs[kMaxCand], grad[kMaxCand], nodal;
+  // the numberings in use (each once), their instance tables one after the
+  // other and then their maps in one device block, and the host's copy of the
+  // instance tables
+  std::vector<Tiling> tile;
+  std::vector<InstDesc> h_inst;
+  void *tables = nullptr;
+  int rhs[kMaxCand], grad[kMaxCand], nodal;   // per candidate, its numbering in tile
   int crhs = 0, cgrad = 0;   // chosen candidates
   Basis1D basis;
   GroupClosure cl;

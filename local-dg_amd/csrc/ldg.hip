@@ -50,27 +50,48 @@ int fail(ldg_handle *h, int code, const char *msg) {
   return code;
 }
 
-// Candidate elements per workgroup of each kernel, per order (the
-// autotuner picks among them; index 0 is the default).
+// Candidate kernels per order (the autotuner picks among them): 0 and 1 are
+// ldg_kernels.hpp's kernels with so many elements per workgroup, 2 is
+// wave_kernels.hpp's (as many elements as one wave has lines for).  Without
+// the autotuner, default_cand chooses.
+constexpr int kWaveCand = 2;
 template <int N> struct Cand;
-template <> struct Cand<2> { static constexpr int rhs[kMaxCand] = {16, 32}, grad[kMaxCand] = {16, 32}; };
-template <> struct Cand<3> { static constexpr int rhs[kMaxCand] = {7, 14}, grad[kMaxCand] = {7, 14}; };
-template <> struct Cand<4> { static constexpr int rhs[kMaxCand] = {4, 8}, grad[kMaxCand] = {4, 8}; };
-template <> struct Cand<5> { static constexpr int rhs[kMaxCand] = {2, 5}, grad[kMaxCand] = {5, 2}; };
-template <> struct Cand<6> { static constexpr int rhs[kMaxCand] = {3, 1}, grad[kMaxCand] = {3, 5}; };
+template <> struct Cand<2> { static constexpr int rhs[2] = {16, 32}, grad[2] = {16, 32}; };
+template <> struct Cand<3> { static constexpr int rhs[2] = {7, 14}, grad[2] = {7, 14}; };
+template <> struct Cand<4> { static constexpr int rhs[2] = {4, 8}, grad[2] = {4, 8}; };
+template <> struct Cand<5> { static constexpr int rhs[2] = {2, 5}, grad[2] = {5, 2}; };
+template <> struct Cand<6> { static constexpr int rhs[2] = {3, 1}, grad[2] = {3, 5}; };
 // elements per workgroup of the nodal gradient kernel (256 threads)
 template <int N> struct NodalE { static constexpr int value = N == 2 ? 16 : N == 3 ? 8 : N == 4 ? 4 : N == 5 ? 2 : 1; };
 int nodal_e(int n) { return n == 2 ? 16 : n == 3 ? 8 : n == 4 ? 4 : n == 5 ? 2 : 1; }
 
+template <int N>
+int cand_e_n(bool rhs, int c) {
+  return c == kWaveCand ? WaveE<N>::value : rhs ? Cand<N>::rhs[c] : Cand<N>::grad[c];
+}
 int cand_e(int n, bool rhs, int c) {
   switch (n) {
-    case 2: return rhs ? Cand<2>::rhs[c] : Cand<2>::grad[c];
-    case 3: return rhs ? Cand<3>::rhs[c] : Cand<3>::grad[c];
-    case 4: return rhs ? Cand<4>::rhs[c] : Cand<4>::grad[c];
-    case 5: return rhs ? Cand<5>::rhs[c] : Cand<5>::grad[c];
-    case 6: return rhs ? Cand<6>::rhs[c] : Cand<6>::grad[c];
+    case 2: return cand_e_n<2>(rhs, c);
+    case 3: return cand_e_n<3>(rhs, c);
+    case 4: return cand_e_n<4>(rhs, c);
+    case 5: return cand_e_n<5>(rhs, c);
+    case 6: return cand_e_n<6>(rhs, c);
   }
   return 1;
+}
+
+// The candidate used unless the autotuner chose one, for a launch over K
+// elements: the wave kernels as long as about all their workgroups are
+// resident at once (3 to 4 per CU of 256 in FP64, 6 to 8 in the mixed path, by
+// LDS).  Measured, us per RK4 step, wave kernels / the others: FP64 p = 4 65 /
+// 111 at 8^3 (256 workgroups), 157 / 165 at 12^3 (864), 202 / 184 at 14^3
+// (1372); p = 2 55 / 89 at 8^3, 103 / 108 at 16^3 (586), 154 / 149 at 20^3
+// (1143).  Mixed p = 4 56 / 96 at 8^3, 153 / 155 at 16^3 (2048), 387 / 357 at
+// 24^3 (6912); p = 2 50 / 78 at 8^3, 99 / 113 at 20^3 (1143), 141 / 133 at 24^3
+// (1975).
+int default_cand(int n, bool mixed, long K) {
+  const int e = cand_e(n, true, kWaveCand);
+  return (K + e - 1) / e <= (mixed ? 1800 : 900) ? kWaveCand : 0;
 }
 
 // largest change made by symmetrize (A is replaced by its symmetric part)
@@ -195,7 +216,7 @@ void launch_grad_e(ldg_handle *h, Group &g, const Tiling &t, StageIn U) {
 template <int N>
 void launch_nodal_n(ldg_handle *h, Group &g, StageIn U) {
   constexpr int E = NodalE<N>::value;
-  const LaunchArgs la = launch_args(g, g.nodal);
+  const LaunchArgs la = launch_args(g, g.tile[g.nodal]);
   const Ops<N, double> *op = (const Ops<N, double> *)g.ops;
   const dim3 grid(8 * la.per_xcd), block(NT);
   if (h->mixed && U.fluct)
@@ -235,16 +256,50 @@ void launch_rhs_e(ldg_handle *h, Group &g, const Tiling &t, StageIn U, const Sta
 }
 
 template <int N>
+void launch_grad_wave(ldg_handle *h, Group &g, StageIn U) {
+  const LaunchArgs la = launch_args(g, g.tile[g.grad[kWaveCand]]);
+  const unsigned char *img = (const unsigned char *)g.sops;
+  const dim3 grid(8 * la.per_xcd), block(WAVE_NTH);
+  if (h->mixed && U.fluct)
+    hipLaunchKernelGGL((ldg_grad_wave_kernel<N, float, float>), grid, block, 0, h->stream, (const float *)U.p,
+                       (float *)g.ff, la, img);
+  else if (h->mixed)
+    hipLaunchKernelGGL((ldg_grad_wave_kernel<N, float, double>), grid, block, 0, h->stream, (const double *)U.p,
+                       (float *)g.ff, la, img);
+  else
+    hipLaunchKernelGGL((ldg_grad_wave_kernel<N, double, double>), grid, block, 0, h->stream, (const double *)U.p,
+                       (double *)g.ff, la, img);
+}
+
+template <int N>
+void launch_rhs_wave(ldg_handle *h, Group &g, StageIn U, const StageArgs &st) {
+  const LaunchArgs la = launch_args(g, g.tile[g.rhs[kWaveCand]]);
+  const unsigned char *img = (const unsigned char *)g.sops;
+  const dim3 grid(8 * la.per_xcd), block(WAVE_NTH);
+  if (h->mixed && U.fluct)
+    hipLaunchKernelGGL((ldg_rhs_wave_kernel<N, float, float>), grid, block, 0, h->stream, (const float *)U.p,
+                       (const float *)g.ff, la, img, st);
+  else if (h->mixed)
+    hipLaunchKernelGGL((ldg_rhs_wave_kernel<N, float, double>), grid, block, 0, h->stream, (const double *)U.p,
+                       (const float *)g.ff, la, img, st);
+  else
+    hipLaunchKernelGGL((ldg_rhs_wave_kernel<N, double, double>), grid, block, 0, h->stream, (const double *)U.p,
+                       (const double *)g.ff, la, img, st);
+}
+
+template <int N>
 void launch_grad_n(ldg_handle *h, Group &g, int c, StageIn U, bool wq) {
-  if (c == 0) launch_grad_e<N, Cand<N>::grad[0]>(h, g, g.grad[0], U);
-  else launch_grad_e<N, Cand<N>::grad[1]>(h, g, g.grad[1], U);
+  if (c == 0) launch_grad_e<N, Cand<N>::grad[0]>(h, g, g.tile[g.grad[0]], U);
+  else if (c == 1) launch_grad_e<N, Cand<N>::grad[1]>(h, g, g.tile[g.grad[1]], U);
+  else launch_grad_wave<N>(h, g, U);
   if (wq) launch_nodal_n<N>(h, g, U);
 }
 
 template <int N>
 void launch_rhs_n(ldg_handle *h, Group &g, int c, StageIn U, const StageArgs &st) {
-  if (c == 0) launch_rhs_e<N, Cand<N>::rhs[0]>(h, g, g.rhs[0], U, st);
-  else launch_rhs_e<N, Cand<N>::rhs[1]>(h, g, g.rhs[1], U, st);
+  if (c == 0) launch_rhs_e<N, Cand<N>::rhs[0]>(h, g, g.tile[g.rhs[0]], U, st);
+  else if (c == 1) launch_rhs_e<N, Cand<N>::rhs[1]>(h, g, g.tile[g.rhs[1]], U, st);
+  else launch_rhs_wave<N>(h, g, U, st);
 }
 
 int launch_grad(ldg_handle *h, Group &g, StageIn U, int c, int wq) {
@@ -349,37 +404,50 @@ int inst_desc(const ldg_config &cfg, const Inst &in, int E, bool bricks, long el
   return LDG_OK;
 }
 
-int build_tiling(ldg_handle *h, Group &g, Tiling &t, int E, bool bricks = false) {
-  t.E = E;
-  t.h_inst.clear();
-  std::vector<int> blk;
-  long off = 0;
-  int boff = 0;
-  for (int idx : g.members) {
-    const Inst &in = h->inst[idx];
-    InstDesc d;
-    if (inst_desc(h->cfg, in, E, bricks, off, boff, d) != LDG_OK)
-      return fail(h, LDG_EINVAL, "mesh too large for the block numbering");
-    for (int b = 0; b < d.nblocks; ++b) blk.push_back(in.slot);
-    off += in.K;
-    boff += d.nblocks;
-    t.h_inst.push_back(d);
+int build_tilings(ldg_handle *h, Group &g) {
+  auto index = [&](int E, bool bricks) -> int {
+    for (size_t i = 0; i < g.tile.size(); ++i)
+      if (g.tile[i].E == E && g.tile[i].bricks == bricks) return (int)i;
+    Tiling t;
+    t.E = E;
+    t.bricks = bricks;
+    g.tile.push_back(t);
+    return (int)g.tile.size() - 1;
+  };
+  for (int c = 0; c < kMaxCand; ++c) {
+    g.rhs[c] = index(cand_e(g.n, true, c), false);
+    g.grad[c] = index(cand_e(g.n, false, c), false);
   }
-  t.nblocks = boff;
-  HIPCHECK(h, hipMalloc((void **)&t.d_inst, sizeof(InstDesc) * t.h_inst.size()));
-  HIPCHECK(h, hipMemcpy(t.d_inst, t.h_inst.data(), sizeof(InstDesc) * t.h_inst.size(), hipMemcpyHostToDevice));
-  if (g.members.size() > 1) {
-    HIPCHECK(h, hipMalloc((void **)&t.d_blk, sizeof(int) * blk.size()));
-    HIPCHECK(h, hipMemcpy(t.d_blk, blk.data(), sizeof(int) * blk.size(), hipMemcpyHostToDevice));
+  g.nodal = index(nodal_e(g.n), true);
+  const size_t ni = g.members.size();
+  std::vector<int> blk;
+  std::vector<size_t> blk0;
+  for (Tiling &t : g.tile) {
+    long off = 0;
+    int boff = 0;
+    blk0.push_back(blk.size());
+    for (int idx : g.members) {
+      const Inst &in = h->inst[idx];
+      InstDesc d;
+      if (inst_desc(h->cfg, in, t.E, t.bricks, off, boff, d) != LDG_OK)
+        return fail(h, LDG_EINVAL, "mesh too large for the block numbering");
+      if (ni > 1) blk.insert(blk.end(), d.nblocks, in.slot);
+      off += in.K;
+      boff += d.nblocks;
+      g.h_inst.push_back(d);
+    }
+    t.nblocks = boff;
+  }
+  const size_t ib = sizeof(InstDesc) * g.h_inst.size();
+  HIPCHECK(h, hipMalloc(&g.tables, ib + sizeof(int) * blk.size()));
+  HIPCHECK(h, hipMemcpy(g.tables, g.h_inst.data(), ib, hipMemcpyHostToDevice));
+  int *const dblk = reinterpret_cast<int *>(static_cast<unsigned char *>(g.tables) + ib);
+  if (ni > 1) HIPCHECK(h, hipMemcpy(dblk, blk.data(), sizeof(int) * blk.size(), hipMemcpyHostToDevice));
+  for (size_t i = 0; i < g.tile.size(); ++i) {
+    g.tile[i].d_inst = static_cast<const InstDesc *>(g.tables) + i * ni;
+    g.tile[i].d_blk = ni > 1 ? dblk + blk0[i] : nullptr;
   }
   return LDG_OK;
-}
-
-void free_tiling(Tiling &t) {
-  if (t.d_inst) (void)hipFree(t.d_inst);
-  if (t.d_blk) (void)hipFree(t.d_blk);
-  t.d_inst = nullptr;
-  t.d_blk = nullptr;
 }
 
 int validate_instance(const ldg_config &c, const ldg_instance &in) {
@@ -473,12 +541,9 @@ int create_impl(const ldg_config *cfg, const ldg_instance *insts, int n, ldg_han
       return bad(LDG_ENOMEM);
     }
     int maxblk = 0;
-    for (int c = 0; c < kMaxCand; ++c) {
-      if (build_tiling(h, g, g.rhs[c], cand_e(g.n, true, c)) || build_tiling(h, g, g.grad[c], cand_e(g.n, false, c)))
-        return bad(LDG_EDEVICE);
-      maxblk = std::max(maxblk, g.rhs[c].nblocks);
-    }
-    if (build_tiling(h, g, g.nodal, nodal_e(g.n), true)) return bad(LDG_EDEVICE);
+    if (build_tilings(h, g)) return bad(LDG_EDEVICE);
+    for (int c = 0; c < kMaxCand; ++c) maxblk = std::max(maxblk, g.tile[g.rhs[c]].nblocks);
+    g.cgrad = g.crhs = default_cand(g.n, h->mixed, g.K);
     std::vector<double> sc;
     for (int idx : g.members) sc.push_back(ke_scale(h->cfg, h->inst[idx]));
     if (hipMalloc((void **)&g.ke_part, sizeof(double) * (maxblk + 1)) != hipSuccess ||
@@ -516,11 +581,8 @@ int set_dt(ldg_handle *h, const double *dt) {
   for (size_t i = 0; i < h->inst.size(); ++i) h->dt_cur[i] = dt[i];
   HIPCHECK(h, hipStreamSynchronize(h->stream));
   for (Group &g : h->groups) {
-    Tiling *ts[2 * kMaxCand] = {&g.rhs[0], &g.rhs[1], &g.grad[0], &g.grad[1]};
-    for (Tiling *t : ts) {
-      for (size_t s = 0; s < g.members.size(); ++s) t->h_inst[s].dt = dt[g.members[s]];
-      HIPCHECK(h, hipMemcpy(t->d_inst, t->h_inst.data(), sizeof(InstDesc) * t->h_inst.size(), hipMemcpyHostToDevice));
-    }
+    for (size_t i = 0; i < g.h_inst.size(); ++i) g.h_inst[i].dt = dt[g.members[i % g.members.size()]];
+    HIPCHECK(h, hipMemcpy(g.tables, g.h_inst.data(), sizeof(InstDesc) * g.h_inst.size(), hipMemcpyHostToDevice));
   }
   return LDG_OK;
 }
@@ -581,7 +643,7 @@ int rk4_step(ldg_handle *h, bool ke, bool in32, bool out32) {
       U = StageIn{bufs[s & 1], h->mixed};
     }
     if (ke) {
-      const Tiling &t = g.rhs[g.crhs];
+      const Tiling &t = g.tile[g.rhs[g.crhs]];
       hipLaunchKernelGGL(ldg_finalize_kernel, dim3(g.members.size()), dim3(NT), 0, h->stream,
                          (const double *)g.ke_part, 1, (const InstDesc *)t.d_inst, (int)h->inst.size(),
                          (const double *)g.d_scale, h->ke_hist + first, (const int *)h->d_step);
@@ -817,8 +879,7 @@ void ldg_destroy(ldg_handle *h) {
     if (g.ff) (void)hipFree(g.ff);
     if (g.ops) (void)hipFree(g.ops);
     if (g.sops) (void)hipFree(g.sops);
-    for (int c = 0; c < kMaxCand; ++c) { free_tiling(g.rhs[c]); free_tiling(g.grad[c]); }
-    free_tiling(g.nodal);
+    if (g.tables) (void)hipFree(g.tables);
     closure_release(g);
   }
   if (h->ke_hist) (void)hipFree(h->ke_hist);
@@ -984,9 +1045,9 @@ int ldg_instance_diagnostics(ldg_handle *h, int i, double out[3]) {
     StageArgs st = empty_stage();
     st.ke_part = g.ke_part;
     st.diag_part = g.diag_part;
-    const int rc = launch_rhs(h, g, state_in(g.u), st);
+    const int rc = launch_rhs(h, g, state_in(g.u), st, 0);
     if (rc) return rc;
-    const Tiling &t = g.rhs[g.crhs];
+    const Tiling &t = g.tile[g.rhs[0]];
     hipLaunchKernelGGL(ldg_finalize_kernel, dim3(g.members.size()), dim3(NT), 0, h->stream, (const double *)g.ke_part,
                        1, (const InstDesc *)t.d_inst, ni, (const double *)g.d_scale, h->scal + first,
                        (const int *)nullptr);
@@ -1048,7 +1109,6 @@ int ldg_autotune(ldg_handle *h, int *chosen) {
       for (int c = 0; c < kMaxCand; ++c) best[c] = 1e30f;
       for (int round = 0; round < 3; ++round) {
         for (int c = 0; c < kMaxCand; ++c) {
-          if (c > 0 && cand_e(g.n, kind == 1, c) == cand_e(g.n, kind == 1, 0)) continue;
           float ms = 0.f;
           for (int rep = 0; rep < 3; ++rep) {    // first launch warms up, not timed
             if (rep == 1) HIPCHECK(h, hipEventRecord(e0, h->stream));
@@ -1145,10 +1205,29 @@ static __device__ __align__(256) unsigned char scratch[LDG_NOALLOC_SCRATCH_BYTES
 
 namespace ldg_host {
 
-constexpr size_t kScrImg = 0, kScrInstGrad = 5120, kScrInstRhs = 6656, kScrFF = 8192;
-static_assert(GImage<6>::BYTES <= kScrInstGrad, "the operator image does not fit its scratch slot");
-static_assert(sizeof(InstDesc) <= kScrInstRhs - kScrInstGrad && sizeof(InstDesc) <= kScrFF - kScrInstRhs,
+constexpr size_t kScrInstGrad = 0, kScrInstRhs = 1536, kScrImg = 3072, kScrFF = 8192;
+static_assert(sizeof(InstDesc) <= kScrInstRhs - kScrInstGrad && sizeof(InstDesc) <= kScrImg - kScrInstRhs,
               "an instance table does not fit its scratch slot");
+static_assert(kScrImg + GImage<6>::BYTES <= kScrFF, "the operator image does not fit its scratch slot");
+
+// The call's operators (FP64-only part and those of the precision in use) and
+// instance tables reach the scratch array as the arguments of one small
+// kernel: three copies from pageable host memory in their place took about
+// 15 us of a 57 us call (12^3, p = 4).
+struct SetupArgs {
+  static constexpr int WORDS = (int)(2 * sizeof(InstDesc) + sizeof(GOpsD<6>) + sizeof(GOps<6, double>)) / 4;
+  int end[4], at[4];          // section i: words [end[i-1], end[i]) go to word at[i] of the scratch array
+  unsigned w[WORDS];
+};
+static_assert(sizeof(SetupArgs) <= 3968, "kernel arguments are limited to 4 KB");
+__global__ void __launch_bounds__(256) ldg_setup_kernel(SetupArgs a, unsigned *__restrict__ dst) {
+  for (int i = threadIdx.x; i < a.end[3]; i += 256) {
+    const int sec = i < a.end[0] ? 0 : i < a.end[1] ? 1 : i < a.end[2] ? 2 : 3;
+    const int first = sec == 0 ? 0 : sec == 1 ? a.end[0] : sec == 2 ? a.end[1] : a.end[2];
+    const int at = sec == 0 ? a.at[0] : sec == 1 ? a.at[1] : sec == 2 ? a.at[2] : a.at[3];
+    dst[at + i - first] = a.w[i];
+  }
+}
 
 constexpr int kMaxDevices = 64;
 std::mutex g_scratch_mu;
@@ -1205,39 +1284,59 @@ template <> const Ops<4, double> &ops_of<4>(const OpsTables &t) { return t.o4; }
 template <> const Ops<5, double> &ops_of<5>(const OpsTables &t) { return t.o5; }
 template <> const Ops<6, double> &ops_of<6>(const OpsTables &t) { return t.o6; }
 
-// The gradient and right-hand-side kernels of ldg_rhs (default tilings, FP64
-// input) with every intermediate in scr.  The host copies of the operators
-// and instance tables are read by the copies before the stream is
-// synchronised (the caller synchronises before returning).
+// The gradient and right-hand-side kernels of ldg_rhs (default candidate, FP64
+// input) with every intermediate in scr.
 template <int N>
 hipError_t noalloc_launch(const ldg_config &cfg, const Inst &in, unsigned char *scr, const double *u, double *k,
-                          hipStream_t s, InstDesc dsc[2], unsigned char *img) {
-  constexpr int EG = Cand<N>::grad[0], ER = Cand<N>::rhs[0];
-  const Ops<N, double> &o = ops_of<N>(ops_tables());
-  if (inst_desc(cfg, in, EG, false, 0, 0, dsc[0]) != LDG_OK || inst_desc(cfg, in, ER, false, 0, 0, dsc[1]) != LDG_OK)
+                          hipStream_t s) {
+  const bool mixed = cfg.precision == LDG_MIXED;
+  const bool wave = default_cand(N, mixed, in.K) == kWaveCand;
+  constexpr int EG = Cand<N>::grad[0], ER = Cand<N>::rhs[0], EW = WaveE<N>::value;
+  InstDesc dsc[2];
+  if (inst_desc(cfg, in, wave ? EW : EG, false, 0, 0, dsc[0]) != LDG_OK ||
+      inst_desc(cfg, in, wave ? EW : ER, false, 0, 0, dsc[1]) != LDG_OK)
     return hipErrorInvalidValue;
   const double a[3] = {dsc[1].ialpha[0], dsc[1].ialpha[1], dsc[1].ialpha[2]};
-  fill_image<N>(img, o, a);
-  hipError_t e = hipMemcpyAsync(scr + kScrImg, img, GImage<N>::BYTES, hipMemcpyHostToDevice, s);
-  if (e == hipSuccess) e = hipMemcpyAsync(scr + kScrInstGrad, &dsc[0], sizeof(InstDesc), hipMemcpyHostToDevice, s);
-  if (e == hipSuccess) e = hipMemcpyAsync(scr + kScrInstRhs, &dsc[1], sizeof(InstDesc), hipMemcpyHostToDevice, s);
-  if (e != hipSuccess) return e;
+  alignas(16) unsigned char img[GImage<N>::BYTES];
+  fill_image<N>(img, ops_of<N>(ops_tables()), a);
+  SetupArgs sa;
+  int words = 0;
+  auto section = [&](int i, size_t at, const void *src, size_t bytes) {
+    std::memcpy(sa.w + words, src, bytes);
+    words += (int)(bytes / 4);
+    sa.end[i] = words;
+    sa.at[i] = (int)(at / 4);
+  };
+  const size_t off = mixed ? GImage<N>::OF : GImage<N>::OD;
+  section(0, kScrInstGrad, &dsc[0], sizeof(InstDesc));
+  section(1, kScrInstRhs, &dsc[1], sizeof(InstDesc));
+  section(2, kScrImg, img, sizeof(GOpsD<N>));
+  section(3, kScrImg + off, img + off, mixed ? sizeof(GOps<N, float>) : sizeof(GOps<N, double>));
+  hipLaunchKernelGGL(ldg_setup_kernel, dim3(1), dim3(256), 0, s, sa, reinterpret_cast<unsigned *>(scr));
   const LaunchArgs lg{reinterpret_cast<const InstDesc *>(scr + kScrInstGrad), nullptr, dsc[0].nblocks,
                       (dsc[0].nblocks + 7) / 8, in.K};
   const LaunchArgs lr{reinterpret_cast<const InstDesc *>(scr + kScrInstRhs), nullptr, dsc[1].nblocks,
                       (dsc[1].nblocks + 7) / 8, in.K};
-  const dim3 gg(8 * lg.per_xcd), gr(8 * lr.per_xcd), bg(Shape<N, EG>::NTH), br(Shape<N, ER>::NTH);
+  const dim3 gg(8 * lg.per_xcd), gr(8 * lr.per_xcd), bg(Shape<N, EG>::NTH), br(Shape<N, ER>::NTH), bw(WAVE_NTH);
   const unsigned char *simg = scr + kScrImg;
   StageArgs st = empty_stage();
   st.kout = k;
-  if (cfg.precision == LDG_MIXED) {
-    float *ff = reinterpret_cast<float *>(scr + kScrFF);
-    hipLaunchKernelGGL((ldg_grad_kernel<N, EG, float, double>), gg, bg, 0, s, u, ff, lg, simg);
-    hipLaunchKernelGGL((ldg_rhs_kernel<N, ER, float, double, false>), gr, br, 0, s, u, (const float *)ff, lr, simg, st);
+  float *const ff32 = reinterpret_cast<float *>(scr + kScrFF);
+  double *const ff64 = reinterpret_cast<double *>(scr + kScrFF);
+  if (mixed && wave) {
+    hipLaunchKernelGGL((ldg_grad_wave_kernel<N, float, double>), gg, bw, 0, s, u, ff32, lg, simg);
+    hipLaunchKernelGGL((ldg_rhs_wave_kernel<N, float, double>), gr, bw, 0, s, u, (const float *)ff32, lr, simg, st);
+  } else if (mixed) {
+    hipLaunchKernelGGL((ldg_grad_kernel<N, EG, float, double>), gg, bg, 0, s, u, ff32, lg, simg);
+    hipLaunchKernelGGL((ldg_rhs_kernel<N, ER, float, double, false>), gr, br, 0, s, u, (const float *)ff32, lr, simg,
+                       st);
+  } else if (wave) {
+    hipLaunchKernelGGL((ldg_grad_wave_kernel<N, double, double>), gg, bw, 0, s, u, ff64, lg, simg);
+    hipLaunchKernelGGL((ldg_rhs_wave_kernel<N, double, double>), gr, bw, 0, s, u, (const double *)ff64, lr, simg, st);
   } else {
-    double *ff = reinterpret_cast<double *>(scr + kScrFF);
-    hipLaunchKernelGGL((ldg_grad_kernel<N, EG, double, double>), gg, bg, 0, s, u, ff, lg, simg);
-    hipLaunchKernelGGL((ldg_rhs_kernel<N, ER, double, double, false>), gr, br, 0, s, u, (const double *)ff, lr, simg, st);
+    hipLaunchKernelGGL((ldg_grad_kernel<N, EG, double, double>), gg, bg, 0, s, u, ff64, lg, simg);
+    hipLaunchKernelGGL((ldg_rhs_kernel<N, ER, double, double, false>), gr, br, 0, s, u, (const double *)ff64, lr, simg,
+                       st);
   }
   return hipGetLastError();
 }
@@ -1283,15 +1382,13 @@ extern "C" int ldg_rhs_noalloc(const ldg_config *cfg, const double *u, double *k
   unsigned char *scr = scratch_on(dev);
   if (!scr) return LDG_EDEVICE;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  InstDesc dsc[2];
-  alignas(16) unsigned char img[GImage<6>::BYTES];   // (read by the copies until the synchronisation below)
   hipError_t e = hipErrorInvalidValue;
   switch (n) {
-    case 2: e = noalloc_launch<2>(*cfg, in, scr, u, k, s, dsc, img); break;
-    case 3: e = noalloc_launch<3>(*cfg, in, scr, u, k, s, dsc, img); break;
-    case 4: e = noalloc_launch<4>(*cfg, in, scr, u, k, s, dsc, img); break;
-    case 5: e = noalloc_launch<5>(*cfg, in, scr, u, k, s, dsc, img); break;
-    case 6: e = noalloc_launch<6>(*cfg, in, scr, u, k, s, dsc, img); break;
+    case 2: e = noalloc_launch<2>(*cfg, in, scr, u, k, s); break;
+    case 3: e = noalloc_launch<3>(*cfg, in, scr, u, k, s); break;
+    case 4: e = noalloc_launch<4>(*cfg, in, scr, u, k, s); break;
+    case 5: e = noalloc_launch<5>(*cfg, in, scr, u, k, s); break;
+    case 6: e = noalloc_launch<6>(*cfg, in, scr, u, k, s); break;
   }
   const hipError_t es = hipStreamSynchronize(s);
   if (e == hipSuccess) e = es;

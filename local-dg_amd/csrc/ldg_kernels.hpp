@@ -351,6 +351,13 @@ __device__ inline float rcp(float x) { return __builtin_amdgcn_rcpf(x); }
 __device__ inline double sqrt_(double x) { return sqrt(x); }
 __device__ inline float sqrt_(float x) { return __builtin_amdgcn_sqrtf(x); }
 
+// The pointwise physics says itself where a multiply-add is fused, and the
+// compiler fuses nothing else there (fp contract(off)): which product of a
+// sum it picks depends on the code around, and the kernels of this file and
+// of wave_kernels.hpp are to agree bit by bit.
+__device__ inline double fma_(double a, double b, double c) { return __builtin_fma(a, b, c); }
+__device__ inline float fma_(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+
 template <typename T>
 struct Bg {
   T rho0, E0, H0, gm1, mu, kappa;
@@ -363,14 +370,22 @@ struct Bg {
 // gradients g[s + 5 l].
 template <typename T>
 __device__ inline void prim_grads(T ir, T E, const T v[3], const T *g, T gv[3][3], T ge[3]) {
+#pragma clang fp contract(off)
 #pragma unroll
   for (int l = 0; l < 3; ++l) {
     const T drho = g[5 * l];
 #pragma unroll
-    for (int i = 0; i < 3; ++i) gv[i][l] = (g[1 + i + 5 * l] - v[i] * drho) * ir;
-    const T dEr = (g[4 + 5 * l] - E * ir * drho) * ir;
-    ge[l] = dEr - (v[0] * gv[0][l] + v[1] * gv[1][l] + v[2] * gv[2][l]);
+    for (int i = 0; i < 3; ++i) gv[i][l] = fma_(-v[i], drho, g[1 + i + 5 * l]) * ir;
+    const T dEr = fma_(-(E * ir), drho, g[4 + 5 * l]) * ir;
+    ge[l] = dEr - fma_(v[2], gv[2][l], fma_(v[1], gv[1][l], v[0] * gv[0][l]));
   }
+}
+
+// p - p0 of the fluctuation w with velocity v
+template <typename T>
+__device__ inline T pressure(const T w[5], const T v[3], const Bg<T> &b) {
+#pragma clang fp contract(off)
+  return b.gm1 * fma_(T(-0.5), fma_(w[3], v[2], fma_(w[2], v[1], w[1] * v[0])), w[4]);
 }
 
 // Volume flux F[s + 5 l] = Fc_l(u) - Fv_l(u, g) (fluxC minus fluxV,
@@ -379,23 +394,27 @@ __device__ inline void prim_grads(T ir, T E, const T v[3], const T *g, T gv[3][3
 // rules integrate d(phi)/dx and the face traces of phi exactly).
 template <typename T>
 __device__ inline void volume_flux(const T w[5], const T *g, const Bg<T> &b, T F[15]) {
+#pragma clang fp contract(off)
   const T rho = b.rho0 + w[0];
   const T ir = rcp(rho);
   const T v[3] = {w[1] * ir, w[2] * ir, w[3] * ir};
-  const T pf = b.gm1 * (w[4] - T(0.5) * (w[1] * v[0] + w[2] * v[1] + w[3] * v[2]));
+  const T pf = pressure(w, v, b);
   const T hv = b.H0 + w[4] + pf;   // E + p
-  T gv[3][3], ge[3];
+  T gv[3][3], ge[3], tau[3][3];
   prim_grads<T>(ir, b.E0 + w[4], v, g, gv, ge);
-  const T div = gv[0][0] + gv[1][1] + gv[2][2];
+  const T m23 = (b.mu * T(2.0 / 3.0)) * (gv[0][0] + gv[1][1] + gv[2][2]);
+#pragma unroll
+  for (int l = 0; l < 3; ++l)
+#pragma unroll
+    for (int i = 0; i <= l; ++i)
+      tau[i][l] = tau[l][i] = i == l ? fma_(b.mu, gv[i][l] + gv[l][i], -m23) : b.mu * (gv[i][l] + gv[l][i]);
 #pragma unroll
   for (int l = 0; l < 3; ++l) {
-    T tau[3];
-#pragma unroll
-    for (int i = 0; i < 3; ++i) tau[i] = b.mu * (gv[i][l] + gv[l][i]) - (i == l ? b.mu * T(2.0 / 3.0) * div : T(0));
     F[5 * l] = w[1 + l];
 #pragma unroll
-    for (int i = 0; i < 3; ++i) F[1 + i + 5 * l] = w[1 + i] * v[l] + (i == l ? pf : T(0)) - tau[i];
-    F[4 + 5 * l] = hv * v[l] - (v[0] * tau[0] + v[1] * tau[1] + v[2] * tau[2] + b.kappa * ge[l]);
+    for (int i = 0; i < 3; ++i) F[1 + i + 5 * l] = fma_(w[1 + i], v[l], i == l ? pf - tau[i][l] : -tau[i][l]);
+    F[4 + 5 * l] =
+        fma_(hv, v[l], -fma_(b.kappa, ge[l], fma_(v[2], tau[2][l], fma_(v[1], tau[1][l], v[0] * tau[0][l]))));
   }
 }
 
@@ -415,26 +434,25 @@ __device__ inline void volume_flux(const T w[5], const T *g, const Bg<T> &b, T F
 // each side's own trace, as the reference does.
 template <typename T, int D>
 __device__ inline void visc_face(const T w[5], T ir, const T v[3], const T *q, const Bg<T> &b, T fv[4]) {
+#pragma clang fp contract(off)
   T gv[3][3], ge[3];
   prim_grads<T>(ir, b.E0 + w[4], v, q, gv, ge);
-  const T div = gv[0][0] + gv[1][1] + gv[2][2];
-  T tau[3];
+  const T m23 = (b.mu * T(2.0 / 3.0)) * (gv[0][0] + gv[1][1] + gv[2][2]);
 #pragma unroll
-  for (int i = 0; i < 3; ++i) tau[i] = b.mu * (gv[i][D] + gv[D][i]) - (i == D ? b.mu * T(2.0 / 3.0) * div : T(0));
-#pragma unroll
-  for (int i = 0; i < 3; ++i) fv[i] = tau[i];
-  fv[3] = v[0] * tau[0] + v[1] * tau[1] + v[2] * tau[2] + b.kappa * ge[D];
+  for (int i = 0; i < 3; ++i)
+    fv[i] = i == D ? fma_(b.mu, gv[i][D] + gv[D][i], -m23) : b.mu * (gv[i][D] + gv[D][i]);
+  fv[3] = fma_(b.kappa, ge[D], fma_(v[2], fv[2], fma_(v[1], fv[1], v[0] * fv[0])));
 }
 
 template <typename T, int D>
 __device__ inline void face_flux_pair(const T wK[5], const T wN[5], const T *q, const Bg<T> &b, T outK[5],
                                       T outN[5]) {
+#pragma clang fp contract(off)
   const T rN = b.rho0 + wN[0], rK = b.rho0 + wK[0];
   const T irN = rcp(rN), irK = rcp(rK);
   const T vN[3] = {wN[1] * irN, wN[2] * irN, wN[3] * irN};
   const T vK[3] = {wK[1] * irK, wK[2] * irK, wK[3] * irK};
-  const T pN = b.gm1 * (wN[4] - T(0.5) * (wN[1] * vN[0] + wN[2] * vN[1] + wN[3] * vN[2]));   // p - p0
-  const T pK = b.gm1 * (wK[4] - T(0.5) * (wK[1] * vK[0] + wK[2] * vK[1] + wK[3] * vK[2]));
+  const T pN = pressure(wN, vN, b), pK = pressure(wK, vK, b);                               // p - p0
   const T hN = b.H0 + wN[4] + pN, hK = b.H0 + wK[4] + pK;                                   // E + p
   const T HN = hN * irN, HK = hK * irK;
   const T qN = vN[D], qK = vK[D];
@@ -442,30 +460,31 @@ __device__ inline void face_flux_pair(const T wK[5], const T wN[5], const T *q, 
   const T iden = rcp(s + T(1));
   T vt[3];
 #pragma unroll
-  for (int i = 0; i < 3; ++i) vt[i] = (s * vN[i] + vK[i]) * iden;
-  const T ht = (s * HN + HK) * iden;
-  const T q2 = vt[0] * vt[0] + vt[1] * vt[1] + vt[2] * vt[2];
+  for (int i = 0; i < 3; ++i) vt[i] = fma_(s, vN[i], vK[i]) * iden;
+  const T ht = fma_(s, HN, HK) * iden;
+  const T q2 = fma_(vt[2], vt[2], fma_(vt[1], vt[1], vt[0] * vt[0]));
   const T qt = vt[D];
-  const T c2 = b.gm1 * (ht - T(0.5) * q2);
+  const T c2 = b.gm1 * fma_(T(-0.5), q2, ht);
   const T c = sqrt_(c2), ic = rcp(c);
   const T l0 = fabs(qt), lp = fabs(qt + c), lm = fabs(qt - c);
   T dd[5];
 #pragma unroll
   for (int k = 0; k < 5; ++k) dd[k] = wN[k] - wK[k];
-  const T dp = b.gm1 * (T(0.5) * q2 * dd[0] - (vt[0] * dd[1] + vt[1] * dd[2] + vt[2] * dd[3]) + dd[4]);
-  const T dV = dd[1 + D] - qt * dd[0];
-  const T s1 = T(0.5) * (lp + lm) - l0, s2 = T(0.5) * (lp - lm);
-  const T A = s1 * dp * ic * ic + s2 * dV * ic;
-  const T B = s2 * dp * ic + s1 * dV;
+  const T dp = b.gm1 * (fma_(T(0.5) * q2, dd[0], -fma_(vt[2], dd[3], fma_(vt[1], dd[2], vt[0] * dd[1]))) + dd[4]);
+  const T dV = fma_(-qt, dd[0], dd[1 + D]);
+  const T s1 = fma_(T(0.5), lp + lm, -l0), s2 = T(0.5) * (lp - lm);
+  const T dpi = dp * ic;
+  const T A = fma_(s1, dpi, s2 * dV) * ic;
+  const T B = fma_(s2, dpi, s1 * dV);
+  // R = (F(N) + F(K) - |A| (uN - uK)) / 2 along D
   T R[5];
-  R[0] = T(0.5) * (rN * qN + rK * qK) - T(0.5) * (l0 * dd[0] + A);
+  R[0] = T(0.5) * (fma_(rN, qN, rK * qK) - fma_(l0, dd[0], A));
 #pragma unroll
   for (int i = 0; i < 3; ++i) {
-    const T pn = (i == D) ? (pN + pK) : T(0);
-    const T bn = (i == D) ? B : T(0);
-    R[1 + i] = T(0.5) * (wN[1 + i] * qN + wK[1 + i] * qK + pn) - T(0.5) * (l0 * dd[1 + i] + A * vt[i] + bn);
+    const T x = fma_(wN[1 + i], qN, wK[1 + i] * qK), y = fma_(l0, dd[1 + i], A * vt[i]);
+    R[1 + i] = T(0.5) * (i == D ? (x + (pN + pK)) - (y + B) : x - y);
   }
-  R[4] = T(0.5) * (hN * qN + hK * qK) - T(0.5) * (l0 * dd[4] + A * ht + B * qt);
+  R[4] = T(0.5) * (fma_(hN, qN, hK * qK) - fma_(l0, dd[4], fma_(A, ht, B * qt)));
   T fK[4], fN[4];
   visc_face<T, D>(wK, irK, vK, q, b, fK);
   visc_face<T, D>(wN, irN, vN, q, b, fN);
@@ -777,7 +796,7 @@ ldg_grad_kernel(const UT *__restrict__ U, T *__restrict__ FF, LaunchArgs la, con
         own[D][s] = us[0];
         T q = nw * nbr[D][s];
 #pragma unroll
-        for (int j = 0; j < N; ++j) q += nrm.r[j] * us[j * ST[D]];
+        for (int j = 0; j < N; ++j) q = fma_(nrm.r[j], us[j * ST[D]], q);
         qn[D][s] = q;
       }
     }
@@ -839,7 +858,7 @@ ldg_grad_kernel(const UT *__restrict__ U, T *__restrict__ FF, LaunchArgs la, con
             sym_apply<N, -1, T>(Dm, x, o);
             T *fd = wk + (15 + f) * FS + N * x0;
 #pragma unroll
-            for (int j = 0; j < N; ++j) fd[j] = al * (o[j] + eta.r[j] * jmp);
+            for (int j = 0; j < N; ++j) fd[j] = al * fma_(eta.r[j], jmp, o[j]);
           }
           const T *g = nb + (NSTATE * D + s) * FS + N * x0;
 #pragma unroll
@@ -892,7 +911,7 @@ ldg_grad_kernel(const UT *__restrict__ U, T *__restrict__ FF, LaunchArgs la, con
             sym_apply<N, -1, T>(Dm, x, o);
             T *fd = wk + (18 + fb) * FS + at;
 #pragma unroll
-            for (int j = 0; j < N; ++j) fd[N * j] = be * (o[j] + eta.r[j] * jmp);
+            for (int j = 0; j < N; ++j) fd[N * j] = be * fma_(eta.r[j], jmp, o[j]);
           }
         }
       }
@@ -1208,7 +1227,7 @@ ldg_rhs_kernel(const UT *__restrict__ U, const T *__restrict__ FF, LaunchArgs la
           for (int q = 0; q < N; ++q) x[q] = p[q];
           sym_apply<N, -1, T>(Dx, x, qx[s]);
 #pragma unroll
-          for (int q = 0; q < N; ++q) qx[s][q] += ax.r[q] * jx[s];
+          for (int q = 0; q < N; ++q) qx[s][q] = fma_(ax.r[q], jx[s], qx[s][q]);
         }
       }
       {
@@ -1223,7 +1242,7 @@ ldg_rhs_kernel(const UT *__restrict__ U, const T *__restrict__ FF, LaunchArgs la
           sym_apply<N, -1, T>(Dy, x, qy[s]);
 #pragma unroll
           for (int q = 0; q < N; ++q) {
-            qy[s][q] += ay.r[q] * jy[s];
+            qy[s][q] = fma_(ay.r[q], jy[s], qy[s][q]);
             if (!L::JB) sB[by + s * NN + N * q] = qy[s][q];
           }
         }
@@ -1251,7 +1270,7 @@ ldg_rhs_kernel(const UT *__restrict__ U, const T *__restrict__ FF, LaunchArgs la
       for (int s = 0; s < NSTATE; ++s) {
         sym_apply<N, -1, T>(Dz, ug[s], kz[s]);
 #pragma unroll
-        for (int q = 0; q < N; ++q) kz[s][q] += az.r[q] * jz[s];
+        for (int q = 0; q < N; ++q) kz[s][q] = fma_(az.r[q], jz[s], kz[s][q]);
       }
     }
     const Bg<T> bg(d.ph);
@@ -1298,7 +1317,7 @@ ldg_rhs_kernel(const UT *__restrict__ U, const T *__restrict__ FF, LaunchArgs la
       T o[N];
       sym_apply<N, -1, T>(Dz, kz[s], o);
 #pragma unroll
-      for (int q = 0; q < N; ++q) kz[s][q] = o[q] - (eta.r[q] * fz[0][s] + eta.r[N - 1 - q] * fz[1][s]);
+      for (int q = 0; q < N; ++q) kz[s][q] = o[q] - fma_(eta.r[q], fz[0][s], eta.r[N - 1 - q] * fz[1][s]);
     }
   }
   if constexpr (DIAG) {
@@ -1326,7 +1345,8 @@ ldg_rhs_kernel(const UT *__restrict__ U, const T *__restrict__ FF, LaunchArgs la
         sym_apply<N, -1, T>(Dh, x, o);
 #pragma unroll
         for (int q = 0; q < N; ++q)
-          p[l == 0 ? q : N * q] = o[q] - (eta.r[q] * (l == 0 ? fx : fy)[0][s] + eta.r[N - 1 - q] * (l == 0 ? fx : fy)[1][s]);
+          p[l == 0 ? q : N * q] =
+              o[q] - fma_(eta.r[q], (l == 0 ? fx : fy)[0][s], eta.r[N - 1 - q] * (l == 0 ? fx : fy)[1][s]);
       }
     }
   }
@@ -1486,7 +1506,7 @@ ldg_rhs_kernel(const UT *__restrict__ U, const T *__restrict__ FF, LaunchArgs la
       for (int q = 0; q < N; ++q) {
         const double *x = md + bz + NF * q;
         const double rho = x[0], m1 = x[NN], m2 = x[2 * NN], m3 = x[3 * NN];
-        kel += opd->w[a] * opd->w[b] * opd->w[q] * (m1 * m1 + m2 * m2 + m3 * m3) / (2.0 * rho);
+        kel += opd->w[a] * opd->w[b] * opd->w[q] * fma_(m3, m3, fma_(m2, m2, m1 * m1)) / (2.0 * rho);
       }
     }
     const double x = group_sum<NTH>(kel, sred);
