@@ -22,6 +22,7 @@
 #include <vector>
 
 #include "closure_kernels.hpp"
+#include "closure_train.hpp"
 #include "handle.hpp"
 
 using namespace ldg_host;
@@ -47,6 +48,15 @@ struct ldg_closure {
         *dY = nullptr, *dH = nullptr, *dZ = nullptr, *Wbat = nullptr;
   long *idx = nullptr;
   double *part = nullptr;
+  // fused training (closure_train.hpp): operands and transposed weights for
+  // batches of up to tB rows, sample indices and loss sums, each grown when a
+  // call needs more
+  unsigned short *tws = nullptr;
+  int tB = 0;
+  long *tidx = nullptr;
+  long tidx_cap = 0;
+  double *tpart = nullptr;
+  long tpart_cap = 0;
   hipStream_t stream = nullptr;
   std::string err;
 };
@@ -178,6 +188,108 @@ int pack_bf16(ldg_closure *c) {
 
 bool fused_ok(const ldg_closure *c) { return c->n == 3 && c->hidden == 256; }
 
+// *p holds at least `need` values after the call (contents are not kept).
+template <typename T>
+int grow(ldg_closure *c, T **p, long *cap, long need) {
+  if (need <= *cap) return LDG_OK;
+  if (*p) (void)hipFree(*p);
+  *p = nullptr;
+  *cap = 0;
+  if (hipMalloc((void **)p, (size_t)need * sizeof(T)) != hipSuccess)
+    return cfail(c, LDG_ENOMEM, "device allocation failed (training workspace)");
+  *cap = need;
+  return LDG_OK;
+}
+
+// Epochs of ldg_closure_train by the two kernels of closure_train.hpp: no
+// device synchronisation inside an epoch, the loss sums of its batches are
+// read at its end.
+int train_fused(ldg_closure *c, int epochs, int batch, double lr, const std::vector<long> &all, long ntrain,
+                std::mt19937_64 &rng, double *losses) {
+  const long nval = (long)all.size() - ntrain;
+  const int ldb = (batch + TPAD - 1) / TPAD * TPAD, nblk = ldb / TROWS;
+  const long nbatch = ntrain / batch, nvb = (nval + batch - 1) / batch;
+  const size_t bf = (size_t)(op_size(TIN, ldb) + 4 * op_size(THID, ldb) + op_size(TOUT, ldb));
+  const size_t fl = (size_t)(bias_size(TOUT, ldb) + 2 * bias_size(THID, ldb));
+  const size_t wt = (size_t)THID * (THID + TOUTP);
+  if (ldb > c->tB) {
+    if (c->tws) (void)hipFree(c->tws);
+    c->tws = nullptr;
+    c->tB = 0;
+    if (hipMalloc((void **)&c->tws, 2 * (wt + bf) + 4 * fl) != hipSuccess)
+      return cfail(c, LDG_ENOMEM, "device allocation failed (training workspace)");
+    c->tB = ldb;
+  }
+  int rc = grow(c, &c->tidx, &c->tidx_cap, ntrain + nval);
+  if (!rc) rc = grow(c, &c->tpart, &c->tpart_cap, (nbatch + nvb) * nblk);
+  if (rc) return rc;
+  const Offs o = offsets(c);
+  static_assert(TINP % 16 == 0 && TOUTP % 16 == 0 && THID % 32 == 0, "whole matrix steps");
+  TrainWeights W;
+  W.W1 = c->Wb;
+  W.W2 = W.W1 + (long)c->hidden * c->k1p;
+  W.W3 = W.W2 + (long)c->hidden * c->hidden;
+  W.W2T = c->tws;
+  W.W3T = W.W2T + (long)THID * THID;
+  TrainOperands t;
+  t.X = c->tws + wt;
+  t.H1 = t.X + op_size(TIN, ldb);
+  t.H2 = t.H1 + op_size(THID, ldb);
+  t.dZ2 = t.H2 + op_size(THID, ldb);
+  t.dZ1 = t.dZ2 + op_size(THID, ldb);
+  t.dY = t.dZ1 + op_size(THID, ldb);
+  t.fY = reinterpret_cast<float *>(t.dY + op_size(TOUT, ldb));
+  t.fZ2 = t.fY + bias_size(TOUT, ldb);
+  t.fZ1 = t.fZ2 + bias_size(THID, ldb);
+  const float *wd = c->normalized ? c->Wd : nullptr;     // per-sample weights (set with the normalisation)
+  const float *b1 = c->params + o.b1, *b2 = c->params + o.b2, *b3 = c->params + o.b3;
+  hipStream_t s = c->stream;
+  hipLaunchKernelGGL(mlp_pack_transposed, dim3(100), dim3(256), 0, s, W);
+  std::vector<long> perm(all.begin(), all.begin() + ntrain);
+  if (nval) CCHECK(c, hipMemcpyAsync(c->tidx + ntrain, all.data() + ntrain, nval * sizeof(long), hipMemcpyHostToDevice, s));
+  std::vector<double> part((nbatch + nvb) * nblk);
+  AdamArgs ad;
+  ad.p = c->params; ad.m = c->m; ad.v = c->v;
+  ad.lr = (float)lr; ad.b1 = 0.9f; ad.b2 = 0.999f; ad.eps = 1e-8f;
+  const float scale = 2.0f / (float)((long)batch * c->nout);
+  for (int ep = 0; ep < epochs; ++ep) {
+    std::shuffle(perm.begin(), perm.end(), rng);
+    CCHECK(c, hipMemcpyAsync(c->tidx, perm.data(), ntrain * sizeof(long), hipMemcpyHostToDevice, s));
+    for (long b = 0; b < nbatch; ++b) {
+      hipLaunchKernelGGL((mlp_train_rows<true>), dim3(nblk), dim3(512), 0, s, (const float *)c->Xd,
+                         (const float *)c->Td, wd, (const long *)(c->tidx + b * batch), batch, ldb, W, b1, b2, b3,
+                         scale, t, c->tpart + b * nblk);
+      ++c->adam_t;
+      ad.bc1 = 1.0f - (float)std::pow(ad.b1, (double)c->adam_t);
+      ad.bc2 = 1.0f - (float)std::pow(ad.b2, (double)c->adam_t);
+      hipLaunchKernelGGL(mlp_train_weights, dim3(TRAIN_TILES / 4 + TRAIN_BIAS_BLOCKS), dim3(256), 0, s,
+                         t, ldb, W, ad);
+    }
+    for (long v = 0; v < nvb; ++v) {
+      const int rows = (int)std::min<long>(batch, nval - v * batch);
+      hipLaunchKernelGGL((mlp_train_rows<false>), dim3((rows + TROWS - 1) / TROWS), dim3(512), 0, s,
+                         (const float *)c->Xd, (const float *)c->Td, wd, (const long *)(c->tidx + ntrain + v * batch),
+                         rows, ldb, W, b1, b2, b3, 0.0f, t, c->tpart + (nbatch + v) * nblk);
+    }
+    CCHECK(c, hipGetLastError());
+    CCHECK(c, hipMemcpyAsync(part.data(), c->tpart, part.size() * sizeof(double), hipMemcpyDeviceToHost, s));
+    CCHECK(c, hipStreamSynchronize(s));
+    double tl = 0.0, vl = 0.0;
+    for (long b = 0; b < nbatch; ++b)
+      tl += std::accumulate(part.begin() + b * nblk, part.begin() + (b + 1) * nblk, 0.0) / ((double)batch * c->nout);
+    for (long v = 0; v < nvb; ++v) {
+      const int rows = (int)std::min<long>(batch, nval - v * batch);
+      const auto p0 = part.begin() + (nbatch + v) * nblk;
+      vl += std::accumulate(p0, p0 + (rows + TROWS - 1) / TROWS, 0.0);
+    }
+    if (losses) {
+      losses[2 * ep] = nbatch ? tl / nbatch : 0.0;
+      losses[2 * ep + 1] = nval ? vl / ((double)nval * c->nout) : 0.0;
+    }
+  }
+  return LDG_OK;
+}
+
 // 1D L2 projection from order pf to order pc on the reference element:
 // P = M_c^{-1} B, B(i, j) = integral of l^c_i l^f_j, both integrals exact
 // (Gauss rules of pc+1 and pf+1 points).
@@ -279,6 +391,9 @@ void free_closure(ldg_closure *c) {
     if (b) (void)hipFree(b);
   if (c->idx) (void)hipFree(c->idx);
   if (c->part) (void)hipFree(c->part);
+  if (c->tws) (void)hipFree(c->tws);
+  if (c->tidx) (void)hipFree(c->tidx);
+  if (c->tpart) (void)hipFree(c->tpart);
   if (c->Wb) (void)hipFree(c->Wb);
   if (c->stream) (void)hipStreamDestroy(c->stream);
   delete c;
@@ -709,13 +824,14 @@ int ldg_closure_train(ldg_closure *c, int epochs, int batch, double lr, double v
   const long nval = (long)std::floor(val_fraction * c->count);
   const long ntrain = c->count - nval;
   if (ntrain < batch) return cfail(c, LDG_EINVAL, "fewer training samples than one batch");
-  int rc = ensure_workspace(c, batch);
-  if (rc) return rc;
   // a seeded random hold-out of nval samples; the rest is reshuffled every epoch
   std::mt19937_64 rng(seed);
   std::vector<long> all(c->count);
   std::iota(all.begin(), all.end(), 0L);
   std::shuffle(all.begin(), all.end(), rng);
+  if (fused_ok(c)) return train_fused(c, epochs, batch, lr, all, ntrain, rng, losses);
+  int rc = ensure_workspace(c, batch);
+  if (rc) return rc;
   std::vector<long> perm(all.begin(), all.begin() + ntrain);
   long *didx = nullptr, *dval = nullptr;
   CCHECK(c, hipMalloc((void **)&didx, std::max<long>(ntrain, 1) * sizeof(long)));
