@@ -33,7 +33,7 @@ struct ldg_closure {
   long nparam = 0;
   float *params = nullptr, *grads = nullptr, *m = nullptr, *v = nullptr;
   float *norm = nullptr;            // in_mean[nin], in_scale[nin] (1/std), out_mean[nout], out_std[nout]
-  unsigned short *Wb = nullptr;     // padded BF16 weight copies for the fused inference kernel
+  unsigned short *Wb = nullptr;     // BF16 weight copies of the fused kernels (none for other sizes)
   int k1p = 0, noutp = 0;
   long adam_t = 0;
   long cap = 0, count = 0;
@@ -173,8 +173,11 @@ int ensure_workspace(ldg_closure *c, int B) {
   return LDG_OK;
 }
 
-// Refreshes the BF16 weight copies used by the fused inference kernel.
+bool fused_ok(const ldg_closure *c) { return c->n == 3 && c->hidden == 256; }
+
+// Refreshes the BF16 weight copies of the fused kernels.
 int pack_bf16(ldg_closure *c) {
+  if (!fused_ok(c)) return LDG_OK;
   const Offs o = offsets(c);
   unsigned short *W1b = c->Wb, *W2b = W1b + (long)c->hidden * c->k1p, *W3b = W2b + (long)c->hidden * c->hidden;
   const long n = (long)c->hidden * c->k1p + (long)c->hidden * c->hidden + (long)c->noutp * c->hidden;
@@ -185,8 +188,6 @@ int pack_bf16(ldg_closure *c) {
   CCHECK(c, hipStreamSynchronize(c->stream));
   return LDG_OK;
 }
-
-bool fused_ok(const ldg_closure *c) { return c->n == 3 && c->hidden == 256; }
 
 // *p holds at least `need` values after the call (contents are not kept).
 template <typename T>
@@ -378,7 +379,7 @@ void launch_infer(hipStream_t s, const ldg_closure *c, const UT *U, const TQ *Q,
                   double bound, int dissipative, double rho_add, double *corr, unsigned char *gate) {
   const Offs o = offsets(c);
   const unsigned short *W1b = c->Wb, *W2b = W1b + (long)c->hidden * c->k1p, *W3b = W2b + (long)c->hidden * c->hidden;
-  hipLaunchKernelGGL((mlp_infer<TQ, UT, 540, 256, 135>), dim3((unsigned)((K + FR - 1) / FR)), dim3(256), 0, s, U, Q,
+  hipLaunchKernelGGL((mlp_infer<TQ, UT, 540, 256, 135>), dim3((unsigned)((K + FR - 1) / FR)), dim3(512), 0, s, U, Q,
                      K, rho0, E0, (const float *)c->norm, W1b, W2b, W3b, (const float *)(c->params + o.b1),
                      (const float *)(c->params + o.b2), (const float *)(c->params + o.b3), bound, dissipative,
                      rho_add, corr, gate);
@@ -497,8 +498,9 @@ int ldg_closure_create(int p, int hidden, long capacity, unsigned long long seed
       hipMalloc((void **)&c->m, pb) != hipSuccess || hipMalloc((void **)&c->v, pb) != hipSuccess ||
       hipMalloc((void **)&c->norm, sizeof(float) * 2 * (c->nin + c->nout)) != hipSuccess ||
       hipMalloc((void **)&c->part, sizeof(double) * kLossBlocks) != hipSuccess ||
-      hipMalloc((void **)&c->Wb, sizeof(unsigned short) * ((size_t)c->hidden * c->k1p + (size_t)c->hidden * c->hidden +
-                                                           (size_t)c->noutp * c->hidden)) != hipSuccess)
+      (fused_ok(c) &&
+       hipMalloc((void **)&c->Wb, sizeof(unsigned short) * ((size_t)c->hidden * c->k1p + (size_t)c->hidden * c->hidden +
+                                                           (size_t)c->noutp * c->hidden)) != hipSuccess))
     return bad(LDG_ENOMEM, "device allocation failed (closure parameters)");
   if (capacity > 0 && (hipMalloc((void **)&c->Xd, (size_t)capacity * c->nin * sizeof(float)) != hipSuccess ||
                        hipMalloc((void **)&c->Td, (size_t)capacity * c->nout * sizeof(float)) != hipSuccess ||

@@ -293,9 +293,18 @@ __global__ void mlp_normalize(float *__restrict__ D, long rows, int width, const
   }
 }
 
-// BF16 copies of the weight matrices for the fused inference kernel, rows
-// padded to a multiple of 16 columns (W1) and the output matrix to a
-// multiple of 32 rows (W3), padding zero:
+// An operand of the matrix cores in the order they take it: for every tile of
+// 32 rows (features) and step of 16 k (samples, or columns of a weight matrix)
+// 64 lanes x 8 values, so that a wave's load is one contiguous KiB.  op_at: the
+// place of (row, k); ldk: the k extent, a multiple of 16.
+__host__ __device__ constexpr long op_size(int rows, int ldk) { return (long)((rows + 31) / 32 * 32) * ldk; }
+__device__ inline long op_at(int row, int k, int ldk) {
+  return ((long)(row >> 5) * (ldk >> 4) + (k >> 4)) * 512 + (((k >> 3) & 1) * 32 + (row & 31)) * 8 + (k & 7);
+}
+
+// BF16 copies of the weight matrices for the fused kernels, in that order:
+// k padded to a multiple of 16 (W1) and the rows of the output matrix to a
+// multiple of 32 (W3), padding zero.
 //   W1b [hid][k1p], W2b [hid][hid], W3b [noutp][hid].
 __global__ void mlp_pack_bf16(const float *__restrict__ W1, const float *__restrict__ W2,
                               const float *__restrict__ W3, int nin, int hid, int nout, int k1p, int noutp,
@@ -306,16 +315,47 @@ __global__ void mlp_pack_bf16(const float *__restrict__ W1, const float *__restr
     if (w < n1) {
       const long r = w / k1p;
       const int c = (int)(w - r * k1p);
-      W1b[w] = c < nin ? to_bf16(W1[r * nin + c]) : 0;
+      W1b[op_at((int)r, c, k1p)] = c < nin ? to_bf16(W1[r * nin + c]) : 0;
     } else if (w < n1 + n2) {
-      W2b[w - n1] = to_bf16(W2[w - n1]);
+      W2b[op_at((int)((w - n1) / hid), (int)((w - n1) % hid), hid)] = to_bf16(W2[w - n1]);
     } else {
       const long v = w - n1 - n2;
       const long r = v / hid;
-      W3b[v] = r < nout ? to_bf16(W3[v]) : 0;
+      W3b[op_at((int)r, (int)(v - r * hid), hid)] = r < nout ? to_bf16(W3[v]) : 0;
     }
   }
 }
+
+// One wave's 32 x 32 tile of A W^T over KS steps of 16: A is 32 rows in LDS
+// (stride LDA), W the tile of weight rows at w (matrix-core order).  The first
+// PF steps' weights are loaded by the constructor (before the barrier that A
+// waits for), the later ones PF steps ahead.
+template <int KS, int PF>
+struct TileProduct {
+  static constexpr int P = PF < KS ? PF : KS;
+  const unsigned short *w;
+  u16x8 buf[P];
+  __device__ inline TileProduct(const unsigned short *__restrict__ W, int tile, int lane)
+      : w(W + (long)tile * KS * 512 + 8 * lane) {
+#pragma unroll
+    for (int p = 0; p < P; ++p) buf[p] = *reinterpret_cast<const u16x8 *>(w + 512 * p);
+  }
+  template <int LDA>
+  __device__ inline floatx16 run(const unsigned short *A, int lr, int kh) {
+    floatx16 acc;
+#pragma unroll
+    for (int j = 0; j < 16; ++j) acc[j] = 0.0f;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      const u16x8 cur = buf[s % P];
+      if (s + P < KS) buf[s % P] = *reinterpret_cast<const u16x8 *>(w + 512 * (s + P));
+      const u16x8 av = *reinterpret_cast<const u16x8 *>(A + lr * LDA + 16 * s + kh);
+      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, av), __builtin_bit_cast(bf16x8, cur),
+                                                    acc, 0, 0, 0);
+    }
+    return acc;
+  }
+};
 
 // Fused inference for p = 2 elements (27 nodes: NIN = 540 inputs, NOUT =
 // 135 outputs) and HID = 256: one workgroup evaluates the network on FR = 32
@@ -324,51 +364,29 @@ __global__ void mlp_pack_bf16(const float *__restrict__ W1, const float *__restr
 // MFMA layers with hidden activations kept in LDS, then the gate and the
 // correction.  Numerically identical to mlp_features + 3 x mlp_gemm +
 // mlp_correction (same roundings, same MFMA sequence over k).
+//
+// Bound by latency: 13,824 elements are 432 workgroups, all resident at once
+// (two to a CU), so the time is that of one workgroup's chain.  Measured there
+// in FP64: 28.6 us, 15 of them the 75 MB at HBM rate; 55 us with four waves
+// that loaded the features in eight dependent batches, divided for each
+// feature's place and read rows of weights 4 steps ahead.
 constexpr int FR = 32;
 
-// One wave: acc[t] += A (32 rows from LDS, row stride LDA) x W_t^T over KS
-// steps of 16, with W_t the 32 weight rows starting at w[t] (BF16, global).
-// Weight vectors are prefetched PF steps ahead so that the L2 latency is
-// covered by the matrix-core work of the steps in between.
-template <int KS, int NTILE, int LDA>
-__device__ inline void wave_layer(const unsigned short *__restrict__ A, const unsigned short *const (&w)[NTILE],
-                                  int lr, int kh, floatx16 (&acc)[NTILE]) {
-  constexpr int PF = 4;
-  u16x8 buf[PF][NTILE];
-#pragma unroll
-  for (int p = 0; p < PF; ++p)
-#pragma unroll
-    for (int t = 0; t < NTILE; ++t)
-      if (p < KS) buf[p][t] = *reinterpret_cast<const u16x8 *>(w[t] + 16 * p + kh);
-#pragma unroll
-  for (int s = 0; s < KS; ++s) {
-    u16x8 cur[NTILE];
-#pragma unroll
-    for (int t = 0; t < NTILE; ++t) {
-      cur[t] = buf[s % PF][t];
-      if (s + PF < KS) buf[s % PF][t] = *reinterpret_cast<const u16x8 *>(w[t] + 16 * (s + PF) + kh);
-    }
-    const u16x8 av = *reinterpret_cast<const u16x8 *>(A + lr * LDA + 16 * s + kh);
-#pragma unroll
-    for (int t = 0; t < NTILE; ++t)
-      acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, av), __builtin_bit_cast(bf16x8, cur[t]),
-                                                       acc[t], 0, 0, 0);
-  }
-}
-
 template <typename TQ, typename UT, int NIN, int HID, int NOUT>
-__global__ void __launch_bounds__(256) mlp_infer(const UT *__restrict__ U, const TQ *__restrict__ Q, long K,
-                                                 double rho0, double E0, const float *__restrict__ norm,
-                                                 const unsigned short *__restrict__ W1b,
-                                                 const unsigned short *__restrict__ W2b,
-                                                 const unsigned short *__restrict__ W3b, const float *__restrict__ b1,
-                                                 const float *__restrict__ b2, const float *__restrict__ b3,
-                                                 double bound, int dissipative, double rho_add,
-                                                 double *__restrict__ corr, unsigned char *__restrict__ gate) {
-  constexpr int DOFS = NIN / 20, NU = 5 * DOFS, NQ = 15 * DOFS;
+__global__ void __launch_bounds__(512, 4) mlp_infer(const UT *__restrict__ U, const TQ *__restrict__ Q, long K,
+                                                    double rho0, double E0, const float *__restrict__ norm,
+                                                    const unsigned short *__restrict__ W1b,
+                                                    const unsigned short *__restrict__ W2b,
+                                                    const unsigned short *__restrict__ W3b,
+                                                    const float *__restrict__ b1, const float *__restrict__ b2,
+                                                    const float *__restrict__ b3, double bound, int dissipative,
+                                                    double rho_add, double *__restrict__ corr,
+                                                    unsigned char *__restrict__ gate) {
+  constexpr int DOFS = NIN / 20, NU = 5 * DOFS, NQ = 15 * DOFS, NTHR = 512;
   constexpr int K1P = (NIN + 15) / 16 * 16, NOUTP = (NOUT + 31) / 32 * 32;
   constexpr int XS = K1P + 8, HS = HID + 8;
-  static_assert(HID == 256, "four waves of 64 hidden columns");
+  static_assert(HID == 256, "eight waves of 32 hidden columns");
+  static_assert(NOUTP / 32 <= 8, "one output tile per wave");
   static_assert(XS >= HS, "the second hidden layer reuses the feature buffer");
   __shared__ __align__(16) unsigned short Xs[FR][XS];
   __shared__ __align__(16) unsigned short Hs[FR][HS];
@@ -378,102 +396,87 @@ __global__ void __launch_bounds__(256) mlp_infer(const UT *__restrict__ U, const
   const int rows = (int)((K - e0) < FR ? (K - e0) : FR);
   const float *mean = norm, *scale = norm + NIN, *omean = norm + 2 * NIN, *ostd = norm + 2 * NIN + NOUT;
 
-  // normalisation to LDS, then the block's state and gradient rows, which
-  // are contiguous in HBM: each thread issues a batch of loads before using
-  // any of them
-  __shared__ float smean[NIN], sscale[NIN];
-  for (int j = tid; j < NIN; j += 256) { smean[j] = mean[j]; sscale[j] = scale[j]; }
-  for (int w = tid; w < FR * (K1P - NIN); w += 256) Xs[w / (K1P - NIN)][NIN + w % (K1P - NIN)] = 0;
+  // the block's state and gradient rows: thread j loads feature j of every
+  // row (past the last row: the last one's), then its share of the features
+  // past the threads, all before the first is used
+  constexpr int XTRA = NIN - NTHR, LX = (FR * XTRA + NTHR - 1) / NTHR;
+  static_assert(NU < NTHR && XTRA > 0, "one state or gradient feature per thread");
+  const UT *Ub = U + e0 * NU + tid;
+  const TQ *Qb = Q + e0 * NQ + (tid - NU);
+  using V = decltype(UT() + TQ());
+  V v[FR];
+  TQ x[LX];
+  if (tid < NU) {
+#pragma unroll
+    for (int r = 0; r < FR; ++r) v[r] = Ub[min(r, rows - 1) * NU];
+  } else {
+#pragma unroll
+    for (int r = 0; r < FR; ++r) v[r] = Qb[min(r, rows - 1) * NQ];
+  }
+  const double mj = (double)mean[tid], sj = (double)scale[tid];
+  float xm[LX], xs[LX];
+#pragma unroll
+  for (int i = 0; i < LX; ++i) {
+    const int w = tid + NTHR * i, r = w / XTRA, j = NTHR + w % XTRA;
+    x[i] = Q[(e0 + min(r, rows - 1)) * NQ + (j - NU)];
+    xm[i] = mean[j];
+    xs[i] = scale[j];
+  }
+  for (int w = tid; w < FR * (K1P - NIN); w += NTHR) Xs[w / (K1P - NIN)][NIN + w % (K1P - NIN)] = 0;
+  const double sub = tid < DOFS ? rho0 : tid >= 4 * DOFS && tid < NU ? E0 : 0.0;
+#pragma unroll
+  for (int r = 0; r < FR; ++r)
+    Xs[r][tid] = to_bf16(r < rows ? (float)(((double)v[r] - sub - mj) * sj) : 0.0f);
+#pragma unroll
+  for (int i = 0; i < LX; ++i) {
+    const int w = tid + NTHR * i, r = w / XTRA, j = NTHR + w % XTRA;
+    if (r < FR)
+      Xs[r][j] = to_bf16(r < rows ? (float)(((double)x[i] - (double)xm[i]) * (double)xs[i]) : 0.0f);
+  }
+  // wave w owns hidden columns [32 w, 32 w + 32)
+  const int lr = lane & 31, kh = (lane >> 5) * 8, c = 32 * wave + lr;
+  auto row_of = [&](int j) { return 8 * (j >> 2) + 4 * (lane >> 5) + (j & 3); };
+  TileProduct<K1P / 16, 17> p1(W1b, wave, lane);
   __syncthreads();
+  TileProduct<HID / 16, 16> p2(W2b, wave, lane);
   {
-    constexpr int B = 8;
-    const UT *Ub = U + e0 * NU;
-    for (int base = 0; base < FR * NU; base += 256 * B) {
-      double v[B];
+    const float bias = b1[c];
+    const floatx16 a = p1.template run<XS>(&Xs[0][0], lr, kh);
 #pragma unroll
-      for (int i = 0; i < B; ++i) {
-        const int idx = base + i * 256 + tid;
-        v[i] = idx < rows * NU ? (double)Ub[idx] : 0.0;
-      }
-#pragma unroll
-      for (int i = 0; i < B; ++i) {
-        const int idx = base + i * 256 + tid;
-        if (idx < FR * NU) {
-          const int r = idx / NU, j = idx - r * NU, s = j / DOFS;
-          const double x = v[i] - (s == 0 ? rho0 : s == 4 ? E0 : 0.0);
-          Xs[r][j] = to_bf16(r < rows ? (float)((x - (double)smean[j]) * (double)sscale[j]) : 0.0f);
-        }
-      }
-    }
-    const TQ *Qb = Q + e0 * NQ;
-    for (int base = 0; base < FR * NQ; base += 256 * B) {
-      double v[B];
-#pragma unroll
-      for (int i = 0; i < B; ++i) {
-        const int idx = base + i * 256 + tid;
-        v[i] = idx < rows * NQ ? (double)Qb[idx] : 0.0;
-      }
-#pragma unroll
-      for (int i = 0; i < B; ++i) {
-        const int idx = base + i * 256 + tid;
-        if (idx < FR * NQ) {
-          const int r = idx / NQ, j = NU + (idx - r * NQ);
-          Xs[r][j] = to_bf16(r < rows ? (float)((v[i] - (double)smean[j]) * (double)sscale[j]) : 0.0f);
-        }
-      }
-    }
+    for (int j = 0; j < 16; ++j) Hs[row_of(j)][c] = to_bf16(silu(a[j] + bias));
   }
   __syncthreads();
-
-  const int lr = lane & 31, kh = (lane >> 5) * 8;
-  // layer 1: wave w owns hidden columns [64 w, 64 w + 64)
-  {
-    floatx16 a[2];
-#pragma unroll
-    for (int j = 0; j < 16; ++j) { a[0][j] = 0.0f; a[1][j] = 0.0f; }
-    const unsigned short *const w[2] = {W1b + (long)(64 * wave + lr) * K1P, W1b + (long)(64 * wave + 32 + lr) * K1P};
-    wave_layer<K1P / 16, 2, XS>(&Xs[0][0], w, lr, kh, a);
-    const int c0 = 64 * wave + lr;
-#pragma unroll
-    for (int j = 0; j < 16; ++j) {
-      const int r = 8 * (j >> 2) + 4 * (lane >> 5) + (j & 3);
-      Hs[r][c0] = to_bf16(silu(a[0][j] + b1[c0]));
-      Hs[r][c0 + 32] = to_bf16(silu(a[1][j] + b1[c0 + 32]));
-    }
-  }
-  __syncthreads();
+  // output tiles of 32 columns, tile w on wave w
+  const bool ow = wave < NOUTP / 32;
+  TileProduct<HID / 16, 16> p3(W3b, ow ? wave : 0, lane);
   // layer 2 into the feature buffer
   {
-    floatx16 a[2];
+    const float bias = b2[c];
+    const floatx16 a = p2.template run<HS>(&Hs[0][0], lr, kh);
 #pragma unroll
-    for (int j = 0; j < 16; ++j) { a[0][j] = 0.0f; a[1][j] = 0.0f; }
-    const unsigned short *const w[2] = {W2b + (long)(64 * wave + lr) * HID, W2b + (long)(64 * wave + 32 + lr) * HID};
-    wave_layer<HID / 16, 2, HS>(&Hs[0][0], w, lr, kh, a);
-    const int c0 = 64 * wave + lr;
-#pragma unroll
-    for (int j = 0; j < 16; ++j) {
-      const int r = 8 * (j >> 2) + 4 * (lane >> 5) + (j & 3);
-      Xs[r][c0] = to_bf16(silu(a[0][j] + b2[c0]));
-      Xs[r][c0 + 32] = to_bf16(silu(a[1][j] + b2[c0 + 32]));
-    }
+    for (int j = 0; j < 16; ++j) Xs[row_of(j)][c] = to_bf16(silu(a[j] + bias));
   }
   __syncthreads();
-  // layer 3: output tiles of 32 columns, tile t on wave t mod 4
-  for (int t = wave; t < NOUTP / 32; t += 4) {
-    floatx16 a[1];
+  constexpr int OT = (NOUT + 63) / 64;
+  float os[OT], om[OT];
 #pragma unroll
-    for (int j = 0; j < 16; ++j) a[0][j] = 0.0f;
-    const unsigned short *const w[1] = {W3b + (long)(32 * t + lr) * HID};
-    wave_layer<HID / 16, 1, XS>(&Xs[0][0], w, lr, kh, a);
-    const int c = 32 * t + lr;
+  for (int t = 0; t < OT; ++t) {
+    os[t] = ostd[min(lane + 64 * t, NOUT - 1)];
+    om[t] = omean[min(lane + 64 * t, NOUT - 1)];
+  }
+  if (ow) {
+    const floatx16 a = p3.template run<XS>(&Xs[0][0], lr, kh);
     if (c < NOUT) {
 #pragma unroll
-      for (int j = 0; j < 16; ++j) Ys[8 * (j >> 2) + 4 * (lane >> 5) + (j & 3)][c] = a[0][j] + b3[c];
+      for (int j = 0; j < 16; ++j) Ys[row_of(j)][c] = a[j] + b3[c];
     }
   }
   __syncthreads();
   // gate and correction, one wave per row
-  for (int r = wave; r < rows; r += 4) {
+#pragma unroll
+  for (int i = 0; i < FR / (NTHR / 64); ++i) {
+    const int r = wave + i * (NTHR / 64);
+    if (r >= rows) break;
     float ss = 0.0f;
     for (int j = lane; j < NOUT; j += 64) ss += Ys[r][j] * Ys[r][j];
 #pragma unroll
@@ -482,8 +485,11 @@ __global__ void __launch_bounds__(256) mlp_infer(const UT *__restrict__ U, const
     const long e = e0 + r;
     if (on && dissipative)
       on = dissipative * ke_production(U + e * NU, rho_add, DOFS, &Ys[r][0], ostd, omean, lane) <= 0.0;
-    for (int j = lane; j < NOUT; j += 64)
-      corr[e * NOUT + j] = on ? (double)Ys[r][j] * (double)ostd[j] + (double)omean[j] : 0.0;
+#pragma unroll
+    for (int t = 0; t < OT; ++t) {
+      const int j = lane + 64 * t;
+      if (j < NOUT) corr[e * NOUT + j] = on ? (double)Ys[r][j] * (double)os[t] + (double)om[t] : 0.0;
+    }
     if (lane == 0) gate[e] = on ? 1 : 0;
   }
 }

@@ -11,8 +11,9 @@
 //                      straight into the matrix cores' registers; then Adam
 //                      on the tile and its BF16 copies.  Other workgroups sum
 //                      the bias gradients.
-// Bound by latency: 2,048 samples are 64 workgroups (30 us, the weights of
-// three layers there and back through each), and 128 dependent matrix
+// Bound by latency: 2,048 samples are 64 workgroups (22 us, the weights of
+// three layers there and back through each; 30 us with weights in plain
+// rows), and 128 dependent matrix
 // instructions per tile of the weight gradients (17 us).  As separate launches,
 // 17 per batch with a device synchronisation for the loss, a batch took
 // 1.85 ms, 1.2 ms of it column sums by 135 or 256 threads.
@@ -32,25 +33,19 @@ constexpr int TIN = 540, THID = 256, TOUT = 135;
 constexpr int TINP = 544, TOUTP = 144;      // k extents padded to the matrix step of 16
 constexpr int TROWS = 32;                   // samples per workgroup
 
-// BF16 copies of the weights, each row a run over k for one operand of one
-// product: W1 [hid][TINP], W2 [hid][hid], W3 [160][hid] for the forward pass
-// (fused inference uses the same, see mlp_pack_bf16), and W2^T [hid][hid],
-// W3^T [hid][TOUTP] for the backward pass.
+// BF16 copies of the weights in matrix-core order (op_at): W1 [hid][TINP],
+// W2 [hid][hid], W3 [160][hid] for the forward pass (those of the fused
+// inference), and W2^T [hid][hid], W3^T [hid][TOUTP] for the backward pass.
 struct TrainWeights {
   unsigned short *W1, *W2, *W3, *W2T, *W3T;
 };
-// Operands of the weight gradients, BF16, in the order the matrix cores take
-// them: per tile of 32 features and step of 16 samples, 64 lanes x 8 samples
-// (op_at), so that a wave's load is one contiguous KiB (as rows of 2,048
-// samples, 32 rows side by side, mlp_train_weights took 38 us, not 17).  Operands
-// of the bias gradients, FP32: per tile of 64 features [sample][64] (bias_at).
+// Operands of the weight gradients, BF16, in the same order (rows: features, k:
+// samples; with a plain row per feature, 32 rows of 2,048 samples side by side,
+// mlp_train_weights took 38 us, not 17).  Operands of the bias gradients, FP32:
+// per tile of 64 features [sample][64] (bias_at).
 // ldb: the samples rounded up to TPAD; the rest are zero in dY, dZ2, dZ1.
 constexpr int TPAD = 128;
-__host__ __device__ constexpr long op_size(int features, int ldb) { return (long)((features + 31) / 32 * 32) * ldb; }
 __host__ __device__ constexpr long bias_size(int features, int ldb) { return (long)((features + 63) / 64 * 64) * ldb; }
-__device__ inline long op_at(int f, int r, int ldb) {
-  return ((long)(f >> 5) * (ldb >> 4) + (r >> 4)) * 512 + (((r >> 3) & 1) * 32 + (f & 31)) * 8 + (r & 7);
-}
 __device__ inline long bias_at(int f, int r, int ldb) { return ((long)(f >> 6) * ldb + r) * 64 + (f & 63); }
 struct TrainOperands {
   unsigned short *X, *H1, *H2, *dY, *dZ2, *dZ1;
@@ -62,36 +57,6 @@ __device__ inline void store4(unsigned short *p, const unsigned short v[4]) {
   typedef unsigned short u16x4 __attribute__((ext_vector_type(4)));
   *reinterpret_cast<u16x4 *>(p) = u16x4{v[0], v[1], v[2], v[3]};
 }
-// One wave's 32 x 32 tile of A W^T over KS steps of 16: A is 32 rows in LDS
-// (stride LDA), W the 32 weight rows at w + (lane's row).  The first PF steps'
-// weights are loaded by the constructor (before the barrier that A waits for),
-// the later ones PF steps ahead.
-template <int KS, int PF>
-struct TileProduct {
-  static constexpr int P = PF < KS ? PF : KS;
-  const unsigned short *w;
-  u16x8 buf[P];
-  __device__ inline TileProduct(const unsigned short *__restrict__ w_, int kh) : w(w_ + kh) {
-#pragma unroll
-    for (int p = 0; p < P; ++p) buf[p] = *reinterpret_cast<const u16x8 *>(w + 16 * p);
-  }
-  template <int LDA>
-  __device__ inline floatx16 run(const unsigned short *A, int lr, int kh) {
-    floatx16 acc;
-#pragma unroll
-    for (int j = 0; j < 16; ++j) acc[j] = 0.0f;
-#pragma unroll
-    for (int s = 0; s < KS; ++s) {
-      const u16x8 cur = buf[s % P];
-      if (s + P < KS) buf[s % P] = *reinterpret_cast<const u16x8 *>(w + 16 * (s + P));
-      const u16x8 av = *reinterpret_cast<const u16x8 *>(A + lr * LDA + 16 * s + kh);
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, av), __builtin_bit_cast(bf16x8, cur),
-                                                    acc, 0, 0, 0);
-    }
-    return acc;
-  }
-};
-
 // Rows [32 b, 32 b + 32) of a batch of B samples (sample r: dataset row
 // idx[r]).  GRAD: also the backward pass and the operands; without it only
 // the loss.  part[b] = sum of rw (Y - T)^2.
@@ -115,7 +80,7 @@ __global__ void __launch_bounds__(512) mlp_train_rows(const float *__restrict__ 
   // holds row 8 (j/4) + 4 (l/32) + j%4, column l%32
   const int lr = lane & 31, kh = (lane >> 5) * 8, c = 32 * wave + lr;
   auto row_of = [&](int j) { return 8 * (j >> 2) + 4 * (lane >> 5) + (j & 3); };
-  TileProduct<TINP / 16, 17> p1(W.W1 + (long)c * TINP, kh);
+  TileProduct<TINP / 16, 17> p1(W.W1, wave, lane);
   if (tid < TROWS) {
     const bool in = r0 + tid < B;
     const long row = in ? idx[r0 + tid] : -1;
@@ -156,7 +121,7 @@ __global__ void __launch_bounds__(512) mlp_train_rows(const float *__restrict__ 
   }
   __syncthreads();
   float z1[16], z2[16];
-  TileProduct<THID / 16, 16> p2(W.W2 + (long)c * THID, kh);
+  TileProduct<THID / 16, 16> p2(W.W2, wave, lane);
   {
     const float bias = b1[c];
     const floatx16 a = p1.template run<XS>(&Xs[0][0], lr, kh);
@@ -184,7 +149,7 @@ __global__ void __launch_bounds__(512) mlp_train_rows(const float *__restrict__ 
   }
   __syncthreads();
   const bool ow = wave < (TOUT + 31) / 32;   // the output layer: tile w (columns [32 w, 32 w + 32) of 135) on wave w
-  TileProduct<THID / 16, 16> p3(W.W3 + (long)(ow ? c : lr) * THID, kh);
+  TileProduct<THID / 16, 16> p3(W.W3, ow ? wave : 0, lane);
   {
     const float bias = b2[c];
     const floatx16 a = p2.template run<HS>(&Hs[0][0], lr, kh);
@@ -202,7 +167,7 @@ __global__ void __launch_bounds__(512) mlp_train_rows(const float *__restrict__ 
     }
   }
   __syncthreads();
-  TileProduct<TOUTP / 16, TOUTP / 16> p4(GRAD ? W.W3T + (long)c * TOUTP : W.W1, kh);
+  TileProduct<TOUTP / 16, TOUTP / 16> p4(GRAD ? W.W3T : W.W1, GRAD ? wave : 0, lane);
   double loss = 0.0;
   if (ow) {
     const floatx16 a = p3.template run<HS>(&Gs[0][0], lr, kh);
@@ -244,7 +209,7 @@ __global__ void __launch_bounds__(512) mlp_train_rows(const float *__restrict__ 
     const float s = 1.0f / (1.0f + __expf(-z));
     return dh * s * __builtin_fmaf(z, 1.0f - s, 1.0f);
   };
-  TileProduct<THID / 16, 16> p5(W.W2T + (long)c * THID, kh);
+  TileProduct<THID / 16, 16> p5(W.W2T, wave, lane);
   {
     const floatx16 a = p4.template run<YS>(&Ys[0][0], lr, kh);
 #pragma unroll
@@ -430,13 +395,13 @@ __global__ void __launch_bounds__(256) mlp_train_weights(TrainOperands in, int l
     if (m < M && n < N) {
       const unsigned short h = to_bf16(adam_update(ad, o + (long)m * N + n, st[j], acc[j]));
       if (layer == 1) {
-        W.W1[(long)m * TINP + n] = h;
+        W.W1[op_at(m, n, TINP)] = h;
       } else if (layer == 2) {
-        W.W2[(long)m * THID + n] = h;
-        W.W2T[(long)n * THID + m] = h;
+        W.W2[op_at(m, n, THID)] = h;
+        W.W2T[op_at(n, m, THID)] = h;
       } else {
-        W.W3[(long)m * THID + n] = h;
-        W.W3T[(long)n * TOUTP + m] = h;
+        W.W3[op_at(m, n, THID)] = h;
+        W.W3T[op_at(n, m, TOUTP)] = h;
       }
     }
   }
@@ -446,10 +411,11 @@ __global__ void __launch_bounds__(256) mlp_train_weights(TrainOperands in, int l
 __global__ void mlp_pack_transposed(TrainWeights W) {
   for (int w = blockIdx.x * blockDim.x + threadIdx.x; w < THID * (THID + TOUTP); w += gridDim.x * blockDim.x) {
     if (w < THID * THID) {
-      W.W2T[w] = W.W2[(w % THID) * THID + w / THID];
+      const int r = w / THID, k = w - r * THID;
+      W.W2T[op_at(r, k, THID)] = W.W2[op_at(k, r, THID)];
     } else {
       const int v = w - THID * THID, r = v / TOUTP, k = v - r * TOUTP;
-      W.W3T[v] = k < TOUT ? W.W3[k * THID + r] : 0;
+      W.W3T[op_at(r, k, TOUTP)] = k < TOUT ? W.W3[op_at(k, r, THID)] : 0;
     }
   }
 }
