@@ -374,13 +374,14 @@ void features_group(ldg_handle *h, Group &g, StageIn U, const float *norm, int n
   }
 }
 
-template <typename TQ, typename UT>
-void launch_infer(hipStream_t s, const ldg_closure *c, const UT *U, const TQ *Q, long K, double rho0, double E0,
-                  double bound, int dissipative, double rho_add, double *corr, unsigned char *gate) {
+template <typename C, typename UT>
+void launch_infer(hipStream_t s, const ldg_closure *c, const UT *U, const InstDesc *inst, const Ops<3, double> *op,
+                  long K, double rho0, double E0, double bound, int dissipative, double rho_add, double *corr,
+                  unsigned char *gate) {
   const Offs o = offsets(c);
   const unsigned short *W1b = c->Wb, *W2b = W1b + (long)c->hidden * c->k1p, *W3b = W2b + (long)c->hidden * c->hidden;
-  hipLaunchKernelGGL((mlp_infer<TQ, UT, 540, 256, 135>), dim3((unsigned)((K + FR - 1) / FR)), dim3(512), 0, s, U, Q,
-                     K, rho0, E0, (const float *)c->norm, W1b, W2b, W3b, (const float *)(c->params + o.b1),
+  hipLaunchKernelGGL((mlp_infer<C, UT, 540, 256, 135>), dim3((unsigned)((K + FR - 1) / FR)), dim3(512), 0, s, U, inst,
+                     op, K, rho0, E0, (const float *)c->norm, W1b, W2b, W3b, (const float *)(c->params + o.b1),
                      (const float *)(c->params + o.b2), (const float *)(c->params + o.b3), bound, dissipative,
                      rho_add, corr, gate);
 }
@@ -404,6 +405,8 @@ void free_closure(ldg_closure *c) {
 
 namespace ldg_host {
 
+bool closure_reads_gradient(const Group &g) { return g.cl.net && !fused_ok(g.cl.net); }
+
 int closure_stage(ldg_handle *h, Group &g, StageIn U, StageArgs &st, int stage) {
   GroupClosure &cl = g.cl;
   if (!cl.net) return LDG_OK;
@@ -424,17 +427,19 @@ int closure_stage(ldg_handle *h, Group &g, StageIn U, StageArgs &st, int stage) 
       const double rho_add = U.fluct ? rho0 : 0.0;     // density = input + rho_add
       if (U.fluct) rho0 = E0 = 0.0;
       const long uo = off * 5 * dofs;
+      const InstDesc *inst = g.tile[0].d_inst + in.slot;
+      const Ops<3, double> *op = (const Ops<3, double> *)g.ops;
+      double *corr = cl.corr + off * c->nout;
+      unsigned char *gate = cl.gate + off;
       if (h->mixed && U.fluct)
-        launch_infer<float, float>(h->stream, c, (const float *)U.p + uo, (const float *)g.q + off * 15 * dofs, in.K,
-                                   rho0, E0, cl.bound, cl.dissipative, rho_add, cl.corr + off * c->nout, cl.gate + off);
+        launch_infer<float, float>(h->stream, c, (const float *)U.p + uo, inst, op, in.K, rho0, E0, cl.bound,
+                                   cl.dissipative, rho_add, corr, gate);
       else if (h->mixed)
-        launch_infer<float, double>(h->stream, c, (const double *)U.p + uo, (const float *)g.q + off * 15 * dofs,
-                                    in.K, rho0, E0, cl.bound, cl.dissipative, rho_add, cl.corr + off * c->nout,
-                                    cl.gate + off);
+        launch_infer<float, double>(h->stream, c, (const double *)U.p + uo, inst, op, in.K, rho0, E0, cl.bound,
+                                    cl.dissipative, rho_add, corr, gate);
       else
-        launch_infer<double, double>(h->stream, c, (const double *)U.p + uo, (const double *)g.q + off * 15 * dofs,
-                                     in.K, rho0, E0, cl.bound, cl.dissipative, rho_add, cl.corr + off * c->nout,
-                                     cl.gate + off);
+        launch_infer<double, double>(h->stream, c, (const double *)U.p + uo, inst, op, in.K, rho0, E0, cl.bound,
+                                     cl.dissipative, rho_add, corr, gate);
       off += in.K;
     }
   } else {

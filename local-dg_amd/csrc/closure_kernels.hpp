@@ -13,6 +13,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include "ldg_kernels.hpp"
+
 namespace ldg_mlp {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -359,22 +361,28 @@ struct TileProduct {
 
 // Fused inference for p = 2 elements (27 nodes: NIN = 540 inputs, NOUT =
 // 135 outputs) and HID = 256: one workgroup evaluates the network on FR = 32
-// elements of one instance entirely on chip -- features from the state and
-// gradient (background removed, normalised, rounded to BF16) into LDS, three
-// MFMA layers with hidden activations kept in LDS, then the gate and the
-// correction.  Numerically identical to mlp_features + 3 x mlp_gemm +
-// mlp_correction (same roundings, same MFMA sequence over k).
+// elements of one instance entirely on chip -- the nodal gradient from the
+// state in type C, the features (background removed, normalised, rounded to
+// BF16) into LDS, three MFMA layers with hidden activations kept in LDS, then
+// the gate and the correction.  Numerically identical to
+// ldg_nodal_grad_kernel + mlp_features + 3 x mlp_gemm + mlp_correction (same
+// roundings, same MFMA sequence over k).
+//
+// The gradient is formed here because a state is 5 of the 20 feature fields:
+// with the gradient written by a kernel of its own and read back, 13,824
+// elements moved 135 MB instead of 45 (FP64).
 //
 // Bound by latency: 13,824 elements are 432 workgroups, all resident at once
 // (two to a CU), so the time is that of one workgroup's chain.  Measured there
-// in FP64: 28.6 us, 15 of them the 75 MB at HBM rate; 55 us with four waves
-// that loaded the features in eight dependent batches, divided for each
-// feature's place and read rows of weights 4 steps ahead.
+// in FP64: 28.8 us, where the gradient kernel took 14.7 and the inference
+// without it 28.7 (55 with four waves that loaded the features in eight
+// dependent batches and rows of weights 4 steps ahead).
 constexpr int FR = 32;
 
-template <typename TQ, typename UT, int NIN, int HID, int NOUT>
-__global__ void __launch_bounds__(512, 4) mlp_infer(const UT *__restrict__ U, const TQ *__restrict__ Q, long K,
-                                                    double rho0, double E0, const float *__restrict__ norm,
+template <typename C, typename UT, int NIN, int HID, int NOUT>
+__global__ void __launch_bounds__(512, 4) mlp_infer(const UT *__restrict__ U, const ldg::InstDesc *__restrict__ inst,
+                                                    const ldg::Ops<3, double> *__restrict__ op, long K, double rho0,
+                                                    double E0, const float *__restrict__ norm,
                                                     const unsigned short *__restrict__ W1b,
                                                     const unsigned short *__restrict__ W2b,
                                                     const unsigned short *__restrict__ W3b,
@@ -382,56 +390,109 @@ __global__ void __launch_bounds__(512, 4) mlp_infer(const UT *__restrict__ U, co
                                                     const float *__restrict__ b3, double bound, int dissipative,
                                                     double rho_add, double *__restrict__ corr,
                                                     unsigned char *__restrict__ gate) {
-  constexpr int DOFS = NIN / 20, NU = 5 * DOFS, NQ = 15 * DOFS, NTHR = 512;
+  constexpr int N = 3, NF = N * N, DOFS = NIN / 20, NU = 5 * DOFS, NTHR = 512;
   constexpr int K1P = (NIN + 15) / 16 * 16, NOUTP = (NOUT + 31) / 32 * 32;
-  constexpr int XS = K1P + 8, HS = HID + 8;
+  constexpr int XS = K1P + 8, HS = HID + 8, YS = NOUT + 1;
+  static_assert(DOFS == N * NF, "27 nodes");
   static_assert(HID == 256, "eight waves of 32 hidden columns");
   static_assert(NOUTP / 32 <= 8, "one output tile per wave");
   static_assert(XS >= HS, "the second hidden layer reuses the feature buffer");
   __shared__ __align__(16) unsigned short Xs[FR][XS];
-  __shared__ __align__(16) unsigned short Hs[FR][HS];
-  __shared__ float Ys[FR][NOUT + 1];
+  // the state until the features are formed, then the hidden layer and the output
+  constexpr int SB = FR * NU * (int)sizeof(C), HB = FR * HS * 2, YB = FR * YS * 4;
+  __shared__ __align__(16) unsigned char buf[SB > HB + YB ? SB : HB + YB];
+  __shared__ float snorm[2 * NU];
+  __shared__ int snb[FR][3];
+  C *const su = reinterpret_cast<C *>(buf);
+  unsigned short(*const Hs)[HS] = reinterpret_cast<unsigned short(*)[HS]>(buf);
+  float(*const Ys)[YS] = reinterpret_cast<float(*)[YS]>(buf + HB);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const long e0 = (long)blockIdx.x * FR;
   const int rows = (int)((K - e0) < FR ? (K - e0) : FR);
-  const float *mean = norm, *scale = norm + NIN, *omean = norm + 2 * NIN, *ostd = norm + 2 * NIN + NOUT;
+  const float *omean = norm + 2 * NIN, *ostd = norm + 2 * NIN + NOUT;
 
-  // the block's state and gradient rows: thread j loads feature j of every
-  // row (past the last row: the last one's), then its share of the features
-  // past the threads, all before the first is used
-  constexpr int XTRA = NIN - NTHR, LX = (FR * XTRA + NTHR - 1) / NTHR;
-  static_assert(NU < NTHR && XTRA > 0, "one state or gradient feature per thread");
-  const UT *Ub = U + e0 * NU + tid;
-  const TQ *Qb = Q + e0 * NQ + (tid - NU);
-  using V = decltype(UT() + TQ());
-  V v[FR];
-  TQ x[LX];
-  if (tid < NU) {
+  // loads: the block's state (contiguous), then the -d neighbours' traces on
+  // their +d faces, both all in flight at once (past the last row: the last
+  // one's, whose results nothing reads).  A thread keeps one variable and face
+  // position, so that its features' means and spreads are loaded once, and
+  // takes the lines there of every RG-th row in all three directions.
+  constexpr int UL = (FR * NU + NTHR - 1) / NTHR, VF = 5 * NF, RG = NTHR / VF, LL = (FR + RG - 1) / RG;
+  UT v[UL], vn[3][LL];
+  const int tot = rows * NU;
 #pragma unroll
-    for (int r = 0; r < FR; ++r) v[r] = Ub[min(r, rows - 1) * NU];
-  } else {
+  for (int i = 0; i < UL; ++i) v[i] = U[e0 * NU + min(tid + NTHR * i, tot - 1)];
+  if (tid < FR) {
+    const int kl = (int)e0 + min(tid, rows - 1);
+    int c[3];
+    ldg::element_coords(*inst, kl, c);
 #pragma unroll
-    for (int r = 0; r < FR; ++r) v[r] = Qb[min(r, rows - 1) * NQ];
+    for (int D = 0; D < 3; ++D) snb[tid][D] = kl + ldg::neighbor_step(*inst, c, D, -1);
   }
-  const double mj = (double)mean[tid], sj = (double)scale[tid];
-  float xm[LX], xs[LX];
-#pragma unroll
-  for (int i = 0; i < LX; ++i) {
-    const int w = tid + NTHR * i, r = w / XTRA, j = NTHR + w % XTRA;
-    x[i] = Q[(e0 + min(r, rows - 1)) * NQ + (j - NU)];
-    xm[i] = mean[j];
-    xs[i] = scale[j];
+  for (int w = tid; w < NU; w += NTHR) {
+    snorm[w] = norm[w];
+    snorm[NU + w] = norm[NIN + w];
   }
   for (int w = tid; w < FR * (K1P - NIN); w += NTHR) Xs[w / (K1P - NIN)][NIN + w % (K1P - NIN)] = 0;
-  const double sub = tid < DOFS ? rho0 : tid >= 4 * DOFS && tid < NU ? E0 : 0.0;
+  __syncthreads();
+  const int g0 = tid / VF, sab = tid - g0 * VF, s = sab / NF, ab = sab - s * NF, a_ = ab % N, b_ = ab / N;
+  const int base[3] = {N * ab, a_ + NF * b_, ab};
+  constexpr int ST[3] = {1, N, NF};
 #pragma unroll
-  for (int r = 0; r < FR; ++r)
-    Xs[r][tid] = to_bf16(r < rows ? (float)(((double)v[r] - sub - mj) * sj) : 0.0f);
+  for (int i = 0; i < LL; ++i)
 #pragma unroll
-  for (int i = 0; i < LX; ++i) {
-    const int w = tid + NTHR * i, r = w / XTRA, j = NTHR + w % XTRA;
-    if (r < FR)
-      Xs[r][j] = to_bf16(r < rows ? (float)(((double)x[i] - (double)xm[i]) * (double)xs[i]) : 0.0f);
+    for (int D = 0; D < 3; ++D)
+      vn[D][i] = U[(long)snb[min(g0 + RG * i, FR - 1)][D] * NU + s * DOFS + base[D] + ST[D] * (N - 1)];
+#pragma unroll
+  for (int i = 0; i < UL; ++i) {
+    const int w = tid + NTHR * i, r = w / NU, j = w - r * NU, vs = j / DOFS;
+    if (w < FR * NU) {
+      su[w] = ldg::fluctuation<C>(v[i], vs, rho0, E0);
+      const double x = (double)v[i] - (vs == 0 ? rho0 : vs == 4 ? E0 : 0.0);
+      Xs[r][j] = to_bf16((float)((x - (double)snorm[j]) * (double)snorm[NU + j]));
+    }
+  }
+  __syncthreads();
+  // nodal gradient (operations and order of ldg_nodal_grad_kernel, nothing
+  // fused across the product with ialpha, which that kernel stores): the own
+  // trace's lift is in column 0 of Dn, the neighbour's has weight -L0
+  if (g0 < RG) {
+#pragma clang fp contract(off)
+    C dn[N][N + 1];
+#pragma unroll
+    for (int q = 0; q < N; ++q) {
+#pragma unroll
+      for (int j = 0; j < N; ++j) dn[q][j] = C(op->Dn[q][j] + (j == 0 ? op->L0[q] : 0.0));
+      dn[q][N] = C(-op->L0[q]);
+    }
+#pragma unroll
+    for (int D = 0; D < 3; ++D) {
+      const C ia = C(inst->ialpha[D]);
+      const int j = NU + (5 * D + s) * DOFS + base[D];
+      double mean[N], scale[N];
+#pragma unroll
+      for (int q = 0; q < N; ++q) {
+        mean[q] = (double)norm[j + ST[D] * q];
+        scale[q] = (double)norm[NIN + j + ST[D] * q];
+      }
+#pragma unroll
+      for (int i = 0; i < LL; ++i) {
+        const int r = g0 + RG * i;
+        if (r < FR) {
+          const C *const us = su + r * NU + s * DOFS + base[D];
+          const C nb = ldg::fluctuation<C>(vn[D][i], s, rho0, E0);
+          C x[N];
+#pragma unroll
+          for (int k = 0; k < N; ++k) x[k] = us[ST[D] * k];
+#pragma unroll
+          for (int q = 0; q < N; ++q) {
+            C g = dn[q][N] * nb;
+#pragma unroll
+            for (int k = 0; k < N; ++k) g = ldg::fma_(dn[q][k], x[k], g);
+            Xs[r][j + ST[D] * q] = to_bf16((float)(((double)(g * ia) - mean[q]) * scale[q]));
+          }
+        }
+      }
+    }
   }
   // wave w owns hidden columns [32 w, 32 w + 32)
   const int lr = lane & 31, kh = (lane >> 5) * 8, c = 32 * wave + lr;

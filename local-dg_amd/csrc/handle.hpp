@@ -130,8 +130,8 @@ struct StageIn {
 inline StageIn state_in(const double *u) { return StageIn{u, false}; }
 
 StageArgs empty_stage();
-// wq: write the nodal gradient Q (1), not (0), or only when a closure is
-// attached (-1)
+// wq: write the nodal gradient Q (1), not (0), or only when a closure that
+// reads it is attached (-1)
 int launch_grad(ldg_handle *h, Group &g, StageIn U, int c = -1, int wq = -1);
 int launch_rhs(ldg_handle *h, Group &g, StageIn U, const StageArgs &st, int c = -1);
 void drop_graph(ldg_handle *h);
@@ -140,9 +140,12 @@ void drop_graph(ldg_handle *h);
 size_t inst_offset(const ldg_handle *h, int i);
 size_t inst_values(const ldg_handle *h, int i);
 
+// closure.hip: whether the group's closure takes its features from g.q (the
+// fused inference forms the gradient itself).
+bool closure_reads_gradient(const Group &g);
 // closure.hip: before a stage's rhs launch, evaluates the group's closure on
-// the stage input U (and the gradient just computed into g.q) and points st
-// at the correction; no-op without a closure.
+// the stage input U (and the gradient just computed into g.q, if it reads it)
+// and points st at the correction; no-op without a closure.
 int closure_stage(ldg_handle *h, Group &g, StageIn U, StageArgs &st, int stage = 0);
 void closure_release(Group &g);
 

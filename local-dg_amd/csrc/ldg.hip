@@ -306,8 +306,8 @@ int launch_grad(ldg_handle *h, Group &g, StageIn U, int c, int wq) {
   if (U.fluct && !h->mixed) return fail(h, LDG_EINVAL, "FP32 stage input outside the mixed path");
   if (c < 0) c = g.cgrad;
   // the nodal gradient is written when asked for, and whenever a closure
-  // (whose features read it) is attached
-  const bool w = wq > 0 || (wq < 0 && g.cl.net != nullptr);
+  // whose features read it is attached
+  const bool w = wq > 0 || (wq < 0 && closure_reads_gradient(g));
   switch (g.n) {
     case 2: launch_grad_n<2>(h, g, c, U, w); break;
     case 3: launch_grad_n<3>(h, g, c, U, w); break;
