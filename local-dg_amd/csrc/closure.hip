@@ -263,7 +263,7 @@ int train_fused(ldg_closure *c, int epochs, int batch, double lr, const std::vec
       ++c->adam_t;
       ad.bc1 = 1.0f - (float)std::pow(ad.b1, (double)c->adam_t);
       ad.bc2 = 1.0f - (float)std::pow(ad.b2, (double)c->adam_t);
-      hipLaunchKernelGGL(mlp_train_weights, dim3(TRAIN_TILES / 4 + TRAIN_BIAS_BLOCKS), dim3(256), 0, s,
+      hipLaunchKernelGGL(mlp_train_weights, dim3(TRAIN_TILES + TRAIN_BIAS_BLOCKS), dim3(256), 0, s,
                          t, ldb, W, ad);
     }
     for (long v = 0; v < nvb; ++v) {

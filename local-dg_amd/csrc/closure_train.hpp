@@ -13,8 +13,8 @@
 //                      the bias gradients.
 // Bound by latency: 2,048 samples are 64 workgroups (22 us, the weights of
 // three layers there and back through each; 30 us with weights in plain
-// rows), and 128 dependent matrix
-// instructions per tile of the weight gradients (17 us).  As separate launches,
+// rows), and the operands of the weight gradients that the other XCDs just
+// wrote (14 us, see mlp_train_weights).  As separate launches,
 // 17 per batch with a device synchronisation for the loss, a batch took
 // 1.85 ms, 1.2 ms of it column sums by 135 or 256 threads.
 //
@@ -264,86 +264,111 @@ __device__ inline float adam_update(const AdamArgs &a, long w, const AdamState &
 
 constexpr int T1M = THID / 32, T1N = (TIN + 31) / 32, T2 = THID / 32, T3M = (TOUT + 31) / 32;
 constexpr int TRAIN_TILES = T1M * T1N + T2 * T2 + T3M * T2;
-constexpr int TRAIN_BIAS_BLOCKS = 2 * (THID / 64) + (TOUT + 63) / 64;
+constexpr int TBF = 32;                     // bias gradients per workgroup
+constexpr int TRAIN_BIAS_BLOCKS = 2 * (THID / TBF) + (TOUT + TBF - 1) / TBF;
 
 // Offsets of W1, b1, W2, b2, W3, b3 in the parameter vector.
 constexpr long TO_B1 = (long)THID * TIN, TO_W2 = TO_B1 + THID, TO_B2 = TO_W2 + (long)THID * THID, TO_W3 = TO_B2 + THID,
                TO_B3 = TO_W3 + (long)TOUT * THID;
 
-// Workgroups [0, TRAIN_TILES / 4): a wave per tile of dW = (rows of one
-// operand) x (rows of the other) summed over the samples; the rest: 64 bias
+// Workgroups [0, TRAIN_TILES): one wave on a tile of dW = (rows of one
+// operand) x (rows of the other) summed over the samples; the rest: TBF bias
 // gradients each.  Either the Adam update, and the weights' BF16 copies.
-__global__ void __launch_bounds__(256) mlp_train_weights(TrainOperands in, int ldb, TrainWeights W, AdamArgs ad) {
-  // bias: BS samples of a tile of 64 features at a time through LDS, summed
-  // sample by sample by one lane per feature while the next are loaded
-  constexpr int BS = TPAD, BL = BS * 64 / 4 / 256;
-  __shared__ __align__(16) float sbias[2][BS][64];
-  static_assert(TRAIN_TILES % 4 == 0, "whole workgroups of tiles");
+//
+// A tile reads 256 KB (2,048 samples) for 1.7 us of matrix instructions, so
+// its time is the rate at which a CU takes operands: a tile per CU (the bias
+// workgroups are why there are four waves; three leave at once).  Workgroups
+// go to the 8 XCDs in turn; each XCD gets an eighth of every layer's tiles,
+// those of the same columns, so that its L2 fetches 3 MB of operands instead
+// of nearly all 6.6.  Measured at 2,048 samples: 14.2 us (tiles alone 11.4, bias
+// gradients alone 12.1); 17.2 with four tiles per workgroup in any order and
+// bias workgroups of 64 features whose additions each waited for LDS.
+__global__ void __launch_bounds__(256, 1) mlp_train_weights(TrainOperands in, int ldb, TrainWeights W, AdamArgs ad) {
+  // bias: BS samples of TBF features at a time through LDS, summed sample by
+  // sample by one lane per feature while the next BG - 1 pieces are loaded
+  constexpr int BS = TPAD, BG = 4, BL = BS * TBF / 4 / 256;
+  __shared__ __align__(16) float sbias[2][BS][TBF];
+  static_assert(T1M == 8 && T2 == 8, "each layer's tiles in 8 equal shares");
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  if ((int)blockIdx.x >= TRAIN_TILES / 4) {
-    // tiles 0-3: dZ1 (256 features), 4-7: dZ2, 8-10: dY (135)
-    const int tile = (int)blockIdx.x - TRAIN_TILES / 4;
-    const float *d = tile < 4 ? in.fZ1 : tile < 8 ? in.fZ2 : in.fY;
-    const int ft = tile < 8 ? tile & 3 : tile - 8, f = 64 * ft + lane;
-    d += (long)ft * ldb * 64;
-    // (the loads of a chunk as one vector value: as an array it went to scratch memory)
-    using Buf = float __attribute__((ext_vector_type(4 * BL)));
+  if ((int)blockIdx.x >= TRAIN_TILES) {
+    // dZ1 (256 features), dZ2 (256), dY (135)
+    constexpr int HB = THID / TBF;
+    const int tile = (int)blockIdx.x - TRAIN_TILES;
+    const float *d = tile < HB ? in.fZ1 : tile < 2 * HB ? in.fZ2 : in.fY;
+    const int f0 = TBF * (tile < 2 * HB ? tile % HB : tile - 2 * HB), f = f0 + lane;
+    d += (long)(f0 >> 6) * ldb * 64 + (f0 & 63);
     using f4 = float __attribute__((ext_vector_type(4)));
-    Buf even, odd;
-    auto load = [&](Buf &buf, int k0) {
-#pragma unroll
-      for (int i = 0; i < BL; ++i) {
-        const f4 v = reinterpret_cast<const f4 *>(d + (long)min(k0, ldb - BS) * 64)[tid + 256 * i];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) buf[4 * i + j] = v[j];
-      }
-    };
+    f4 buf[BG][BL];
+    constexpr int Q = TBF / 4;                 // 16-byte pieces of a sample
     float s = 0.0f;
-    auto chunk = [&](float (&sb)[BS][64], Buf &buf, int k0) {
+    const f4 *const src = reinterpret_cast<const f4 *>(d) + tid / Q * 16 + tid % Q;
+    auto load = [&](f4 (&v)[BL], int k0) {
 #pragma unroll
-      for (int i = 0; i < BL; ++i)
-        reinterpret_cast<f4 *>(&sb[0][0])[tid + 256 * i] =
-            f4{buf[4 * i], buf[4 * i + 1], buf[4 * i + 2], buf[4 * i + 3]};
-      __syncthreads();   // (the sums of two chunks ago, from the same buffer, ended before it)
-      load(buf, k0 + 2 * BS);
+      for (int i = 0; i < BL; ++i) v[i] = src[(long)(min(k0, ldb - BS) + i * (256 / Q)) * 16];
+    };
+    auto piece = [&](f4 (&v)[BL], int g, auto then) {
+#pragma unroll
+      for (int i = 0; i < BL; ++i) reinterpret_cast<f4 *>(&sbias[g & 1][0][0])[tid + 256 * i] = v[i];
+      __syncthreads();   // (the sums of two pieces ago, from the same buffer, ended before it)
+      then();
       if (wave == 0) {
-#pragma unroll 32
-        for (int k = 0; k < BS; ++k) s += sb[k][lane];
+        // 32 values on their way while 32 are added (left to the scheduler,
+        // every two additions wait for their own read: 38 us)
+        constexpr int R = 32;
+        float x[2][R];
+#pragma unroll
+        for (int k = 0; k < R; ++k) x[0][k] = sbias[g & 1][k][lane & (TBF - 1)];
+#pragma unroll
+        for (int c = 0; c < BS / R; ++c) {
+          if (c + 1 < BS / R) {
+#pragma unroll
+            for (int k = 0; k < R; ++k) x[(c + 1) & 1][k] = sbias[g & 1][(c + 1) * R + k][lane & (TBF - 1)];
+          }
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int k = 0; k < R; ++k) s += x[c & 1][k];
+          __builtin_amdgcn_sched_barrier(0);
+        }
       }
     };
-    load(even, 0);
-    load(odd, BS);
-    for (int k0 = 0; k0 < ldb; k0 += 2 * BS) {
-      chunk(sbias[0], even, k0);
-      if (k0 + BS < ldb) chunk(sbias[1], odd, k0 + BS);
+#pragma unroll
+    for (int g = 0; g < BG; ++g) load(buf[g], g * BS);
+    int k0 = 0;
+    // (no condition inside the loop: at a join of paths every load is waited for)
+    for (; k0 + BG * BS <= ldb; k0 += BG * BS) {
+#pragma unroll
+      for (int g = 0; g < BG; ++g) piece(buf[g], g, [&] { load(buf[g], k0 + (g + BG) * BS); });
     }
-    if (wave == 0 && f < (tile < 8 ? THID : TOUT)) {
-      const long w = (tile < 4 ? TO_B1 : tile < 8 ? TO_B2 : TO_B3) + f;
+#pragma unroll
+    for (int g = 0; g < BG - 1; ++g)
+      if (k0 + g * BS < ldb) piece(buf[g], g, [] {});
+    if (wave == 0 && lane < TBF && f < (tile < 2 * HB ? THID : TOUT)) {
+      const long w = (tile < HB ? TO_B1 : tile < 2 * HB ? TO_B2 : TO_B3) + f;
       adam_update(ad, w, adam_load(ad, w), s);
     }
     return;
   }
-  const int blk = 4 * (int)blockIdx.x + wave;
+  if (wave > 0) return;
   const unsigned short *A, *Bp;
   int m0, n0, M, N;
   long o;
   int layer;
-  if (blk < T1M * T1N) {
+  const int xcd = (int)blockIdx.x & 7, i = (int)blockIdx.x >> 3;   // i: tile of the XCD's share
+  if (i < T1N) {
     layer = 1;
-    m0 = blk / T1N * 32;
-    n0 = blk % T1N * 32;
+    const int k = T1N * xcd + i;
+    m0 = k % T1M * 32;
+    n0 = k / T1M * 32;
     A = in.dZ1; Bp = in.X; M = THID; N = TIN; o = 0;
-  } else if (blk < T1M * T1N + T2 * T2) {
-    const int b = blk - T1M * T1N;
+  } else if (i < T1N + T2) {
     layer = 2;
-    m0 = b / T2 * 32;
-    n0 = b % T2 * 32;
+    m0 = (i - T1N) * 32;
+    n0 = xcd * 32;
     A = in.dZ2; Bp = in.H1; M = THID; N = THID; o = TO_W2;
   } else {
-    const int b = blk - T1M * T1N - T2 * T2;
     layer = 3;
-    m0 = b / T2 * 32;
-    n0 = b % T2 * 32;
+    m0 = (i - T1N - T2) * 32;
+    n0 = xcd * 32;
     A = in.dY; Bp = in.H2; M = TOUT; N = THID; o = TO_W3;
   }
   const int lr = lane & 31;
@@ -361,10 +386,10 @@ __global__ void __launch_bounds__(256) mlp_train_weights(TrainOperands in, int l
     const int m = row_of(j) < M ? row_of(j) : M - 1;
     st[j] = adam_load(ad, o + (long)m * N + (n < N ? n : N - 1));
   }
-  // two groups of PF matrix steps in flight: the operands were just written by
+  // PG groups of PF matrix steps in flight: the operands were just written by
   // the other XCDs, so every read goes past the L2
-  constexpr int PF = TPAD / 16;
-  u16x8 ba[2][PF], bb[2][PF];
+  constexpr int PF = TPAD / 16, PG = 2;
+  u16x8 ba[PG][PF], bb[PG][PF];
   auto load = [&](int g, int k0) {
 #pragma unroll
     for (int p = 0; p < PF; ++p) {
@@ -379,16 +404,24 @@ __global__ void __launch_bounds__(256) mlp_train_weights(TrainOperands in, int l
                                                     __builtin_bit_cast(bf16x8, bb[g][p]), acc, 0, 0, 0);
   };
   const int last = ldb - TPAD;
-  load(0, 0);
-  load(1, TPAD < last ? TPAD : last);
-  for (int k0 = 0; k0 < ldb; k0 += 2 * TPAD) {
-    product(0);
-    load(0, k0 + 2 * TPAD < last ? k0 + 2 * TPAD : last);
-    if (k0 + TPAD < ldb) {
-      product(1);
-      load(1, k0 + 3 * TPAD < last ? k0 + 3 * TPAD : last);
+#pragma unroll
+  for (int g = 0; g < PG; ++g) {
+    load(g, min(g * TPAD, last));
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  int k0 = 0;
+  for (; k0 + PG * TPAD <= ldb; k0 += PG * TPAD) {   // (no condition inside, as above)
+#pragma unroll
+    for (int g = 0; g < PG; ++g) {
+      product(g);
+      __builtin_amdgcn_sched_barrier(0);   // keep the groups in order: their loads are waited for in order
+      load(g, min(k0 + (g + PG) * TPAD, last));
+      __builtin_amdgcn_sched_barrier(0);
     }
   }
+#pragma unroll
+  for (int g = 0; g < PG - 1; ++g)
+    if (k0 + g * TPAD < ldb) product(g);
 #pragma unroll
   for (int j = 0; j < 16; ++j) {
     const int m = row_of(j);
