@@ -92,7 +92,7 @@ struct ldg_handle {
   hipEvent_t ev_fork = nullptr;
   std::vector<hipEvent_t> ev_join;
   double *ke_hist = nullptr, *scal = nullptr;
-  int *d_step = nullptr;
+  int *d_step = nullptr;            // per instance (group by group): next history row of a graph replay
   size_t ke_hist_cap = 0;          // kKeHistSteps x instances, allocated at create
   std::vector<double> dt_cur;       // dt currently written into the instance tables
   bool use_graph = false;

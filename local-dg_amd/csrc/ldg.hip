@@ -547,7 +547,7 @@ int create_impl(const ldg_config *cfg, const ldg_instance *insts, int n, ldg_han
     std::vector<double> sc;
     for (int idx : g.members) sc.push_back(ke_scale(h->cfg, h->inst[idx]));
     if (hipMalloc((void **)&g.ke_part, sizeof(double) * (maxblk + 1)) != hipSuccess ||
-        hipMalloc((void **)&g.diag_part, sizeof(double) * 2 * (maxblk + 1)) != hipSuccess ||
+        hipMalloc((void **)&g.diag_part, sizeof(double) * 3 * (maxblk + 1)) != hipSuccess ||
         hipMalloc((void **)&g.d_scale, sizeof(double) * sc.size()) != hipSuccess) {
       h->err = "device allocation failed (partials)";
       return bad(LDG_ENOMEM);
@@ -561,7 +561,7 @@ int create_impl(const ldg_config *cfg, const ldg_instance *insts, int n, ldg_han
   // out chunk by chunk, so a step call never allocates
   h->ke_hist_cap = (size_t)kKeHistSteps * n;
   if (hipMalloc((void **)&h->scal, sizeof(double) * 3 * n) != hipSuccess ||
-      hipMalloc((void **)&h->d_step, sizeof(int)) != hipSuccess ||
+      hipMalloc((void **)&h->d_step, sizeof(int) * n) != hipSuccess ||
       hipMalloc((void **)&h->ke_hist, sizeof(double) * h->ke_hist_cap) != hipSuccess) {
     h->err = "device allocation failed (scalars)";
     return bad(LDG_ENOMEM);
@@ -588,14 +588,15 @@ int set_dt(ldg_handle *h, const double *dt) {
 }
 
 // One RK4 step of every group (eager launches).  With ke, each group's
-// kinetic energies of u^{n+1} go to row *d_step of the KE history.  In the
+// kinetic energies of u^{n+1} go to the given row of the KE history (row < 0:
+// the row the device counters name).  In the
 // mixed path without a closure, a step
 // that follows another one in the same call (in32) reads its stage-1 input
 // as the FP32 fluctuations the previous step's stage 4 left in ub (out32);
 // ub is free then (stage 4 reads ua) and is only rewritten by stage 2.  The
 // kernels round an FP64 stage-1 input to the same FP32 values, so results do
 // not depend on how steps are split into calls or graph replays.
-int rk4_step(ldg_handle *h, bool ke, bool in32, bool out32) {
+int rk4_step(ldg_handle *h, bool ke, int row, bool in32, bool out32) {
   static const double b[4] = {1 / 6.0, 1 / 3.0, 1 / 3.0, 1 / 6.0};
   static const double a[3] = {0.5, 0.5, 1.0};
   // with several order groups each runs on its own stream between a fork
@@ -644,9 +645,9 @@ int rk4_step(ldg_handle *h, bool ke, bool in32, bool out32) {
     }
     if (ke) {
       const Tiling &t = g.tile[g.rhs[g.crhs]];
-      hipLaunchKernelGGL(ldg_finalize_kernel, dim3(g.members.size()), dim3(NT), 0, h->stream,
+      hipLaunchKernelGGL(ldg_finalize_kernel, dim3(g.members.size()), dim3(FIN_NT), 0, h->stream,
                          (const double *)g.ke_part, 1, (const InstDesc *)t.d_inst, (int)h->inst.size(),
-                         (const double *)g.d_scale, h->ke_hist + first, (const int *)h->d_step);
+                         (const double *)g.d_scale, h->ke_hist + first, row, h->d_step + first);
       HIPCHECK(h, hipGetLastError());
     }
     if (fork) {
@@ -658,10 +659,6 @@ int rk4_step(ldg_handle *h, bool ke, bool in32, bool out32) {
   }
   if (fork)
     for (hipEvent_t ev : h->ev_join) HIPCHECK(h, hipStreamWaitEvent(main, ev, 0));
-  if (ke) {
-    hipLaunchKernelGGL(ldg_advance_kernel, dim3(1), dim3(1), 0, h->stream, h->d_step);
-    HIPCHECK(h, hipGetLastError());
-  }
   return LDG_OK;
 }
 
@@ -698,8 +695,8 @@ int get_graph(ldg_handle *h, bool ke, bool first, hipGraphExec_t *out) {
   gs = ldg_handle::GraphSlot();
   hipGraph_t graph = nullptr;
   HIPCHECK(h, hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
-  int rc = rk4_step(h, ke, !first, true);
-  if (!rc) rc = rk4_step(h, ke, true, true);
+  int rc = rk4_step(h, ke, -1, !first, true);
+  if (!rc) rc = rk4_step(h, ke, -1, true, true);
   hipError_t e = hipStreamEndCapture(h->stream, &graph);
   if (rc) { if (graph) (void)hipGraphDestroy(graph); return rc; }
   if (e != hipSuccess) return fail(h, LDG_EDEVICE, std::string("hipStreamEndCapture: ") + hipGetErrorString(e));
@@ -735,13 +732,12 @@ int step_impl(ldg_handle *h, const double *dt, int nsteps, double *ke) {
   // chunks of at most kKeHistSteps steps when the KE history is recorded:
   // the device history row counter restarts and the rows are copied out
   // after each chunk
-  const int zero = 0;
   int done = 0;
   while (done < nsteps) {
     const int n = ke ? std::min<int>((int)(h->ke_hist_cap / ni), nsteps - done) : nsteps - done;
-    if (ke) HIPCHECK(h, hipMemcpyAsync(h->d_step, &zero, sizeof(int), hipMemcpyHostToDevice, h->stream));
     int k = 0;
     if (h->use_graph && n >= 2) {
+      if (ke) HIPCHECK(h, hipMemsetAsync(h->d_step, 0, sizeof(int) * ni, h->stream));
       // the first replay of a call reads the FP64 state, later ones the FP32
       // stage-1 input the step before left
       hipGraphExec_t first = nullptr, later = nullptr;
@@ -751,7 +747,7 @@ int step_impl(ldg_handle *h, const double *dt, int nsteps, double *ke) {
       for (; k + 2 <= n; k += 2) HIPCHECK(h, hipGraphLaunch(done + k ? later : first, h->stream));
     }
     for (; k < n; ++k) {
-      rc = rk4_step(h, ke != nullptr, done + k > 0, done + k + 1 < nsteps);
+      rc = rk4_step(h, ke != nullptr, k, done + k > 0, done + k + 1 < nsteps);
       if (rc) return rc;
     }
     if (ke)
@@ -1043,17 +1039,13 @@ int ldg_instance_diagnostics(ldg_handle *h, int i, double out[3]) {
   int first = 0;
   for (Group &g : h->groups) {
     StageArgs st = empty_stage();
-    st.ke_part = g.ke_part;
     st.diag_part = g.diag_part;
     const int rc = launch_rhs(h, g, state_in(g.u), st, 0);
     if (rc) return rc;
     const Tiling &t = g.tile[g.rhs[0]];
-    hipLaunchKernelGGL(ldg_finalize_kernel, dim3(g.members.size()), dim3(NT), 0, h->stream, (const double *)g.ke_part,
-                       1, (const InstDesc *)t.d_inst, ni, (const double *)g.d_scale, h->scal + first,
-                       (const int *)nullptr);
-    hipLaunchKernelGGL(ldg_finalize_kernel, dim3(g.members.size()), dim3(NT), 0, h->stream,
-                       (const double *)g.diag_part, 2, (const InstDesc *)t.d_inst, ni, (const double *)g.d_scale,
-                       h->scal + ni + 2 * first, (const int *)nullptr);
+    hipLaunchKernelGGL(ldg_finalize_kernel, dim3(g.members.size(), 3), dim3(FIN_NT), 0, h->stream,
+                       (const double *)g.diag_part, 3, (const InstDesc *)t.d_inst, ni, (const double *)g.d_scale,
+                       h->scal + 3 * first, 0, (int *)nullptr);
     HIPCHECK(h, hipGetLastError());
     first += (int)g.members.size();
   }
@@ -1063,11 +1055,7 @@ int ldg_instance_diagnostics(ldg_handle *h, int i, double out[3]) {
   // instances are numbered group by group in the arrays above
   const std::vector<int> order = group_order(h);
   for (int pos = 0; pos < ni; ++pos) {
-    if (order[pos] == i) {
-      out[0] = all[pos];
-      out[1] = all[ni + 2 * pos];
-      out[2] = all[ni + 2 * pos + 1];
-    }
+    if (order[pos] == i) std::copy(&all[3 * pos], &all[3 * pos] + 3, out);
   }
   for (int k = 0; k < 3; ++k)
     if (!std::isfinite(out[k])) return fail(h, LDG_ENONFINITE, "diagnostic is non-finite");

@@ -90,7 +90,7 @@ struct StageArgs {
   double cb, ca;      // RK4 coefficients b_s, a_s (times each instance's dt)
   int acc_init;       // 1: acc = u0 + dt b k   0: acc += dt b k
   double *ke_part;    // per-workgroup partial sums of the reference KE of acc
-  double *diag_part;  // per-workgroup partial sums (Gauss KE, enstrophy)
+  double *diag_part;  // or those of the diagnostics (reference KE, Gauss KE, enstrophy)
   const double *corr;          // learned closure: k += corr where gate[element] != 0
   const unsigned char *gate;
 };
@@ -495,21 +495,6 @@ __device__ inline void face_flux_pair(const T wK[5], const T wN[5], const T *q, 
     outK[1 + i] = R[1 + i] - fK[i];
     outN[1 + i] = fN[i] - R[1 + i];
   }
-}
-
-// ---------------------------------------------------------------------
-// Block-wide deterministic sum of one double per thread -> every thread: a
-// fixed butterfly inside each wave (every lane ends with the same wave
-// total), then the NT/64 wave totals in a fixed order through sw[NT/64].
-// A caller that sums again with the same sw puts a barrier in between.
-// ---------------------------------------------------------------------
-__device__ inline double block_sum(double v, double *sw) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  if ((threadIdx.x & 63) == 0) sw[threadIdx.x >> 6] = v;
-  __syncthreads();
-  static_assert(NT == 256, "four wave totals");
-  return (sw[0] + sw[1]) + (sw[2] + sw[3]);
 }
 
 // ---------------------------------------------------------------------
@@ -1055,9 +1040,8 @@ struct RhsLds {
   static constexpr int WAVES = sizeof(T) == 4 && N <= 5 ? 3 : 2;
 };
 
-// DIAG: instead of the rate, the diagnostics of the state U: st.ke_part and
-// st.diag_part (the nodal and the Gauss-point sums), from the state and its
-// gradient at the Gauss points; no face fluxes are read.
+// DIAG: instead of the rate, the diagnostics of the state U to st.diag_part
+// (the nodal and the two Gauss-point sums), from the state and its gradient at the Gauss points; no face fluxes are read.
 template <int N, int E, typename T, typename UT, bool DIAG>
 __global__ void __launch_bounds__((Shape<N, E>::NTH), (RhsLds<N, E, T>::WAVES))
 ldg_rhs_kernel(const UT *__restrict__ U, const T *__restrict__ FF, LaunchArgs la,
@@ -1074,7 +1058,8 @@ ldg_rhs_kernel(const UT *__restrict__ U, const T *__restrict__ FF, LaunchArgs la
   const InstDesc &d = block_span(la, lb, E, kl, ne);
   if (ne <= 0) {                      // padding block: empty partial sums
     if (t == 0 && st.ke_part) st.ke_part[lb] = 0.0;
-    if (DIAG && t == 0) st.diag_part[2 * lb] = st.diag_part[2 * lb + 1] = 0.0;
+    if (DIAG && t == 0)
+      for (int j = 0; j < 3; ++j) st.diag_part[3 * lb + j] = 0.0;
     return;
   }
   const long k0 = d.elem_off + kl;
@@ -1323,9 +1308,9 @@ ldg_rhs_kernel(const UT *__restrict__ U, const T *__restrict__ FF, LaunchArgs la
   if constexpr (DIAG) {
     const double n = group_sum<NTH>(dkn, sred), x = group_sum<NTH>(dke, sred), y = group_sum<NTH>(dens, sred);
     if (t == 0) {
-      st.ke_part[lb] = n;
-      st.diag_part[2 * lb] = x;
-      st.diag_part[2 * lb + 1] = y;
+      st.diag_part[3 * lb] = n;
+      st.diag_part[3 * lb + 1] = x;
+      st.diag_part[3 * lb + 2] = y;
     }
     return;
   }
@@ -1515,47 +1500,45 @@ ldg_rhs_kernel(const UT *__restrict__ U, const T *__restrict__ FF, LaunchArgs la
 }
 
 // Ordered per-instance sums of per-workgroup partials, one workgroup per
-// instance: out[(row * row_stride + i) * stride + j] = scale_i * (sum over
-// the instance's blocks b of part[b * stride + j]), row = *step (0 if null).
-static __global__ void __launch_bounds__(NT) ldg_finalize_kernel(const double *__restrict__ part, int stride,
+// instance i and partial j of `stride`: out[(row * row_stride + i) * stride + j] = scale_i * (sum over
+// the instance's blocks b of part[b * stride + j]).  With `step` a row of a
+// history: row >= 0 is the row, row < 0 (graph replays) the instance's own
+// counter step[i], which is left at the row after it; without it row 0.
+//
+// One workgroup reads every partial, so what counts is the loads in flight:
+// 128 KB (64^3, p = 4: 131,072 partials in 27 us; 33 with 256 threads).
+constexpr int FIN_NT = 1024;
+static __global__ void __launch_bounds__(FIN_NT) ldg_finalize_kernel(const double *__restrict__ part, int stride,
                                                             const InstDesc *__restrict__ inst, int row_stride,
                                                             const double *__restrict__ scale, double *__restrict__ out,
-                                                            const int *__restrict__ step) {
-  __shared__ double sred[NT / 64];
-  const int i = blockIdx.x;
+                                                            int row, int *__restrict__ step) {
+  __shared__ double sred[FIN_NT / 64];
+  const int i = blockIdx.x, j = blockIdx.y;
   const int b0 = inst[i].block_off, b1 = b0 + inst[i].nblocks;
-  const long row = step ? *step : 0;
-  constexpr int A = 32;   // accumulators per thread: loads in flight (one workgroup reads every partial)
-  for (int j = 0; j < stride; ++j) {
-    // thread t sums blocks b0 + t + k NT into accumulator k mod A; the
-    // order depends only on b - b0
-    double acc[A];
+  const long r = !step ? 0 : row >= 0 ? row : step[i];
+  constexpr int A = 16;   // accumulators per thread
+  // thread t sums blocks b0 + t + k FIN_NT into accumulator k mod A; the
+  // order depends only on b - b0
+  double acc[A];
 #pragma unroll
-    for (int k = 0; k < A; ++k) acc[k] = 0.0;
-    for (int base = b0 + threadIdx.x; base < b1; base += A * NT) {
-      double x[A];
+  for (int k = 0; k < A; ++k) acc[k] = 0.0;
+  for (int base = b0 + threadIdx.x; base < b1; base += A * FIN_NT) {
+    double x[A];
 #pragma unroll
-      for (int k = 0; k < A; ++k) {
-        const int b = base + k * NT;
-        x[k] = b < b1 ? part[(long)b * stride + j] : 0.0;
-      }
-#pragma unroll
-      for (int k = 0; k < A; ++k) acc[k] += x[k];
+    for (int k = 0; k < A; ++k) {
+      const int b = base + k * FIN_NT;
+      x[k] = b < b1 ? part[(long)b * stride + j] : 0.0;
     }
 #pragma unroll
-    for (int h = A / 2; h > 0; h /= 2)
-#pragma unroll
-      for (int k = 0; k < h; ++k) acc[k] += acc[k + h];
-    const double v = acc[0];
-    const double t = block_sum(v, sred);
-    if (threadIdx.x == 0) out[(row * row_stride + i) * stride + j] = t * scale[i];
-    __syncthreads();
+    for (int k = 0; k < A; ++k) acc[k] += x[k];
   }
-}
-
-// Advances the history row written by ldg_finalize_kernel (one thread).
-static __global__ void ldg_advance_kernel(int *step) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) *step += 1;
+#pragma unroll
+  for (int h = A / 2; h > 0; h /= 2)
+#pragma unroll
+    for (int k = 0; k < h; ++k) acc[k] += acc[k + h];
+  const double t = group_sum<FIN_NT>(acc[0], sred);
+  if (threadIdx.x == 0) out[(r * row_stride + i) * stride + j] = t * scale[i];
+  if (step && threadIdx.x == 0) step[i] = (int)r + 1;
 }
 
 // Taylor-Green initial state at the CGL nodes (solver.cpp:194-236).
