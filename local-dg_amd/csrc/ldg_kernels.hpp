@@ -131,16 +131,11 @@ struct InstDesc {
   int tb[3];             // brick of tb[0] x tb[1] x tb[2] blocks (x blocks, y rows, z planes)
   int nbrick[3];         // bricks per direction
   FastDiv div_bs, div_nb0, div_nb1, div_tb0, div_tb1;   // by tb0 tb1 tb2, nbrick[0], nbrick[1], tb[0], tb[1]
-  // spans (see span_elements): ncy strips of rows, cut into ncx columns of
-  // pieces of rows (ncx = 0: whole rows)
-  int ncx, ncy, nbr;                     // nbr: workgroups per row (pieces) or per strip plane (whole rows)
-  int rows, main_blocks;                 // whole rows: rows per strip, workgroups of all strips but the last
+  // spans (see span_elements): ncy strips of `rows` rows (the last one of the
+  // rest); nbr workgroups per strip plane, main_blocks in all strips but the last
+  int ncy, rows, nbr, main_blocks;
   FastDiv div_nx, div_ny, div_nz;
-  FastDiv div_row, div_nbr;              // by nz nbr (pieces) and nbr
-  FastDiv div_last;                      // by the last strip's workgroups per plane
-  int h0, w0;                            // strip heights h0, h0 + 1; column widths w0, w0 + 1
-  FastDiv div_ncx, div_ncy;
-  FastDiv div_col[2], div_pl[2][2], div_w[2];   // by h nz, h w, w
+  FastDiv div_nbr, div_last;             // by nbr, and by the last strip's workgroups per plane
   double ialpha[3];      // 2 / dx_l
   double dt;             // its time step
   PhysArgs ph;
@@ -171,92 +166,65 @@ __host__ __device__ inline void block_elements(const InstDesc &d, int E, int lbl
 // Elements of an instance's logical workgroup lbl in the span numbering of
 // the gradient and right-hand-side kernels: E consecutive elements kl ..
 // kl + ne - 1 (ne < E only at the end of a run; there are no empty
-// workgroups).  The mesh is cut into columns along z that are walked plane by
-// plane: strips of rows in y and, where rows are long, pieces of rows in x,
-// the strip heights (and piece widths, in workgroups) differing by at most
-// one.  The traces a workgroup gathers from its -y and -z neighbours were
-// read one row and one plane of the column earlier and are still in the XCD's
-// L2.  Whole rows of a strip are consecutive elements, so there a run is the
-// strip's part of a plane.
+// workgroups).  The mesh is cut into strips of whole rows in y that are walked
+// plane by plane along z; a strip's part of a plane is a run of consecutive
+// elements.  The traces a workgroup gathers from its -y and -z neighbours were
+// read one row and one plane of the strip earlier and are still in the XCD's
+// L2 (or, where a plane is large, in the memory-side cache).
 __host__ __device__ inline void span_elements(const InstDesc &d, int E, int lbl, int &kl, int &ne) {
-  int start, len, j;
-  if (d.ncx == 0) {
-    int st, z;
-    if (lbl < d.main_blocks) {
-      const int run = d.div_nbr.div(lbl);
-      j = lbl - run * d.nbr;
-      st = d.div_nz.div(run);
-      z = run - st * d.nz;
-    } else {
-      const int r = lbl - d.main_blocks, last = d.ny - (d.ncy - 1) * d.rows, nb = (last * d.nx + E - 1) / E;
-      st = d.ncy - 1;
-      z = d.div_last.div(r);
-      j = r - z * nb;
-    }
-    const int y0 = st * d.rows;
-    start = (z * d.ny + y0) * d.nx;
-    len = (d.ny - y0 < d.rows ? d.ny - y0 : d.rows) * d.nx;
+  int st, z, j;
+  if (lbl < d.main_blocks) {
+    const int run = d.div_nbr.div(lbl);
+    j = lbl - run * d.nbr;
+    st = d.div_nz.div(run);
+    z = run - st * d.nz;
   } else {
-    // strip i has rows floor(i ny / ncy) .. floor((i + 1) ny / ncy) - 1, so
-    // row y is in strip floor(((y + 1) ncy - 1) / ny); columns alike
-    const int st = d.div_ny.div((d.div_row.div(lbl) + 1) * d.ncy - 1);
-    const int y0 = d.div_ncy.div(st * d.ny), h = d.div_ncy.div((st + 1) * d.ny) - y0, hi = h - d.h0;
-    const int r = lbl - y0 * d.nz * d.nbr;
-    const int cx = d.div_nbr.div((d.div_col[hi].div(r) + 1) * d.ncx - 1);
-    const int b0 = d.div_ncx.div(cx * d.nbr), w = d.div_ncx.div((cx + 1) * d.nbr) - b0, wi = w - d.w0;
-    const int q = r - b0 * h * d.nz;
-    const int z = d.div_pl[hi][wi].div(q), p = q - z * h * w;
-    const int y = d.div_w[wi].div(p);
-    start = (z * d.ny + y0 + y) * d.nx;
-    len = d.nx;
-    j = b0 + p - y * w;
+    const int r = lbl - d.main_blocks, last = d.ny - (d.ncy - 1) * d.rows, nb = (last * d.nx + E - 1) / E;
+    st = d.ncy - 1;
+    z = d.div_last.div(r);
+    j = r - z * nb;
   }
-  kl = start + j * E;
+  const int y0 = st * d.rows;
+  const int len = (d.ny - y0 < d.rows ? d.ny - y0 : d.rows) * d.nx;
+  kl = (z * d.ny + y0) * d.nx + j * E;
   ne = len - j * E < E ? len - j * E : E;
 }
 
 // Sets d's span numbering (d.nx, ny, nz, nelem given) for workgroups of E
-// elements with n nodes per direction; returns the number of workgroups.  A
-// column's part of a plane is about 1 MB of FP64 state: with the face fluxes
-// the two planes in use at a time fill about the 4 MB of an XCD's L2.
-// Columns about as wide as deep cost the fewest reads across their sides
-// (64^3, p = 4, FP64: the gradient kernel reads 1.2x the state instead of
-// 1.8x with columns of single rows).
+// elements with n nodes per direction; returns the number of workgroups.  An
+// eighth of the rows to a strip: logical_block gives each of the 8 XCDs an
+// eighth of the workgroups, so that an XCD walks a strip of its own.  Below
+// 96 MB of state a strip's part of a plane is about 1 MB, a quarter of an
+// XCD's L2: the same time alone, and 0.5 % less in an ensemble, where an XCD
+// walks whole instances (48 of them, 2 steps 5.64 ms).  Measured against columns of about
+// 16 x 16 elements (p = 4, 1 MB of a plane) and against strips of 2 to 12 rows,
+// ms per step mixed / FP64: 64^3 p = 4 8 rows 6.28 / 10.15, columns 6.58 /
+// 10.39, 4 rows 6.46 / 10.28, 12 rows 6.41 / 10.21; 80^3 p = 4 12.2 / 19.7
+// against 13.2 / 20.3; 100^3 p = 2 6.43 / 10.0 against 6.93 / 10.6; 61x37x29
+// p = 4 1.65 / 2.54 against 1.75 / 2.64; planes of 10 MB (128 x 128) 6.31 / 9.88
+// against 6.67 / 10.1; 24^3, p = 5 2 %.  More rows where the runs' last
+// workgroups would be more than 2 % of all: 24^3, p = 2 has 2112 instead of
+// 1992 with 3 rows, 8.25 instead of 7.8 per CU, and took 9 % longer; 31x17x23, p = 3, mixed takes
+// 449 us for 2 steps instead of 506 with two strips of 9 and 8 rows.
 inline long make_spans(InstDesc &d, int n, int E) {
-  const double el = 8.0 * NSTATE * n * n * n, want = 1024.0 * 1024;
-  const double side = std::sqrt(want / el);               // elements
-  long nb;
-  if (d.nx <= 1.5 * side) {                               // whole rows
-    d.ncx = 0;
-    const int r = std::max(1, (int)(want / (el * d.nx)));
+  const double el = 8.0 * NSTATE * n * n * n;
+  long nbr, nl, main, nb;
+  int r = el * d.nx * d.ny * d.nz > 96e6 ? (d.ny + 7) / 8 : std::min(d.ny, std::max(1, (int)(1048576.0 / (el * d.nx))));
+  for (;; ++r) {
     d.ncy = (d.ny + r - 1) / r;
     d.rows = (d.ny + d.ncy - 1) / d.ncy;
     d.ncy = (d.ny + d.rows - 1) / d.rows;
     const int last = d.ny - (d.ncy - 1) * d.rows;
-    d.nbr = (int)(((long)d.rows * d.nx + E - 1) / E);
-    const long nl = ((long)last * d.nx + E - 1) / E, main = (long)(d.ncy - 1) * d.nz * d.nbr;
+    nbr = ((long)d.rows * d.nx + E - 1) / E;
+    nl = ((long)last * d.nx + E - 1) / E;
+    main = (long)(d.ncy - 1) * d.nz * nbr;
     nb = main + nl * d.nz;
-    if (nb > (1L << 30)) return nb;
-    d.main_blocks = (int)main;
-    d.div_last = make_fastdiv((int)nl);
-  } else {
-    d.nbr = (d.nx + E - 1) / E;
-    d.ncx = std::max(1, (int)(d.nx / side + 0.5));
-    d.ncx = std::min(d.ncx, d.nbr);
-    d.ncy = std::min(d.ny, std::max(1, (int)(d.ny / side + 0.5)));
-    nb = (long)d.nbr * d.ny * d.nz;
-    if (nb > (1L << 30)) return nb;
-    d.h0 = d.ny / d.ncy;
-    d.w0 = d.nbr / d.ncx;
-    d.div_row = make_fastdiv(d.nz * d.nbr);
-    d.div_ncx = make_fastdiv(d.ncx);
-    d.div_ncy = make_fastdiv(d.ncy);
-    for (int a = 0; a < 2; ++a) {
-      d.div_col[a] = make_fastdiv((d.h0 + a) * d.nz);
-      d.div_w[a] = make_fastdiv(d.w0 + a);
-      for (int b = 0; b < 2; ++b) d.div_pl[a][b] = make_fastdiv((d.h0 + a) * (d.w0 + b));
-    }
+    if (r >= d.ny || nb * E <= 1.02 * d.nx * d.ny * d.nz) break;
   }
+  if (nb > (1L << 30)) return nb;
+  d.nbr = (int)nbr;
+  d.main_blocks = (int)main;
+  d.div_last = make_fastdiv((int)nl);
   d.div_nbr = make_fastdiv(d.nbr);
   d.div_nx = make_fastdiv(d.nx);
   d.div_ny = make_fastdiv(d.ny);
@@ -676,8 +644,7 @@ __device__ inline T fluctuation(UT x, int s, double rho0, double E0) {
 // The three directions take turns in one set of face fields, with the own
 // traces and normal derivatives waiting in registers: against all three at
 // once the LDS footprint is 915 instead of 1620 values per element (p = 4;
-// 0.56 -> 0.41 ms mixed, 1.20 -> 0.89 ms FP64 at 64^3 with the column
-// numbering of span_elements).
+// 0.56 -> 0.41 ms mixed, 1.20 -> 0.89 ms FP64 at 64^3).
 //
 // Measured at 64^3, p = 4: mixed 0.41 ms (0.68 with the gradient at the face
 // nodes, 21 interpolated fields and lifted fluxes), bound by vector issue (91 %
