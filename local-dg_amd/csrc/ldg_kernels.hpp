@@ -196,16 +196,17 @@ __host__ __device__ inline void span_elements(const InstDesc &d, int E, int lbl,
 // eighth of the workgroups, so that an XCD walks a strip of its own.  Below
 // 96 MB of state a strip's part of a plane is about 1 MB, a quarter of an
 // XCD's L2: the same time alone, and 0.5 % less in an ensemble, where an XCD
-// walks whole instances (48 of them, 2 steps 5.64 ms).  Measured against columns of about
-// 16 x 16 elements (p = 4, 1 MB of a plane) and against strips of 2 to 12 rows,
-// ms per step mixed / FP64: 64^3 p = 4 8 rows 6.28 / 10.15, columns 6.58 /
-// 10.39, 4 rows 6.46 / 10.28, 12 rows 6.41 / 10.21; 80^3 p = 4 12.2 / 19.7
-// against 13.2 / 20.3; 100^3 p = 2 6.43 / 10.0 against 6.93 / 10.6; 61x37x29
-// p = 4 1.65 / 2.54 against 1.75 / 2.64; planes of 10 MB (128 x 128) 6.31 / 9.88
-// against 6.67 / 10.1; 24^3, p = 5 2 %.  More rows where the runs' last
-// workgroups would be more than 2 % of all: 24^3, p = 2 has 2112 instead of
-// 1992 with 3 rows, 8.25 instead of 7.8 per CU, and took 9 % longer; 31x17x23, p = 3, mixed takes
-// 449 us for 2 steps instead of 506 with two strips of 9 and 8 rows.
+// walks whole instances (48 of them, 2 steps 5.64 ms).  Measured against
+// columns of about 16 x 16 elements (p = 4, 1 MB of a plane) and against strips
+// of 2 to 12 rows, ms per step mixed / FP64: 64^3 p = 4 8 rows 6.28 / 10.15,
+// columns 6.58 / 10.39, 4 rows 6.46 / 10.28, 12 rows 6.41 / 10.21; 80^3 p = 4
+// 12.2 / 19.7 against 13.2 / 20.3; 100^3 p = 2 6.43 / 10.0 against 6.93 / 10.6;
+// 61x37x29 p = 4 1.65 / 2.54 against 1.75 / 2.64; planes of 10 MB (128 x 128)
+// 6.31 / 9.88 against 6.67 / 10.1; 24^3 p = 5 2 % less.
+// More rows where the runs' last workgroups would be more than 2 % of all:
+// 24^3, p = 2 has 2112 instead of 1992 with 3 rows, 8.25 instead of 7.8 per CU,
+// and took 9 % longer; 31x17x23, p = 3, mixed takes 449 us for 2 steps instead
+// of 506 with two strips of 9 and 8 rows.
 inline long make_spans(InstDesc &d, int n, int E) {
   const double el = 8.0 * NSTATE * n * n * n;
   long nbr, nl, main, nb;
