@@ -648,8 +648,8 @@ __device__ inline T fluctuation(UT x, int s, double rho0, double E0) {
 // 0.56 -> 0.41 ms mixed, 1.20 -> 0.89 ms FP64 at 64^3).
 //
 // Measured at 64^3, p = 4: mixed 0.41 ms (0.68 with the gradient at the face
-// nodes, 21 interpolated fields and lifted fluxes), bound by vector issue (91 %
-// of it); FP64 0.89 ms (1.22), vector issue and LDS at 52 % each.
+// nodes, 21 interpolated fields and lifted fluxes), bound by vector issue (95 %
+// of it); FP64 0.89 ms (1.22), vector issue and LDS at 53 % each.
 // ---------------------------------------------------------------------
 template <int N, int E, typename T>
 struct GradLds {
@@ -987,10 +987,10 @@ __global__ void __launch_bounds__(NT) ldg_nodal_grad_kernel(const UT *__restrict
 //   yi   I^-1 along y;   xi   along x
 //   epilogue: rate, running sum, next stage input (flat, coalesced)
 //
-// Measured at 64^3, p = 4, average of the four stages: mixed 1.18 ms (1.42
-// with sweeps at the nodes and one line of one variable per thread), 4.8 TB/s
+// Measured at 64^3, p = 4, average of the four stages: mixed 1.13 ms (1.42
+// with sweeps at the nodes and one line of one variable per thread), 5.1 TB/s
 // of HBM traffic where a streaming kernel with the same mix of reads and
-// writes reaches 5.4; FP64 1.57 ms (2.26), 4.8 TB/s, LDS busy for 57 %.
+// writes reaches 5.4; FP64 1.56 ms (2.26), 4.9 TB/s, LDS busy for 60 %.
 // ---------------------------------------------------------------------
 template <int N, int E, typename T>
 struct RhsLds {
