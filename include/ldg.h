@@ -120,7 +120,9 @@ int ldg_step(ldg_handle *h, double dt, int nsteps, double *ke);
    out[2] = enstrophy by Gauss quadrature of the interpolated state and LDG
    gradient (no reference counterpart).  There is no separate kinetic-energy
    or enstrophy entry point: the reference's per-step KE record (kes,
-   solver.cpp:437) is ldg_step's ke output, and this call covers the rest. */
+   solver.cpp:437) is ldg_step's ke output, and this call covers the rest.
+   A state that has no right-hand side (NaN or infinite values in any
+   variable, a face without a sound speed) is refused with LDG_ENONFINITE. */
 int ldg_diagnostics(ldg_handle *h, double out[3]);
 
 /* Average device time per launch of each kernel over nsteps RK4 steps of

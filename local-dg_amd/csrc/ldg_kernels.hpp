@@ -40,6 +40,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <limits>
 #include <type_traits>
 
 #include "symop.hpp"
@@ -411,6 +412,25 @@ __device__ inline void visc_face(const T w[5], T ir, const T v[3], const T *q, c
   for (int i = 0; i < 3; ++i)
     fv[i] = i == D ? fma_(b.mu, gv[i][D] + gv[D][i], -m23) : b.mu * (gv[i][D] + gv[D][i]);
   fv[3] = fma_(b.kappa, ge[D], fma_(v[2], fv[2], fma_(v[1], fv[1], v[0] * fv[0])));
+}
+
+// Whether the Roe flux between the traces wK and wN is a number: the squared
+// sound speed of their Roe average (the operations of face_flux_pair) is
+// positive and finite.
+template <typename T>
+__device__ inline bool roe_defined(const T wK[5], const T wN[5], const Bg<T> &b) {
+#pragma clang fp contract(off)
+  const T irN = rcp(b.rho0 + wN[0]), irK = rcp(b.rho0 + wK[0]);
+  const T vN[3] = {wN[1] * irN, wN[2] * irN, wN[3] * irN};
+  const T vK[3] = {wK[1] * irK, wK[2] * irK, wK[3] * irK};
+  const T HN = (b.H0 + wN[4] + pressure(wN, vN, b)) * irN, HK = (b.H0 + wK[4] + pressure(wK, vK, b)) * irK;
+  const T s = sqrt_((b.rho0 + wN[0]) * irK), iden = rcp(s + T(1));
+  T vt[3];
+#pragma unroll
+  for (int i = 0; i < 3; ++i) vt[i] = fma_(s, vN[i], vK[i]) * iden;
+  const T q2 = fma_(vt[2], vt[2], fma_(vt[1], vt[1], vt[0] * vt[0]));
+  const T c2 = b.gm1 * fma_(T(-0.5), q2, fma_(s, HN, HK) * iden);
+  return c2 > T(0) && c2 <= std::numeric_limits<T>::max();
 }
 
 template <typename T, int D>
@@ -1009,7 +1029,13 @@ struct RhsLds {
 };
 
 // DIAG: instead of the rate, the diagnostics of the state U to st.diag_part
-// (the nodal and the two Gauss-point sums), from the state and its gradient at the Gauss points; no face fluxes are read.
+// (the nodal and the two Gauss-point sums), from the state and its gradient at
+// the Gauss points; no face fluxes are read.  A sum is NaN if the state has no
+// right-hand side, although kinetic energy and enstrophy may be finite then
+// (a NaN or infinite energy, a negative density): the pressure has to be
+// finite at every Gauss point, and the Roe average of every face to have a
+// sound speed.  The traces for that come from the element's own lines and the
+// jumps, at the points the face kernel evaluates the flux at.
 template <int N, int E, typename T, typename UT, bool DIAG>
 __global__ void __launch_bounds__((Shape<N, E>::NTH), (RhsLds<N, E, T>::WAVES))
 ldg_rhs_kernel(const UT *__restrict__ U, const T *__restrict__ FF, LaunchArgs la,
@@ -1046,6 +1072,20 @@ ldg_rhs_kernel(const UT *__restrict__ U, const T *__restrict__ FF, LaunchArgs la
 
   // ---- x
   double dkn = 0.0, dke = 0.0, dens = 0.0;   // (DIAG)
+  bool defined = true;
+  auto face_defined = [&](const T (&own)[NSTATE], const T (&jump)[NSTATE]) {
+    T wK[NSTATE];
+#pragma unroll
+    for (int s = 0; s < NSTATE; ++s) wK[s] = own[s] - jump[s];
+    defined = defined && roe_defined<T>(wK, own, Bg<T>(d.ph));
+  };
+  // the trace of a line's polynomial at the - face from its Gauss values
+  auto trace = [&](const T (&x)[N]) -> T {
+    T r = T(0);
+#pragma unroll
+    for (int q = 0; q < N; ++q) r = fma_(op->eta[q] * T(opd->w[q]), x[q], r);
+    return r;
+  };
   if (act) {
     const double rho0 = d.ph.rho0, E0 = d.ph.E0;
     const UT *const ue = U + (k0 + e) * EV;
@@ -1172,26 +1212,31 @@ ldg_rhs_kernel(const UT *__restrict__ U, const T *__restrict__ FF, LaunchArgs la
       {
         const SymMat<N, T> Dx = uniform_load<SymMat<N, T>, T>(&op->Dg[0]);
         const Vec ax = uniform_load<Vec, T>(reinterpret_cast<const Vec *>(op->aeta[0]));
+        T own[NSTATE];
 #pragma unroll
         for (int s = 0; s < NSTATE; ++s) {
           const T *p = sA + bx + s * NN;
           T x[N];
 #pragma unroll
           for (int q = 0; q < N; ++q) x[q] = p[q];
+          if constexpr (DIAG) own[s] = trace(x);
           sym_apply<N, -1, T>(Dx, x, qx[s]);
 #pragma unroll
           for (int q = 0; q < N; ++q) qx[s][q] = fma_(ax.r[q], jx[s], qx[s][q]);
         }
+        if constexpr (DIAG) face_defined(own, jx);
       }
       {
         const SymMat<N, T> Dy = uniform_load<SymMat<N, T>, T>(&op->Dg[1]);
         const Vec ay = uniform_load<Vec, T>(reinterpret_cast<const Vec *>(op->aeta[1]));
+        T own[NSTATE];
 #pragma unroll
         for (int s = 0; s < NSTATE; ++s) {
           const T *p = sA + by + s * NN;
           T x[N];
 #pragma unroll
           for (int q = 0; q < N; ++q) x[q] = p[N * q];
+          if constexpr (DIAG) own[s] = trace(x);
           sym_apply<N, -1, T>(Dy, x, qy[s]);
 #pragma unroll
           for (int q = 0; q < N; ++q) {
@@ -1199,6 +1244,7 @@ ldg_rhs_kernel(const UT *__restrict__ U, const T *__restrict__ FF, LaunchArgs la
             if (!L::JB) sB[by + s * NN + N * q] = qy[s][q];
           }
         }
+        if constexpr (DIAG) face_defined(own, jy);
       }
     }
     __syncthreads();
@@ -1227,6 +1273,12 @@ ldg_rhs_kernel(const UT *__restrict__ U, const T *__restrict__ FF, LaunchArgs la
       }
     }
     const Bg<T> bg(d.ph);
+    if constexpr (DIAG) {
+      T own[NSTATE];
+#pragma unroll
+      for (int s = 0; s < NSTATE; ++s) own[s] = trace(ug[s]);
+      face_defined(own, jz);
+    }
 #pragma unroll
     for (int q = 0; q < N; ++q) {
       T w[NSTATE], g[NGRAD], F[NGRAD];
@@ -1247,6 +1299,8 @@ ldg_rhs_kernel(const UT *__restrict__ U, const T *__restrict__ FF, LaunchArgs la
         prim_grads<double>(ir, d.ph.E0 + (double)w[4], vv, gd, gv, ge);
         const double w1 = gv[2][1] - gv[1][2], w2 = gv[0][2] - gv[2][0], w3 = gv[1][0] - gv[0][1];
         const double wq = opd->w[a] * opd->w[b] * opd->w[q];
+        const T irt = rcp(bg.rho0 + w[0]), vt[3] = {w[1] * irt, w[2] * irt, w[3] * irt};
+        defined = defined && fabs(pressure(w, vt, bg)) <= std::numeric_limits<T>::max();
         dke += wq * 0.5 * ((double)w[1] * vv[0] + (double)w[2] * vv[1] + (double)w[3] * vv[2]);
         dens += wq * 0.5 * rho * (w1 * w1 + w2 * w2 + w3 * w3);
         continue;
@@ -1274,6 +1328,7 @@ ldg_rhs_kernel(const UT *__restrict__ U, const T *__restrict__ FF, LaunchArgs la
     }
   }
   if constexpr (DIAG) {
+    if (!defined) dke = std::numeric_limits<double>::quiet_NaN();
     const double n = group_sum<NTH>(dkn, sred), x = group_sum<NTH>(dke, sred), y = group_sum<NTH>(dens, sred);
     if (t == 0) {
       st.diag_part[3 * lb] = n;
