@@ -415,8 +415,7 @@ __device__ inline void visc_face(const T w[5], T ir, const T v[3], const T *q, c
 }
 
 // Whether the Roe flux between the traces wK and wN is a number: the squared
-// sound speed of their Roe average (the operations of face_flux_pair) is
-// positive and finite.
+// sound speed of their Roe average (face_flux_pair's c2) is positive and finite.
 template <typename T>
 __device__ inline bool roe_defined(const T wK[5], const T wN[5], const Bg<T> &b) {
 #pragma clang fp contract(off)
@@ -424,12 +423,12 @@ __device__ inline bool roe_defined(const T wK[5], const T wN[5], const Bg<T> &b)
   const T vN[3] = {wN[1] * irN, wN[2] * irN, wN[3] * irN};
   const T vK[3] = {wK[1] * irK, wK[2] * irK, wK[3] * irK};
   const T HN = (b.H0 + wN[4] + pressure(wN, vN, b)) * irN, HK = (b.H0 + wK[4] + pressure(wK, vK, b)) * irK;
-  const T s = sqrt_((b.rho0 + wN[0]) * irK), iden = rcp(s + T(1));
-  T vt[3];
+  const T s = sqrt_((b.rho0 + wN[0]) * irK);
+  T vt[3];   // times s + 1, as the velocities of the average
 #pragma unroll
-  for (int i = 0; i < 3; ++i) vt[i] = fma_(s, vN[i], vK[i]) * iden;
+  for (int i = 0; i < 3; ++i) vt[i] = fma_(s, vN[i], vK[i]);
   const T q2 = fma_(vt[2], vt[2], fma_(vt[1], vt[1], vt[0] * vt[0]));
-  const T c2 = b.gm1 * fma_(T(-0.5), q2, fma_(s, HN, HK) * iden);
+  const T c2 = fma_(T(-0.5), q2, fma_(s, HN, HK) * (s + T(1)));   // times (s + 1)^2 / (gamma - 1)
   return c2 > T(0) && c2 <= std::numeric_limits<T>::max();
 }
 
@@ -1073,19 +1072,6 @@ ldg_rhs_kernel(const UT *__restrict__ U, const T *__restrict__ FF, LaunchArgs la
   // ---- x
   double dkn = 0.0, dke = 0.0, dens = 0.0;   // (DIAG)
   bool defined = true;
-  auto face_defined = [&](const T (&own)[NSTATE], const T (&jump)[NSTATE]) {
-    T wK[NSTATE];
-#pragma unroll
-    for (int s = 0; s < NSTATE; ++s) wK[s] = own[s] - jump[s];
-    defined = defined && roe_defined<T>(wK, own, Bg<T>(d.ph));
-  };
-  // the trace of a line's polynomial at the - face from its Gauss values
-  auto trace = [&](const T (&x)[N]) -> T {
-    T r = T(0);
-#pragma unroll
-    for (int q = 0; q < N; ++q) r = fma_(op->eta[q] * T(opd->w[q]), x[q], r);
-    return r;
-  };
   if (act) {
     const double rho0 = d.ph.rho0, E0 = d.ph.E0;
     const UT *const ue = U + (k0 + e) * EV;
@@ -1197,7 +1183,29 @@ ldg_rhs_kernel(const UT *__restrict__ U, const T *__restrict__ FF, LaunchArgs la
         for (int s = 0; s < NSTATE; ++s) f[g][s] = (ffo + ((2 * l + g) * NSTATE + s) * plane)[(unsigned)t];
     }
   };
-  if constexpr (!DIAG) load_faces(fz, 2);
+  if constexpr (!DIAG) {
+    load_faces(fz, 2);
+  } else if (act) {
+    // the thread's point of the three - faces: a line's polynomial there is
+    // sum_q L_q(-1) u_q (32^3, p = 4, FP64: 114 us without this check, 130 with;
+    // taken from the sweeps below, whose lines these are, it is 125, but FP64 then
+    // needs 256 registers instead of 174 at p = 4 and spills at p = 5)
+    const Bg<T> bg(d.ph);
+#pragma unroll
+    for (int l = 0; l < 3; ++l) {
+      const T *const p = sA + (l == 0 ? bx : l == 1 ? by : bz);
+      const int stp = l == 0 ? 1 : l == 1 ? N : NF;
+      T wN[NSTATE], wK[NSTATE];
+#pragma unroll
+      for (int s = 0; s < NSTATE; ++s) {
+        wN[s] = T(0);
+#pragma unroll
+        for (int q = 0; q < N; ++q) wN[s] = fma_(op->eta[q] * T(opd->w[q]), p[s * NN + stp * q], wN[s]);
+        wK[s] = wN[s] - sJ[(l * NSTATE + s) * (E * NF) + t];
+      }
+      defined = defined && roe_defined<T>(wK, wN, bg);
+    }
+  }
   T jz[NSTATE];
   {
     T qx[NSTATE][N], qy[NSTATE][N];
@@ -1212,31 +1220,26 @@ ldg_rhs_kernel(const UT *__restrict__ U, const T *__restrict__ FF, LaunchArgs la
       {
         const SymMat<N, T> Dx = uniform_load<SymMat<N, T>, T>(&op->Dg[0]);
         const Vec ax = uniform_load<Vec, T>(reinterpret_cast<const Vec *>(op->aeta[0]));
-        T own[NSTATE];
 #pragma unroll
         for (int s = 0; s < NSTATE; ++s) {
           const T *p = sA + bx + s * NN;
           T x[N];
 #pragma unroll
           for (int q = 0; q < N; ++q) x[q] = p[q];
-          if constexpr (DIAG) own[s] = trace(x);
           sym_apply<N, -1, T>(Dx, x, qx[s]);
 #pragma unroll
           for (int q = 0; q < N; ++q) qx[s][q] = fma_(ax.r[q], jx[s], qx[s][q]);
         }
-        if constexpr (DIAG) face_defined(own, jx);
       }
       {
         const SymMat<N, T> Dy = uniform_load<SymMat<N, T>, T>(&op->Dg[1]);
         const Vec ay = uniform_load<Vec, T>(reinterpret_cast<const Vec *>(op->aeta[1]));
-        T own[NSTATE];
 #pragma unroll
         for (int s = 0; s < NSTATE; ++s) {
           const T *p = sA + by + s * NN;
           T x[N];
 #pragma unroll
           for (int q = 0; q < N; ++q) x[q] = p[N * q];
-          if constexpr (DIAG) own[s] = trace(x);
           sym_apply<N, -1, T>(Dy, x, qy[s]);
 #pragma unroll
           for (int q = 0; q < N; ++q) {
@@ -1244,7 +1247,6 @@ ldg_rhs_kernel(const UT *__restrict__ U, const T *__restrict__ FF, LaunchArgs la
             if (!L::JB) sB[by + s * NN + N * q] = qy[s][q];
           }
         }
-        if constexpr (DIAG) face_defined(own, jy);
       }
     }
     __syncthreads();
@@ -1273,12 +1275,6 @@ ldg_rhs_kernel(const UT *__restrict__ U, const T *__restrict__ FF, LaunchArgs la
       }
     }
     const Bg<T> bg(d.ph);
-    if constexpr (DIAG) {
-      T own[NSTATE];
-#pragma unroll
-      for (int s = 0; s < NSTATE; ++s) own[s] = trace(ug[s]);
-      face_defined(own, jz);
-    }
 #pragma unroll
     for (int q = 0; q < N; ++q) {
       T w[NSTATE], g[NGRAD], F[NGRAD];
