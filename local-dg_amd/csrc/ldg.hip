@@ -546,7 +546,8 @@ int create_impl(const ldg_config *cfg, const ldg_instance *insts, int n, ldg_han
     g.cgrad = g.crhs = default_cand(g.n, h->mixed, g.K);
     std::vector<double> sc;
     for (int idx : g.members) sc.push_back(ke_scale(h->cfg, h->inst[idx]));
-    if (hipMalloc((void **)&g.ke_part, sizeof(double) * (maxblk + 1)) != hipSuccess ||
+    const long nke = ke_per_element(g.n) ? g.K : maxblk;
+    if (hipMalloc((void **)&g.ke_part, sizeof(double) * (nke + 1)) != hipSuccess ||
         hipMalloc((void **)&g.diag_part, sizeof(double) * 3 * (maxblk + 1)) != hipSuccess ||
         hipMalloc((void **)&g.d_scale, sizeof(double) * sc.size()) != hipSuccess) {
       h->err = "device allocation failed (partials)";
@@ -645,7 +646,8 @@ int rk4_step(ldg_handle *h, bool ke, int row, bool in32, bool out32) {
     }
     if (ke) {
       const Tiling &t = g.tile[g.rhs[g.crhs]];
-      hipLaunchKernelGGL(ldg_finalize_kernel, dim3(g.members.size()), dim3(FIN_NT), 0, h->stream,
+      hipLaunchKernelGGL(ke_per_element(g.n) ? ldg_finalize_kernel<true> : ldg_finalize_kernel<false>,
+                         dim3(g.members.size()), dim3(FIN_NT), 0, h->stream,
                          (const double *)g.ke_part, 1, (const InstDesc *)t.d_inst, (int)h->inst.size(),
                          (const double *)g.d_scale, h->ke_hist + first, row, h->d_step + first);
       HIPCHECK(h, hipGetLastError());
@@ -1043,7 +1045,7 @@ int ldg_instance_diagnostics(ldg_handle *h, int i, double out[3]) {
     const int rc = launch_rhs(h, g, state_in(g.u), st, 0);
     if (rc) return rc;
     const Tiling &t = g.tile[g.rhs[0]];
-    hipLaunchKernelGGL(ldg_finalize_kernel, dim3(g.members.size(), 3), dim3(FIN_NT), 0, h->stream,
+    hipLaunchKernelGGL(ldg_finalize_kernel<false>, dim3(g.members.size(), 3), dim3(FIN_NT), 0, h->stream,
                        (const double *)g.diag_part, 3, (const InstDesc *)t.d_inst, ni, (const double *)g.d_scale,
                        h->scal + 3 * first, 0, (int *)nullptr);
     HIPCHECK(h, hipGetLastError());

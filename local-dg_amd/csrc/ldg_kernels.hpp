@@ -609,6 +609,24 @@ __device__ inline double group_sum(double v, double *sw) {
   return v;
 }
 
+// Kinetic-energy partial sums: one per workgroup, or at p = 5 one per element.
+// Without the autotuner a launch takes its kernels by its number of elements
+// (an ensemble's together), and an instance's energy must not depend on which:
+// at p <= 4 both take the same elements to a workgroup and number them alike,
+// at p = 5 the large kernel takes 3 and the wave kernel 1.
+__host__ __device__ constexpr bool ke_per_element(int n) { return n == 6; }
+
+// Sum over an element of the values its N^2 lines left at v, by one wave (the
+// butterfly of group_sum, idle lanes zero).
+template <int N>
+__device__ inline double element_sum(const double *v) {
+  const int l = threadIdx.x & 63;
+  double x = l < N * N ? v[l] : 0.0;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o, 64);
+  return x;
+}
+
 // Face-flux array FF, T: 30 planes (direction 2 d + side, state), each of
 // the launch's elements x N^2 face Gauss points: the fluxes times a_d, side 0
 // the element's own -d face, side 1 its +d face (written by the +d
@@ -1049,12 +1067,9 @@ ldg_rhs_kernel(const UT *__restrict__ U, const T *__restrict__ FF, LaunchArgs la
   const int t = threadIdx.x;
   int kl, ne;
   const InstDesc &d = block_span(la, lb, E, kl, ne);
-  if (ne <= 0) {                      // padding block: empty partial sums
-    if (t == 0 && st.ke_part) st.ke_part[lb] = 0.0;
-    if (DIAG && t == 0)
-      for (int j = 0; j < 3; ++j) st.diag_part[3 * lb + j] = 0.0;
-    return;
-  }
+  // (no span is empty; without this line the compiler moves the loads up and
+  // the mixed kernel takes 144 instead of 140 registers, 0.5 % more at 64^3, p = 4)
+  if (ne <= 0) return;
   const long k0 = d.elem_off + kl;
   const int e = t / NF, ab = t - e * NF, b = ab / N, a = ab - b * N;
   const bool act = e < ne;
@@ -1513,30 +1528,43 @@ ldg_rhs_kernel(const UT *__restrict__ U, const T *__restrict__ FF, LaunchArgs la
         kel += opd->w[a] * opd->w[b] * opd->w[q] * fma_(m3, m3, fma_(m2, m2, m1 * m1)) / (2.0 * rho);
       }
     }
-    const double x = group_sum<NTH>(kel, sred);
-    if (t == 0) st.ke_part[lb] = x;
+    if constexpr (ke_per_element(N)) {
+      __syncthreads();
+      if (act) md[t] = kel;
+      __syncthreads();
+      for (int i = t >> 6; i < ne; i += NTH / 64) {
+        const double x = element_sum<N>(md + i * NF);
+        if ((t & 63) == 0) st.ke_part[k0 + i] = x;
+      }
+    } else {
+      const double x = group_sum<NTH>(kel, sred);
+      if (t == 0) st.ke_part[lb] = x;
+    }
   }
 }
 
-// Ordered per-instance sums of per-workgroup partials, one workgroup per
-// instance i and partial j of `stride`: out[(row * row_stride + i) * stride + j] = scale_i * (sum over
-// the instance's blocks b of part[b * stride + j]).  With `step` a row of a
+// Ordered per-instance sums of partials, one workgroup per instance i and
+// partial j of `stride`: out[(row * row_stride + i) * stride + j] = scale_i * (sum
+// over the instance's partials b of part[b * stride + j]).  The partials are the
+// instance's workgroups' or (BY_ELEM) its elements'.  With `step` a row of a
 // history: row >= 0 is the row, row < 0 (graph replays) the instance's own
 // counter step[i], which is left at the row after it; without it row 0.
 //
 // One workgroup reads every partial, so what counts is the loads in flight:
 // 128 KB (64^3, p = 4: 131,072 partials in 27 us; 33 with 256 threads).
 constexpr int FIN_NT = 1024;
+template <bool BY_ELEM>
 static __global__ void __launch_bounds__(FIN_NT) ldg_finalize_kernel(const double *__restrict__ part, int stride,
                                                             const InstDesc *__restrict__ inst, int row_stride,
                                                             const double *__restrict__ scale, double *__restrict__ out,
                                                             int row, int *__restrict__ step) {
   __shared__ double sred[FIN_NT / 64];
   const int i = blockIdx.x, j = blockIdx.y;
-  const int b0 = inst[i].block_off, b1 = b0 + inst[i].nblocks;
+  const int b0 = BY_ELEM ? (int)inst[i].elem_off : inst[i].block_off;
+  const int b1 = b0 + (BY_ELEM ? (int)inst[i].nelem : inst[i].nblocks);
   const long r = !step ? 0 : row >= 0 ? row : step[i];
   constexpr int A = 16;   // accumulators per thread
-  // thread t sums blocks b0 + t + k FIN_NT into accumulator k mod A; the
+  // thread t sums partials b0 + t + k FIN_NT into accumulator k mod A; the
   // order depends only on b - b0
   double acc[A];
 #pragma unroll

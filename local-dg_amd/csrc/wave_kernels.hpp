@@ -20,8 +20,9 @@
 // waves hold 50 lines at p = 4, every wave repeats the index arithmetic).
 //
 // The arithmetic of every value is that of ldg_kernels.hpp, operation by
-// operation (and the kinetic-energy sum is taken in the same order), so a
-// launch's choice of kernels does not show in its results.
+// operation, and the kinetic-energy sum is taken in the same order (from the
+// same partial sums: ke_per_element), so a launch's choice between these
+// kernels and ldg_kernels.hpp's default does not show in its results.
 #pragma once
 
 #include "ldg_kernels.hpp"
@@ -249,10 +250,7 @@ ldg_rhs_wave_kernel(const UT *__restrict__ U, const T *__restrict__ FF, LaunchAr
   const int t = threadIdx.x, l = t & 63, s = __builtin_amdgcn_readfirstlane(t >> 6);
   int kl, ne;
   const InstDesc &d = block_span(la, lb, E, kl, ne);
-  if (ne <= 0) {
-    if (t == 0 && st.ke_part) st.ke_part[lb] = 0.0;
-    return;
-  }
+  if (ne <= 0) return;
   const long k0 = d.elem_off + kl;
   const int e = l / NF, ab = l - e * NF, b = ab / N, a = ab - b * N;
   const bool act = e < ne;
@@ -498,7 +496,8 @@ ldg_rhs_wave_kernel(const UT *__restrict__ U, const T *__restrict__ FF, LaunchAr
         }
       }
       const double x = group_sum<64>(kel, nullptr);
-      if (t == 0) st.ke_part[lb] = x;
+      static_assert(E == 1 || !ke_per_element(N), "one element to a partial sum");
+      if (t == 0) st.ke_part[ke_per_element(N) ? k0 : lb] = x;
     }
   }
 }
