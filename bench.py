@@ -213,6 +213,14 @@ def timed_run(ldg_amd, p, nx, prec, steps, warmup, autotune=True):
     return g, dt, wall, np.concatenate([ke_w, ke]), tiling
 
 
+def tiling_record(t):
+    """The autotuner's (p, gradient, rhs) as elements per workgroup, with the
+    kernels it took (the small-mesh ones are reported negative)."""
+    return {"p": t[0], "grad_elements_per_workgroup": abs(t[1]), "rhs_elements_per_workgroup": abs(t[2]),
+            "grad_kernel": "ldg_grad_wave_kernel" if t[1] < 0 else "ldg_grad_kernel",
+            "rhs_kernel": "ldg_rhs_wave_kernel" if t[2] < 0 else "ldg_rhs_kernel"}
+
+
 def ensemble_bench(ldg_amd, args):
     """Seeded ensemble of uneven Taylor-Green instances (ldg_ensemble_sample):
     mixed precision, tilings autotuned, timed with eager launches and with
@@ -440,8 +448,7 @@ def main():
                    "ldg_rhs_kernel": {"avg_ms": v["kt"]["rhs_ms"],
                                       "alg_GBs": alg_bytes(dof, name == "mixed", p)[1] / (v["kt"]["rhs_ms"] * 1e-3) / 1e9},
                    "ms_per_step": v["wall"] / args.steps * 1e3,
-                   "tiling": {"p": v["tiling"][0][0], "grad_elements_per_workgroup": v["tiling"][0][1],
-                              "rhs_elements_per_workgroup": v["tiling"][0][2]} if v["tiling"] else "default"}
+                   "tiling": tiling_record(v["tiling"][0]) if v["tiling"] else "default"}
             for name, v in runs.items()},
     }
     if not args.no_cpu:

@@ -181,11 +181,13 @@ int ldg_ensemble_step(ldg_handle *h, const double *dt, int nsteps, double *ke);
    launched eagerly).  Results are identical. */
 int ldg_set_graph(ldg_handle *h, int enable);
 
-/* Times the candidate elements-per-workgroup tilings of each kernel on the
-   resident state and keeps the fastest per order.  The state is not
+/* Times the candidates of each kernel (elements-per-workgroup tilings, and
+   the kernels for small meshes, which give each variable a wave of its own)
+   on the resident state and keeps the fastest per order.  The state is not
    changed.  If chosen is not NULL it receives, per order group in order of
    first appearance, (p, elements per workgroup of the gradient kernel, of
-   the right-hand-side kernel): 3 ints per group, at most 5 groups. */
+   the right-hand-side kernel), the latter two negative where the kernel for
+   small meshes was chosen: 3 ints per group, at most 5 groups. */
 int ldg_autotune(ldg_handle *h, int *chosen);
 
 /* ------------------------------------------------------------------------

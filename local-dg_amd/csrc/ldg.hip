@@ -80,6 +80,10 @@ int cand_e(int n, bool rhs, int c) {
   return 1;
 }
 
+// What the autotuner reports of candidate c: its elements per workgroup, the
+// wave kernels' negative (at most orders candidate 0 has as many).
+int reported_cand(int n, bool rhs, int c) { return c == kWaveCand ? -cand_e(n, rhs, c) : cand_e(n, rhs, c); }
+
 // The candidate used unless the autotuner chose one, for a launch over K
 // elements: the wave kernels as long as about all their workgroups are
 // resident at once (3 to 4 per CU of 256 in FP64, 6 to 8 in the mixed path, by
@@ -1125,8 +1129,8 @@ int ldg_autotune(ldg_handle *h, int *chosen) {
     }
     if (chosen) {
       chosen[3 * gi] = g.n - 1;
-      chosen[3 * gi + 1] = cand_e(g.n, false, g.cgrad);
-      chosen[3 * gi + 2] = cand_e(g.n, true, g.crhs);
+      chosen[3 * gi + 1] = reported_cand(g.n, false, g.cgrad);
+      chosen[3 * gi + 2] = reported_cand(g.n, true, g.crhs);
     }
     ++gi;
   }

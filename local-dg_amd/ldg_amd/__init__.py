@@ -240,8 +240,9 @@ class LDG:
         self._check(self._lib.ldg_set_graph(self._h, int(bool(enable))))
 
     def autotune(self):
-        """Pick the fastest tiling per kernel (ldg_autotune); returns
-        [(p, elements per workgroup of the gradient, of the rhs), ...]."""
+        """Pick the fastest candidate per kernel (ldg_autotune); returns
+        [(p, elements per workgroup of the gradient, of the rhs), ...],
+        negative where the kernel for small meshes was picked."""
         out = (ctypes.c_int * 15)()
         self._check(self._lib.ldg_autotune(self._h, out))
         ng = len({p for p in getattr(self, "orders", [self.p])})
