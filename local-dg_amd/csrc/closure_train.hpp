@@ -21,8 +21,10 @@
 // The arithmetic is that of the layer-by-layer kernels (closure_kernels.hpp):
 // operands rounded to BF16 at the same places, the same matrix instructions
 // over k in the same order, the same FP32 operations in Adam, bias gradients
-// summed sample by sample.  Trained parameters are equal bit by bit; only the
-// loss record is summed in another order (FP64).
+// summed sample by sample.  Trained parameters came out equal bit by bit to
+// those kernels' (3 epochs on 700 to 20,480 samples, batches of 32, 129, 300
+// and 2048, with and without weights); only the loss record is summed in
+// another order (FP64).
 #pragma once
 
 #include "closure_kernels.hpp"

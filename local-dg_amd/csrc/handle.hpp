@@ -61,7 +61,7 @@ struct Group {
   double *u = nullptr, *acc = nullptr, *k = nullptr;
   void *ua = nullptr, *ub = nullptr;  // stage inputs: FP64 state, or FP32 fluctuations in the mixed path
   void *q = nullptr;
-  void *ff = nullptr;     // face fluxes written by the gradient kernel, lifted by the rhs kernel
+  void *ff = nullptr;     // face fluxes written by the gradient kernel, subtracted by the rhs kernel
   double *ke_part = nullptr, *diag_part = nullptr, *d_scale = nullptr;
   void *ops = nullptr;
   void *sops = nullptr;   // the kernels' operator images (GImage), one per member

@@ -87,12 +87,19 @@ int reported_cand(int n, bool rhs, int c) { return c == kWaveCand ? -cand_e(n, r
 // The candidate used unless the autotuner chose one, for a launch over K
 // elements: the wave kernels as long as about all their workgroups are
 // resident at once (3 to 4 per CU of 256 in FP64, 6 to 8 in the mixed path, by
-// LDS).  Measured, us per RK4 step, wave kernels / the others: FP64 p = 4 65 /
-// 111 at 8^3 (256 workgroups), 157 / 165 at 12^3 (864), 202 / 184 at 14^3
-// (1372); p = 2 55 / 89 at 8^3, 103 / 108 at 16^3 (586), 154 / 149 at 20^3
-// (1143).  Mixed p = 4 56 / 96 at 8^3, 153 / 155 at 16^3 (2048), 387 / 357 at
-// 24^3 (6912); p = 2 50 / 78 at 8^3, 99 / 113 at 20^3 (1143), 141 / 133 at 24^3
-// (1975).
+// LDS).  Measured, us per RK4 step, wave kernels / the others (workgroups of the
+// wave kernels), on either side of where they are equal:
+//   FP64  p = 1  61 / 84 (500), 97 / 97 (864), 134 / 123 (1372)
+//         p = 2  99 / 105 (586), 133 / 119 (834), 149 / 145 (1143)
+//         p = 3  113 / 130 (686), 154 / 144 (844), 162 / 153 (1024)
+//         p = 4  153 / 162 (864), 168 / 173 (1099), 198 / 183 (1372)
+//         p = 5  115 / 145 (729), 161 / 189 (1000), 197 / 193 (1331)
+//   mixed p = 1  84 / 92 (1372), 106 / 103 (2048)
+//         p = 2  95 / 108 (1143), 137 / 128 (1975)
+//         p = 3  114 / 126 (1458), 148 / 143 (2000)
+//         p = 4  115 / 135 (1372), 150 / 153 (2048)
+//         p = 5  133 / 151 (1728), 156 / 157 (2197), 180 / 172 (2744)
+// Well below the line the wave kernels take 0.45 to 0.6 of the others' time.
 int default_cand(int n, bool mixed, long K) {
   const int e = cand_e(n, true, kWaveCand);
   return (K + e - 1) / e <= (mixed ? 1800 : 900) ? kWaveCand : 0;
@@ -540,7 +547,7 @@ int create_impl(const ldg_config *cfg, const ldg_instance *insts, int n, ldg_han
     }
     // face fluxes: per element 3 directions x 2 sides x 5 states x n^2 face nodes
     const int wb = h->mixed ? (int)sizeof(float) : (int)sizeof(double);
-    if (hipMalloc(&g.ff, (size_t)g.K * 6 * ff_chunk(g.n, wb) * wb) != hipSuccess) {
+    if (hipMalloc(&g.ff, (size_t)g.K * 6 * ff_chunk(g.n) * wb) != hipSuccess) {
       h->err = "device allocation failed (face fluxes)";
       return bad(LDG_ENOMEM);
     }
@@ -1361,7 +1368,7 @@ extern "C" int ldg_rhs_noalloc(const ldg_config *cfg, const double *u, double *k
   const int n = in.p + 1;
   // the face fluxes (6 chunks of 5 n^2 values per element)
   const int wb = cfg->precision == LDG_MIXED ? 4 : 8;
-  const double qbytes = (double)in.K * 6 * ff_chunk(n, wb) * wb;
+  const double qbytes = (double)in.K * 6 * ff_chunk(n) * wb;
   if (kScrFF + qbytes > (double)LDG_NOALLOC_SCRATCH_BYTES) {
     char msg[256];
     std::snprintf(msg, sizeof(msg),

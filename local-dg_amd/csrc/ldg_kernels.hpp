@@ -7,7 +7,8 @@
 //                    elements of every face (solver.cpp:643-698, 750-814,
 //                    891-921, 1194-1374)
 //   ldg_rhs_kernel   the volume gradient and volume integrals, minus the
-//                    face terms, inverse mass and the fused RK4 stage
+//                    face terms, the return to the nodes (with W^-1 in the
+//                    operators: the inverse mass) and the fused RK4 stage
 //                    epilogue (solver.cpp:510-535 and 410-434)
 // Both stage a block of E consecutive elements in LDS, work in 1D "lines"
 // of N = p+1 values owned by one thread (in-place sum-factorised sweeps in
@@ -16,10 +17,11 @@
 // straight from HBM (the on-device form of the single-rank halo exchange,
 // solver.cpp:929-998).
 //
-// Precision: the state, the RK4 combination, the inverse mass and every
-// reduction are FP64.  The interpolation, flux evaluation and test-function
-// contractions run in the compute type T (double for the plain path, float
-// for the mixed path), on fluctuations about the constant background
+// Precision: the state, the RK4 combination, the return to the nodes (I^-1
+// along three directions) and every reduction are FP64.  The interpolation,
+// flux evaluation, derivatives and face terms (Dh, eta, which hold the
+// inverse mass's W^-1) run in the compute type T (double for the plain path,
+// float for the mixed path), on fluctuations about the constant background
 // (rho0, 0, 0, 0, E0 = p0/(gamma-1)): the background is subtracted in FP64
 // when U is loaded (exact, both values are close), so the O(1/M0^2) part of
 // the energy never enters the T-precision arithmetic.  A constant state is a
@@ -69,9 +71,6 @@ struct Ops {
 
 struct MeshArgs {
   int nx, ny, nz;
-  long nelem;
-  int nblocks;           // logical workgroups (ceil(nelem / E))
-  int per_xcd;           // ceil(nblocks / 8)
   double ialpha[3];      // 2 / dx_l
 };
 
@@ -243,8 +242,8 @@ struct LaunchArgs {
 };
 
 // Workgroups are dispatched round-robin over the 8 XCDs; give each XCD a
-// contiguous range of element blocks so that face neighbours in x and y
-// share that XCD's L2.  Returns -1 for padding workgroups.
+// contiguous range of element blocks so that face neighbours share that
+// XCD's L2.  Returns -1 for padding workgroups.
 __device__ inline int logical_block(const LaunchArgs &la) {
   const int b = blockIdx.x;
   const int lb = (b & 7) * la.per_xcd + (b >> 3);
@@ -269,7 +268,6 @@ __device__ inline const InstDesc &block_instance(const LaunchArgs &la, int lb, M
                                                  int &ne) {
   const InstDesc &d = la.inst[la.blk_inst ? la.blk_inst[lb] : 0];
   m.nx = d.nx; m.ny = d.ny; m.nz = d.nz;
-  m.nelem = d.nelem;
   m.ialpha[0] = d.ialpha[0]; m.ialpha[1] = d.ialpha[1]; m.ialpha[2] = d.ialpha[2];
   block_elements(d, E, lb - d.block_off, ec, ne);
   kl = ec[0] + (long)d.nx * (ec[1] + (long)d.ny * ec[2]);
@@ -296,16 +294,6 @@ __device__ inline void fill_neighbors(const MeshArgs &m, const int ec[3], long o
     nb[e][f] = off + x + (long)m.nx * (y + (long)m.ny * z);
   }
 }
-
-// node index of position i along direction d in the line with face
-// coordinates (a, b): x-lines (iy, iz), y-lines (ix, iz), z-lines (ix, iy)
-// -- the same (a, b) order as the reference's face map (mesh.cpp:428-501).
-template <int N>
-__device__ inline int line_base(int d, int a, int b) {
-  return d == 0 ? (N * a + N * N * b) : d == 1 ? (a + N * N * b) : (a + N * b);
-}
-template <int N>
-__device__ inline int line_stride(int d) { return d == 0 ? 1 : d == 1 ? N : N * N; }
 
 // ---------------------------------------------------------------------
 // Pointwise physics in fluctuation form, textbook forms of
@@ -633,7 +621,7 @@ __device__ inline double element_sum(const double *v) {
 // neighbour's workgroup, see ldg_grad_kernel).  Plane-major, so that a
 // workgroup's threads (element, point) read and write each plane in one
 // contiguous piece.
-__host__ __device__ constexpr int ff_chunk(int n, int /*bytes*/) { return NSTATE * n * n; }
+__host__ __device__ constexpr int ff_chunk(int n) { return NSTATE * n * n; }
 
 // Coordinates of element kl of an instance.
 __host__ __device__ inline void element_coords(const InstDesc &d, int kl, int c[3]) {

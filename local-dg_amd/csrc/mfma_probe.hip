@@ -1,16 +1,19 @@
-// mfma_probe.hip -- the rhs kernel's y/z test-function contraction at p = 4
-// in three forms, to measure whether matrix cores pay for it (a measurement,
-// not part of the solver).
+// mfma_probe.hip -- the y/z test-function contraction of the nodal scheme at
+// p = 4 in three forms, to measure whether matrix cores pay for such sweeps (a
+// measurement, not part of the solver).
 //
 // Per element (N = 5 nodes per direction, node x + 5 y + 25 z), from the 15
 // weighted flux fields F_x, F_y, F_z (5 states each):
 //   O_x = (I^T (x) I^T) F_x                    over (y, z), every x and state
 //   O_g = (D^T (x) I^T) F_y + (I^T (x) D^T) F_z
-// which is what ldg_rhs_kernel's z and y contraction sweeps compute
-// (solver.cpp:701-741, 817-864, restated in sum-factorised form).  As in
-// the solver, the results overwrite F_x and F_y in the element's LDS buffer.
-//   variant 0: vector ALU, the solver's two in-place sum-factorised sweeps
-//              with the even/odd split
+// (solver.cpp:701-741, 817-864, restated in sum-factorised form), the sweeps
+// with the most work per value when the operators act on nodal values.
+// ldg_rhs_kernel works at the Gauss points, where each flux field is swept
+// once, along its own direction: less vector work on the same values, for the
+// same dense slab product.  The results overwrite F_x and F_y in the element's
+// LDS buffer.
+//   variant 0: vector ALU, two in-place sum-factorised sweeps with the even/odd
+//              split
 //   variant 1: v_mfma_f32_32x32x2_f32 on the dense 25x25 slab operators
 //              (FP32 inputs)
 //   variant 2: v_mfma_f32_32x32x16_f16 on the slab operators with every

@@ -3,8 +3,8 @@
 // The 1D operators of the tensor-product element live on node sets that
 // are symmetric about the element centre (Chebyshev-Gauss-Lobatto nodes,
 // Gauss points), so every operator A used by the sweeps satisfies
-//   A[N-1-q][N-1-j] = S A[q][j],   S = +1 (interpolation, its transpose, the
-//                                  inverse mass) or -1 (differentiation).
+//   A[N-1-q][N-1-j] = S A[q][j],   S = +1 (interpolation and its inverse) or
+//                                  -1 (differentiation).
 // With e_j = v_j + v_{N-1-j} and o_j = v_j - v_{N-1-j} (j < H = N/2) and, for
 // odd N, the middle value v_m (m = H):
 //   (A v)_q = sum_j P[q][j] e_j + C[q] v_m + sum_j R[q][j] o_j
@@ -15,12 +15,12 @@
 // and the part F that flips,
 //   (A v)_q = K_q + F_q,   (A v)_{N-1-q} = K_q - F_q,   (A v)_m = K_m,
 // so only rows q < ceil(N/2) are evaluated: N = 5 takes 21 operations per
-// line instead of 25, N = 6 30 instead of 36, and a sum of two operators
-// (D^T a + I^T b, the fused contraction sweeps) 38 instead of 50 at N = 5.
-// At N = 3, 4 the operation count is about the same, but the operator needs
-// half the coefficients (registers and LDS loads): measured rhs -15 % at
-// N = 4 and -4 % at N = 3 (mixed).  At N = 2 the split costs more and the
-// plain product is used.  This is the even-odd decomposition of
+// line instead of 25, N = 6 30 instead of 36.  At N = 3, 4 the operation count
+// is about the same, but the operator needs half the coefficients, which the
+// solver's kernels keep in scalar registers.  At N = 2 the split costs more
+// and the plain product is used.  A sum of two operators (sym_apply2; 38
+// operations instead of 50 at N = 5) is what the matrix-core measurement
+// compares with.  This is the even-odd decomposition of
 // spectral-element codes (Solomonoff, "A fast algorithm for spectral
 // differentiation", J. Comput. Phys. 98, 1992; Kopriva, "Implementing
 // Spectral Methods for Partial Differential Equations", 2009).
@@ -88,7 +88,8 @@ inline void symmetrize(double (&A)[N][N], int S) {
     for (int j = 0; j < N; ++j) A[q][j] = B[q][j];
 }
 
-// Coefficient registers of one operator (loaded once per phase from LDS).
+// Coefficient registers of one operator (the matrix-core measurement loads
+// them from LDS).
 template <int N, typename T>
 struct SymReg {
   SymMat<N, T> m;
@@ -162,7 +163,7 @@ __host__ __device__ inline void sym_apply(const SymMat<N, T> &M, const T (&v)[N]
   }
 }
 
-// out = A1 v1 + A2 v2   (the fused contraction sweeps)
+// out = A1 v1 + A2 v2
 template <int N, int S1, int S2, typename T>
 __host__ __device__ inline void sym_apply2(const SymMat<N, T> &M1, const T (&v1)[N], const SymMat<N, T> &M2,
                                            const T (&v2)[N], T (&out)[N]) {

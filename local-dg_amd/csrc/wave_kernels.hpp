@@ -14,8 +14,8 @@
 // about a fifth as long.
 //
 // Measured, us per RK4 step (8 of these launches and the kinetic energy), these
-// kernels / ldg_kernels.hpp's: FP64 8^3 p = 2 55 / 89, 8^3 p = 4 65 / 111, mixed
-// 8^3 p = 4 56 / 96.  What is left there is the launches themselves (about 5 us
+// kernels / ldg_kernels.hpp's: FP64 8^3 p = 2 51 / 86, 8^3 p = 4 61 / 108, mixed
+// 8^3 p = 4 54 / 94, 8^3 p = 5 64 / 115.  What is left there is the launches themselves (about 5 us
 // each) and HBM latency.  On large meshes these kernels take longer (64-lane
 // waves hold 50 lines at p = 4, every wave repeats the index arithmetic).
 //
