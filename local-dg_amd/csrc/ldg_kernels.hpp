@@ -1074,8 +1074,8 @@ __global__ void __launch_bounds__(NT) ldg_nodal_grad_kernel(const UT *__restrict
 //
 // Measured at 64^3, p = 4, average of the four stages: mixed 1.13 ms (1.42
 // with sweeps at the nodes and one line of one variable per thread), 5.1 TB/s
-// of HBM traffic where a streaming kernel with the same mix of reads and
-// writes reaches 5.4; FP64 1.56 ms (2.26), 4.9 TB/s, LDS busy for 60 %.
+// of HBM traffic where a streaming kernel with two reads to a write
+// reaches 5.8; FP64 1.56 ms (2.26), 4.9 TB/s, LDS busy for 60 %.
 // ---------------------------------------------------------------------
 template <int N, int E, typename T>
 struct RhsLds {
