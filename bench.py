@@ -7,7 +7,7 @@ reduction) of the compressible Taylor-Green vortex at 64^3 elements, p=4
 updates per second: 4 * steps * K * (p+1)^3 * 5 / wall.
 
 Both paths are timed on the same workload: the mixed path (FP32
-interpolation / flux / contractions, FP64 state, RK4, inverse mass and
+interpolation / flux / derivatives, FP64 state, RK4, return to the nodes and
 reductions) is `value`; the FP64 plain path is reported beside it with the
 speed-up, and the mixed state's relative L2 error against the FP64 state
 after the timed steps (both start from the same initial state) together with
@@ -427,7 +427,7 @@ def main():
         "higher_is_better": True,
         "scaling": "weak",
         "vs_baseline": None,
-        "dtype": "f32 flux/quadrature + f64 state, RK4, inverse mass, reductions" if mixed else "f64",
+        "dtype": "f32 flux/quadrature/derivatives + f64 state, RK4, return to the nodes, reductions" if mixed else "f64",
         "data": "synthetic: compressible Taylor-Green initial state (Re 1600, Mach 0.1), no files",
         "config": {"workload": f"LDG RHS + RK4, Taylor-Green {nx}^3 elements p={p} ({dof} DOF), "
                                f"dt = 0.01 dx/(2p+1)", "elements": r["K"], "p": p, "dof": dof,
